@@ -89,11 +89,7 @@ struct m3_hip_device {
     char name[256];
     uint64_t total_bytes;
     uint32_t compute_units;
-    uint32_t lds_per_block; /* bytes of LDS one workgroup may use */
     uint32_t wall_clock_khz; /* rate of s_memrealtime; 0 if unknown */
-    /* M3_HIP_SOFTMAX_LATE_US at open (negative when unset): when a wave of
-     * the lane-row softmax counts as late (m3_hip_softmax.hip) */
-    float softmax_late_us;
     /* M3_HIP_SOFTMAX_HOLD_US at open (negative when unset): how long after
      * its start a wave of the lane-row softmax holds its stores */
     float softmax_hold_us;

@@ -297,10 +297,8 @@ extern "C" int m3_hip_device_open(int ordinal, m3_hip_device **device_output,
                                  : nullptr;
     device->total_bytes = (uint64_t)properties.totalGlobalMem;
     device->compute_units = (uint32_t)properties.multiProcessorCount;
-    device->lds_per_block = (uint32_t)properties.sharedMemPerBlock;
     {
         int rate = 0;
-        const char *late = std::getenv("M3_HIP_SOFTMAX_LATE_US");
         const char *hold = std::getenv("M3_HIP_SOFTMAX_HOLD_US");
         const char *wide = std::getenv("M3_HIP_SOFTMAX_WIDE_GRID");
 
@@ -309,9 +307,6 @@ extern "C" int m3_hip_device_open(int ordinal, m3_hip_device **device_output,
                                   ordinal) == hipSuccess && rate > 0
                 ? (uint32_t)rate
                 : 0U;
-        device->softmax_late_us =
-            late != nullptr && late[0] != '\0' ? std::strtof(late, nullptr)
-                                                : -1.0F;
         device->softmax_hold_us =
             hold != nullptr && hold[0] != '\0' ? std::strtof(hold, nullptr)
                                                 : -1.0F;

@@ -18,28 +18,20 @@
  *   - p_j is the IEEE F32 quotient e_j / sum, formed as
  *     RN_f32(e_j * RN_f64(1/sum)) where that is exact (m3_softmax_scale4).
  *
- * Kernels for rows contiguous along the last axis, by width; "VEC" rows
- * have aligned starts and a width that is a multiple of 4 and move in 16-
- * or 8-byte accesses, other rows element by element; row starts may be
- * evenly spaced or follow several outer axes (m3_softmax_row):
- *   - VEC rows of 513..1024 columns, and of 257..512 columns with 16-bit
- *     input or output: four rows per wave, one per 16-lane DPP row, the
- *     in-order sums carried in registers by additions whose addends are
- *     broadcast from lane to lane (row_newbcast), with no LDS traffic
- *     (m3_softmax_lane_rows_kernel).
- *   - other rows up to 2048 columns: wave-independent rows
- *     (m3_softmax_rows_kernel). A wave holds R rows in VGPRs, reduces max
- *     and k, forms e_j in place and streams 256-column chunks through a
- *     wave-private LDS tile where the in-order sums run; no workgroup
- *     barrier separates the phases, so waves overlap memory and
- *     arithmetic.
- *   - VEC rows with evenly spaced starts up to 8192 columns: a 256-thread
- *     workgroup owns a tile of whole rows in LDS (m3_softmax_tiled_kernel);
- *     phase 1 loads a row, reduces max and k and writes e_j to LDS; phase 2
- *     has one lane per row sum its row in order and form 1/sum in double;
- *     phase 3 reads e_j back, scales, rounds and stores coalesced. LDS rows
- *     are padded by 4 floats so the per-row walks hit distinct banks.
- *   - any other row: three streamed passes over 256-column chunks
+ * Kernels for rows contiguous along the last axis, by width. Rows may
+ * start at any element and have any width (a lane reads and writes four
+ * columns in one access at any alignment; the lane that holds a row's end
+ * moves them into place), be evenly spaced or follow several outer axes
+ * (m3_softmax_row):
+ *   - up to 256 columns: m3_softmax_short_rows_kernel, four rows per wave,
+ *     one per 16-lane DPP row, the in-order sums carried in registers and
+ *     passed from lane to lane;
+ *   - 257..1024 columns: m3_softmax_lane_rows_kernel, the same layout with
+ *     stores held back while the launch's reads are in flight; up to 2048
+ *     columns a row takes a pair of DPP rows;
+ *   - 2049..65536 columns: m3_softmax_wide_kernel, a workgroup per row held
+ *     in registers, the in-order sum in parallel;
+ *   - wider rows: three streamed passes over 256-column chunks
  *     (m3_softmax_stream_kernel), carrying the in-order sum across chunks
  *     and reading the row again for the scale pass.
  * A last axis that is not contiguous runs one thread per row through the
@@ -56,27 +48,30 @@ namespace {
 
 constexpr uint32_t kThreads = 256U;
 constexpr uint32_t kWaves = kThreads / 64U;
-constexpr uint32_t kStaticLds = 1024U; /* room for the static arrays */
-constexpr uint32_t kTiledLdsCap = 65536U; /* dynamic LDS of the tiled kernel */
-constexpr uint32_t kMaxTileRows = 16U;
-constexpr uint32_t kMaxWidth = 8192U;
 constexpr uint32_t kPad = 4U;
 constexpr uint32_t kChunk = 256U;         /* columns per LDS chunk */
 constexpr uint32_t kLine = kChunk + kPad; /* LDS floats per chunk row */
 constexpr uint64_t kMaxGrid = 1U << 20;   /* workgroups; waves loop beyond */
-constexpr uint64_t kMaxLaneGrid = 0x7fffffffU; /* grid x limit */
+constexpr uint64_t kMaxGridX = 1U << 20; /* workgroups per grid row */
 constexpr double kHbmBytesPerUs = 8.0e6; /* MI355X peak, 8 TB/s */
-constexpr double kLateFactor = 0.95;
-constexpr double kLateFloorUs = 3.0;
-constexpr double kHoldFactor = 1.25;
+constexpr double kHoldFactor = 1.07;
 constexpr uint32_t kLaneRowWavesPerSimd = 4U; /* amdgpu_waves_per_eu */
 constexpr uint32_t kStreamRows = 4U; /* rows per workgroup, streamed kernel */
 
-/* Four F32 -inf: what a load past the end of a row reads instead. Never
- * written; not const, so that it is in the global address space like the
- * rows and a select between the two stays a global load. */
-__device__ float4 m3_minus_inf4 = {-INFINITY, -INFINITY, -INFINITY,
-                                   -INFINITY};
+/* Four -inf of each float dtype: what a load past the end of a row reads
+ * instead, a line that stays in the caches. Never written; not const, so
+ * that it is in the global address space like the rows and a select between
+ * the two stays a global load. */
+__device__ __align__(16) uint32_t m3_minus_inf[3][4] = {
+    {0xff800000U, 0xff800000U, 0xff800000U, 0xff800000U}, /* F32 */
+    {0xfc00fc00U, 0xfc00fc00U, 0U, 0U},                   /* F16 */
+    {0xff80ff80U, 0xff80ff80U, 0U, 0U}};                  /* BF16 */
+
+/* Vectors read and written at any element alignment. */
+typedef float m3_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t m3_u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef _Float16 m3_f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 m3_bf16x4 __attribute__((ext_vector_type(4)));
 
 struct m3_softmax_args {
     const uint8_t *input;
@@ -86,10 +81,6 @@ struct m3_softmax_args {
     uint32_t width;
     uint32_t in_dtype;
     uint32_t out_dtype;
-    uint32_t tile_rows;
-    /* lane-row kernel: s_memrealtime ticks after its start past which a
-     * wave still waiting for its rows counts as late */
-    uint32_t late_ticks;
     /* lane-row kernel: s_memrealtime ticks after its start before which a
      * wave does not store its results (0: no hold) */
     uint32_t hold_ticks;
@@ -119,6 +110,22 @@ __device__ __forceinline__ const uint8_t *m3_softmax_row(
         rest = q;
     }
     return a.input + offset;
+}
+
+/* This workgroup's index in a launch of m3_softmax_grid. */
+__device__ __forceinline__ uint64_t m3_softmax_block()
+{
+    return (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
+/* A grid of at least `blocks` workgroups: the runtime takes fewer than
+ * 2^32 work-items along x, so more than kMaxGridX workgroups go to rows of
+ * the grid (those past the tensor's rows store nothing). */
+dim3 m3_softmax_grid(uint64_t blocks)
+{
+    const uint64_t x = std::min(blocks, kMaxGridX);
+
+    return dim3((uint32_t)x, (uint32_t)((blocks + x - 1U) / x));
 }
 
 /* Wave64 reductions through DPP row operations, which stay in the VALU
@@ -181,61 +188,130 @@ __device__ __forceinline__ float m3_uniform_f32(float v)
     return __builtin_bit_cast(float, m3_uniform_u32(m3_f32_bits(v)));
 }
 
-/* Lane `k`'s double, as a wave-uniform value. */
-__device__ __forceinline__ double m3_lane_f64(double v, int k)
+/* Four 16-bit values widened to F32. The conversions are the hardware's:
+ * softmax inputs hold no NaN (checked before the kernel runs), and for
+ * every other value v_cvt_f32_f16 gives the bits of m3_f16_to_f32_bits. */
+__device__ __forceinline__ float4 m3_widen4(m3_u32x2 h, uint32_t dtype)
 {
-    uint64_t bits = __builtin_bit_cast(uint64_t, v);
-    uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, k);
-    uint32_t hi =
-        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32U), k);
+    if (dtype == M3N_F16) {
+        const m3_f16x4 x = __builtin_bit_cast(m3_f16x4, h);
 
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32U) | lo);
-}
-
-/* Four 16-bit values widened to F32. */
-__device__ __forceinline__ float4 m3_widen4(uint32_t lo, uint32_t hi,
-                                            uint32_t dtype)
-{
-    return make_float4(
-        m3_bits_f32(m3_load_as_f32_bits(lo & 0xffffU, dtype)),
-        m3_bits_f32(m3_load_as_f32_bits(lo >> 16U, dtype)),
-        m3_bits_f32(m3_load_as_f32_bits(hi & 0xffffU, dtype)),
-        m3_bits_f32(m3_load_as_f32_bits(hi >> 16U, dtype)));
-}
-
-/* A load that is nontemporal (data read once) or ordinary (data read
- * again soon, which the caches may keep). */
-template <bool NT, typename T>
-__device__ __forceinline__ T m3_softmax_read(const T *p)
-{
-    if (NT) {
-        return __builtin_nontemporal_load(p);
+        return make_float4((float)x[0], (float)x[1], (float)x[2],
+                           (float)x[3]);
     }
-    return *p;
+    return make_float4(m3_bits_f32(h[0] << 16U),
+                       m3_bits_f32(h[0] & 0xffff0000U),
+                       m3_bits_f32(h[1] << 16U),
+                       m3_bits_f32(h[1] & 0xffff0000U));
 }
 
-/* Four consecutive row elements starting at column c, as F32, from an
- * aligned row (16 bytes for F32, 8 for 16-bit dtypes); nontemporal unless
- * NT is false. */
+/* Four results rounded to a 16-bit dtype, to nearest even, by the
+ * hardware: no result is NaN, and on the others v_cvt_f16_f32 and
+ * v_cvt_pk_bf16_f32 give the bits of m3_store_from_f32_bits, subnormal
+ * sources and results included (one or half an instruction per value
+ * against four or more). */
+__device__ __forceinline__ m3_u32x2 m3_narrow4(float4 p, uint32_t dtype)
+{
+    const m3_f32x4 x = {p.x, p.y, p.z, p.w};
+
+    if (dtype == M3N_F16) {
+        return __builtin_bit_cast(m3_u32x2,
+                                  __builtin_convertvector(x, m3_f16x4));
+    }
+    return __builtin_bit_cast(m3_u32x2,
+                              __builtin_convertvector(x, m3_bf16x4));
+}
+
+/* Where the lane at column c of a row of at least four elements reads its
+ * four columns: at c, at the row's last four columns when the row ends
+ * inside them (m3_softmax_edge4 moves them into place), or -inf for a
+ * column past the width. No load is under a branch, so the compiler can
+ * wait for each alone. A row that is not RAGGED has a multiple of four
+ * columns, which no float4 straddles. */
+template <bool F32IO, bool RAGGED = true>
+__device__ __forceinline__ const uint8_t *m3_softmax_source(
+    const uint8_t *row, uint32_t c, uint32_t width, uint32_t dtype)
+{
+    const uint64_t column = RAGGED ? min(c, width - 4U) : c;
+
+    return c < width
+               ? row + column * (F32IO || dtype == M3N_F32 ? 4U : 2U)
+               : (const uint8_t *)m3_minus_inf[F32IO ? (uint32_t)M3N_F32
+                                                     : dtype];
+}
+
+/* Four consecutive elements at p, as F32, in one 16-byte (F32) or 8-byte
+ * (16-bit) access at any element alignment: gfx950 serves global accesses
+ * at any alignment, so rows of odd width or odd start move in the same
+ * instructions as aligned ones. Nontemporal (data read once) unless NT is
+ * false (data read again soon, which the caches may keep). */
 template <bool F32IO, bool NT = true>
-__device__ __forceinline__ float4 m3_softmax_load4(const uint8_t *row,
-                                                   uint64_t c, uint32_t dtype)
+__device__ __forceinline__ float4 m3_softmax_load4(const uint8_t *p,
+                                                   uint32_t dtype)
 {
     if (F32IO || dtype == M3N_F32) {
-        const m3_f32x4 w =
-            m3_softmax_read<NT>((const m3_f32x4 *)(row + c * 4U));
+        m3_f32x4 w;
 
+        if constexpr (NT) {
+            w = __builtin_nontemporal_load((const m3_f32x4_any *)p);
+        } else {
+            w = *(const m3_f32x4_any *)p;
+        }
         return make_float4(w[0], w[1], w[2], w[3]);
     }
-    const m3_u32x2 h = m3_softmax_read<NT>((const m3_u32x2 *)(row + c * 2U));
+    m3_u32x2 h;
 
-    return m3_widen4(h[0], h[1], dtype);
+    if constexpr (NT) {
+        h = __builtin_nontemporal_load((const m3_u32x2_any *)p);
+    } else {
+        h = *(const m3_u32x2_any *)p;
+    }
+    return m3_widen4(h, dtype);
 }
 
-/* Columns c..c+3 of a row of `width` elements at any alignment, element
- * by element; columns at or past the width read as -inf. */
-template <bool F32IO>
-__device__ __forceinline__ float4 m3_softmax_load4_masked(
+/* The block, of `columns` columns, that holds the end of a row whose last
+ * float4 is partial; none (~0) when the width is a multiple of four. */
+__device__ __forceinline__ uint32_t m3_softmax_edge_block(uint32_t width,
+                                                          uint32_t columns)
+{
+    return (width & 3U) != 0U ? width / columns : ~0U;
+}
+
+/* The four columns from c on, given what m3_softmax_source read for them:
+ * a float4 that the row's end cuts is moved down to its place, with -inf
+ * behind it (a float4 past the width is -inf throughout and stays so).
+ * Only the block that holds the end needs it. */
+__device__ __forceinline__ float4 m3_softmax_edge4(float4 x, uint32_t c,
+                                                   uint32_t width)
+{
+    const uint32_t d = c - min(c, width - 4U);
+    const float none = -INFINITY;
+
+    if ((d & 1U) != 0U) {
+        x = make_float4(x.y, x.z, x.w, none);
+    }
+    if ((d & 2U) != 0U) {
+        x = make_float4(x.z, x.w, none, none);
+    }
+    return x;
+}
+
+/* Columns c..c+3 of a row of at least four elements; columns at or past
+ * the width read as -inf. */
+template <bool F32IO, bool NT = true>
+__device__ __forceinline__ float4 m3_softmax_get4(const uint8_t *row,
+                                                  uint32_t c, uint32_t width,
+                                                  uint32_t dtype)
+{
+    return m3_softmax_edge4(
+        m3_softmax_load4<F32IO, NT>(
+            m3_softmax_source<F32IO>(row, c, width, dtype), dtype),
+        c, width);
+}
+
+/* Columns c..c+3 of a row of any width, element by element; columns at or
+ * past the width read as -inf. For rows of fewer than four elements. */
+__device__ __forceinline__ float4 m3_softmax_load4_elements(
     const uint8_t *row, uint32_t c, uint32_t width, uint32_t dtype)
 {
     float x[4];
@@ -243,48 +319,49 @@ __device__ __forceinline__ float4 m3_softmax_load4_masked(
 #pragma unroll
     for (uint32_t i = 0U; i < 4U; ++i) {
         const uint32_t col = min(c + i, width - 1U);
-        float value;
+        const float value =
+            dtype == M3N_F32
+                ? *(const float *)(row + (uint64_t)col * 4U)
+                : m3_bits_f32(m3_load_as_f32_bits(
+                      *(const uint16_t *)(row + (uint64_t)col * 2U), dtype));
 
-        if (F32IO || dtype == M3N_F32) {
-            value = *(const float *)(row + (uint64_t)col * 4U);
-        } else {
-            value = m3_bits_f32(m3_load_as_f32_bits(
-                *(const uint16_t *)(row + (uint64_t)col * 2U), dtype));
-        }
         x[i] = c + i < width ? value : -INFINITY;
     }
     return make_float4(x[0], x[1], x[2], x[3]);
 }
 
 /* Four results at column c, rounded to the output dtype (streaming
- * stores). */
+ * stores, at any element alignment). */
 template <bool F32IO>
 __device__ __forceinline__ void m3_softmax_store4(uint8_t *row, uint64_t c,
                                                   uint32_t dtype, float4 p)
 {
     if (F32IO || dtype == M3N_F32) {
-        m3_stream_store((float4 *)(row + c * 4U), p);
+        const m3_f32x4_any w = {p.x, p.y, p.z, p.w};
+
+        __builtin_nontemporal_store(w, (m3_f32x4_any *)(row + c * 4U));
         return;
     }
-    uint2 packed;
+    const m3_u32x2_any h = m3_narrow4(p, dtype);
 
-    packed.x = m3_store_from_f32_bits(m3_f32_bits(p.x), dtype) |
-               (m3_store_from_f32_bits(m3_f32_bits(p.y), dtype) << 16U);
-    packed.y = m3_store_from_f32_bits(m3_f32_bits(p.z), dtype) |
-               (m3_store_from_f32_bits(m3_f32_bits(p.w), dtype) << 16U);
-    m3_stream_store((uint2 *)(row + c * 2U), packed);
+    __builtin_nontemporal_store(h, (m3_u32x2_any *)(row + c * 2U));
 }
 
-/* Stores the columns of c..c+3 that are inside the width, element by
- * element (output rows of any width). */
+/* Stores the columns of c..c+3 that are inside the width: all four at
+ * once, or element by element in the lane that holds the row's end. */
 template <bool F32IO>
-__device__ __forceinline__ void m3_softmax_store4_masked(
-    uint8_t *row, uint32_t c, uint32_t width, uint32_t dtype, float4 p)
+__device__ __forceinline__ void m3_softmax_put4(uint8_t *row, uint32_t c,
+                                                uint32_t width, uint32_t dtype,
+                                                float4 p)
 {
-    const float x[4] = {p.x, p.y, p.z, p.w};
+    if (c + 4U <= width) {
+        m3_softmax_store4<F32IO>(row, c, dtype, p);
+        return;
+    }
+    const float x[3] = {p.x, p.y, p.z};
 
 #pragma unroll
-    for (uint32_t i = 0U; i < 4U; ++i) {
+    for (uint32_t i = 0U; i < 3U; ++i) {
         if (c + i >= width) {
             continue;
         }
@@ -297,51 +374,6 @@ __device__ __forceinline__ void m3_softmax_store4_masked(
                 (uint16_t *)(row + (uint64_t)(c + i) * 2U));
         }
     }
-}
-
-/* Loads and stores of four columns, vectorised for aligned rows whose
- * width is a multiple of 4 (VEC) and element-wise otherwise. No load sits
- * under a branch: a column past the width loads from an address that is
- * always valid (m3_minus_inf4, or the row's first columns) and the result
- * is replaced, so the compiler can wait for each load alone instead of
- * for every load in flight. */
-template <bool F32IO, bool VEC, bool NT = true>
-__device__ __forceinline__ float4 m3_softmax_get4(const uint8_t *row,
-                                                  uint32_t c, uint32_t width,
-                                                  uint32_t dtype)
-{
-    if (!VEC) {
-        return m3_softmax_load4_masked<F32IO>(row, c, width, dtype);
-    }
-    const bool inside = c < width;
-
-    if (F32IO || dtype == M3N_F32) {
-        const m3_f32x4 *source =
-            inside ? (const m3_f32x4 *)(row + (uint64_t)c * 4U)
-                   : (const m3_f32x4 *)&m3_minus_inf4;
-        const m3_f32x4 w = m3_softmax_read<NT>(source);
-
-        return make_float4(w[0], w[1], w[2], w[3]);
-    }
-    const float4 x =
-        m3_softmax_load4<F32IO, NT>(row, inside ? c : 0U, dtype);
-
-    return inside ? x
-                  : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-}
-
-template <bool F32IO, bool VEC>
-__device__ __forceinline__ void m3_softmax_put4(uint8_t *row, uint32_t c,
-                                                uint32_t width, uint32_t dtype,
-                                                float4 p)
-{
-    if (VEC) {
-        if (c < width) {
-            m3_softmax_store4<F32IO>(row, c, dtype, p);
-        }
-        return;
-    }
-    m3_softmax_store4_masked<F32IO>(row, c, width, dtype, p);
 }
 
 /* p = e / sum, the IEEE F32 quotient, for e >= 0 and sum >= 1 given
@@ -402,439 +434,6 @@ __device__ __forceinline__ float4 m3_softmax_scale4(float4 e, double inverse)
     return p;
 }
 
-/* The reference's left-to-right F32 sum of `width` values (a multiple of
- * 4) at `line` in LDS. Loads run one 16-element block ahead of the
- * dependent additions so LDS latency overlaps the chain. */
-__device__ __forceinline__ float m3_row_sum_in_order(const float *line,
-                                                     uint32_t width)
-{
-    float sum = 0.0F;
-    uint32_t c = 0U;
-
-    if (width >= 16U) {
-        float4 current[4];
-        float4 next[4];
-
-#pragma unroll
-        for (uint32_t k = 0U; k < 4U; ++k) {
-            current[k] = *(const float4 *)(line + 4U * k);
-        }
-        for (c = 16U; c + 16U <= width; c += 16U) {
-#pragma unroll
-            for (uint32_t k = 0U; k < 4U; ++k) {
-                next[k] = *(const float4 *)(line + c + 4U * k);
-            }
-#pragma unroll
-            for (uint32_t k = 0U; k < 4U; ++k) {
-                sum = sum + current[k].x;
-                sum = sum + current[k].y;
-                sum = sum + current[k].z;
-                sum = sum + current[k].w;
-            }
-#pragma unroll
-            for (uint32_t k = 0U; k < 4U; ++k) {
-                current[k] = next[k];
-            }
-        }
-#pragma unroll
-        for (uint32_t k = 0U; k < 4U; ++k) {
-            sum = sum + current[k].x;
-            sum = sum + current[k].y;
-            sum = sum + current[k].z;
-            sum = sum + current[k].w;
-        }
-    }
-    for (; c < width; c += 4U) {
-        float4 e = *(const float4 *)(line + c);
-
-        sum = sum + e.x;
-        sum = sum + e.y;
-        sum = sum + e.z;
-        sum = sum + e.w;
-    }
-    return sum;
-}
-
-/* Per-row state shared through LDS between the phases. */
-struct m3_row_state {
-    float maximum;
-    uint32_t infinities;
-    double inverse;      /* 1/sum for finite rows */
-    float one_over_count; /* 1/k for rows whose maximum is +inf */
-    uint32_t pad;
-};
-
-template <bool F32IO>
-__global__ __launch_bounds__(256) void m3_softmax_tiled_kernel(
-    m3_softmax_args a)
-{
-    if (m3_gate_closed(a.list_gate)) {
-        return; /* a check earlier in the list failed */
-    }
-    extern __shared__ float lds[];
-    __shared__ m3_row_state state[kMaxTileRows];
-    __shared__ uint64_t exp_table[32];
-    const uint32_t lane = threadIdx.x & 63U;
-    const uint32_t wave = threadIdx.x >> 6U;
-    const uint32_t width = a.width;
-    const uint32_t pitch = width + kPad;
-    const uint32_t in_dtype = F32IO ? (uint32_t)M3N_F32 : a.in_dtype;
-    const uint32_t out_dtype = F32IO ? (uint32_t)M3N_F32 : a.out_dtype;
-    const uint32_t out_size = out_dtype == M3N_F32 ? 4U : 2U;
-
-    if (threadIdx.x < 32U) {
-        exp_table[threadIdx.x] = m3_expf_table[threadIdx.x];
-    }
-    for (uint64_t tile = blockIdx.x; tile * a.tile_rows < a.rows;
-         tile += gridDim.x) {
-        const uint64_t first_row = tile * a.tile_rows;
-        const uint32_t tile_rows =
-            (uint32_t)min((uint64_t)a.tile_rows, a.rows - first_row);
-
-        __syncthreads();
-        /* Phase 1: max, +inf count and e_j for each row of this wave. */
-        for (uint32_t r = wave; r < tile_rows; r += kWaves) {
-            const uint8_t *row = a.input + (first_row + r) * a.row_stride;
-            float *line = lds + (uint64_t)r * pitch;
-            float maximum = -INFINITY;
-            uint32_t infinities = 0U;
-
-            for (uint32_t c = lane * 4U; c < width; c += 256U) {
-                float4 v = m3_softmax_load4<F32IO>(row, c, in_dtype);
-
-                maximum = fmaxf(maximum, fmaxf(fmaxf(v.x, v.y),
-                                               fmaxf(v.z, v.w)));
-                infinities += (v.x == INFINITY) + (v.y == INFINITY) +
-                              (v.z == INFINITY) + (v.w == INFINITY);
-                *(float4 *)(line + c) = v;
-            }
-            maximum = m3_wave_max(maximum);
-            infinities = m3_wave_sum(infinities);
-            if (maximum != INFINITY && maximum != -INFINITY) {
-                for (uint32_t c = lane * 4U; c < width; c += 256U) {
-                    float4 v = *(float4 *)(line + c);
-                    float4 e;
-
-                    e.x = m3_expf_with_table(v.x - maximum, exp_table);
-                    e.y = m3_expf_with_table(v.y - maximum, exp_table);
-                    e.z = m3_expf_with_table(v.z - maximum, exp_table);
-                    e.w = m3_expf_with_table(v.w - maximum, exp_table);
-                    *(float4 *)(line + c) = e;
-                }
-            }
-            if (lane == 0U) {
-                state[r].maximum = maximum;
-                state[r].infinities = infinities;
-            }
-        }
-        __syncthreads();
-        /* Phase 2: the reference's left-to-right F32 sum, one lane per row. */
-        if (threadIdx.x < tile_rows) {
-            m3_row_state *s = &state[threadIdx.x];
-            float maximum = s->maximum;
-
-            if (maximum != INFINITY && maximum != -INFINITY) {
-                s->inverse = 1.0 / (double)m3_row_sum_in_order(
-                                       lds + (uint64_t)threadIdx.x * pitch,
-                                       width);
-            } else if (maximum == INFINITY) {
-                s->one_over_count = 1.0F / (float)s->infinities;
-            }
-        }
-        __syncthreads();
-        /* Phase 3: scale, round to the output dtype, store. */
-        for (uint32_t r = wave; r < tile_rows; r += kWaves) {
-            const float *line = lds + (uint64_t)r * pitch;
-            uint8_t *out = a.output + (first_row + r) * (uint64_t)width *
-                                          out_size;
-            const m3_row_state s = state[r];
-
-            for (uint32_t c = lane * 4U; c < width; c += 256U) {
-                float4 v = *(const float4 *)(line + c);
-                float4 p;
-
-                if (s.maximum == -INFINITY) {
-                    p = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
-                } else if (s.maximum == INFINITY) {
-                    p.x = v.x == INFINITY ? s.one_over_count : 0.0F;
-                    p.y = v.y == INFINITY ? s.one_over_count : 0.0F;
-                    p.z = v.z == INFINITY ? s.one_over_count : 0.0F;
-                    p.w = v.w == INFINITY ? s.one_over_count : 0.0F;
-                } else {
-                    p = m3_softmax_scale4(v, s.inverse);
-                }
-                m3_softmax_store4<F32IO>(out, c, out_dtype, p);
-            }
-        }
-    }
-}
-
-/* Adds four floats to s in order. */
-__device__ __forceinline__ float m3_add4(float s, float4 e)
-{
-    s = s + e.x;
-    s = s + e.y;
-    s = s + e.z;
-    return s + e.w;
-}
-
-/* Sum of the first n (a multiple of 4, at most 256) floats of an LDS line,
- * continuing the left-to-right F32 sum s. A full chunk keeps DEPTH 16-byte
- * loads in flight ahead of the dependent additions; a partial chunk (the
- * end of a trimmed row) issues four loads per 16 elements before adding
- * them, so LDS latency is paid once per 16 additions, not per 4. */
-template <int DEPTH>
-__device__ __forceinline__ float m3_chunk_sum(float s, const float *line,
-                                              uint32_t n)
-{
-    if (n == kChunk) {
-        float4 ahead[DEPTH];
-
-#pragma unroll
-        for (int i = 0; i < DEPTH; ++i) {
-            ahead[i] = *(const float4 *)(line + 4 * i);
-        }
-#pragma unroll
-        for (int i = 0; i < (int)kChunk / 4; ++i) {
-            float4 e = ahead[i % DEPTH];
-
-            if (i + DEPTH < (int)kChunk / 4) {
-                ahead[i % DEPTH] = *(const float4 *)(line + 4 * (i + DEPTH));
-            }
-            s = m3_add4(s, e);
-        }
-        return s;
-    }
-    uint32_t c = 0U;
-
-    for (; c + 16U <= n; c += 16U) {
-        float4 a = *(const float4 *)(line + c);
-        float4 b = *(const float4 *)(line + c + 4U);
-        float4 d = *(const float4 *)(line + c + 8U);
-        float4 f = *(const float4 *)(line + c + 12U);
-
-        s = m3_add4(s, a);
-        s = m3_add4(s, b);
-        s = m3_add4(s, d);
-        s = m3_add4(s, f);
-    }
-    for (; c < n; c += 4U) {
-        s = m3_add4(s, *(const float4 *)(line + c));
-    }
-    return s;
-}
-
-/* Orders this wave's LDS writes before its later LDS reads of other lanes'
- * data (the LDS executes one wave's operations in issue order). */
-__device__ __forceinline__ void m3_wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-/* Scales and stores one row of a register-resident task: p_j = e_j / sum
- * for a finite maximum, zeros for an all -inf row, 1/k on the k +inf
- * entries of a row whose maximum is +inf. `v` holds e_j (finite rows) or
- * the inputs (other rows). */
-template <int VPL, bool F32IO, bool VEC>
-__device__ __forceinline__ void m3_softmax_emit_row(
-    const float4 (&v)[VPL], float maximum, double inverse, uint8_t *out,
-    uint32_t lane, uint32_t width, uint32_t out_dtype)
-{
-    if (maximum != INFINITY && maximum != -INFINITY) {
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            const uint32_t c = lane * 4U + kChunk * j;
-
-            if (VEC && c >= width) {
-                continue;
-            }
-            m3_softmax_put4<F32IO, VEC>(out, c, width, out_dtype,
-                                        m3_softmax_scale4(v[j], inverse));
-        }
-        return;
-    }
-    float one_over_count = 0.0F;
-
-    if (maximum == INFINITY) {
-        uint32_t count = 0U;
-
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            count += (v[j].x == INFINITY) + (v[j].y == INFINITY) +
-                     (v[j].z == INFINITY) + (v[j].w == INFINITY);
-        }
-        one_over_count = 1.0F / (float)m3_wave_sum(count);
-    }
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        const uint32_t c = lane * 4U + kChunk * j;
-        float4 p;
-
-        if (VEC && c >= width) {
-            continue;
-        }
-        p.x = v[j].x == INFINITY ? one_over_count : 0.0F;
-        p.y = v[j].y == INFINITY ? one_over_count : 0.0F;
-        p.z = v[j].z == INFINITY ? one_over_count : 0.0F;
-        p.w = v[j].w == INFINITY ? one_over_count : 0.0F;
-        m3_softmax_put4<F32IO, VEC>(out, c, width, out_dtype, p);
-    }
-}
-
-/* Wave-independent rows (width <= 256 * VPL). Each wave takes R
- * consecutive rows at a time and keeps them in VGPRs, lane l holding
- * columns 4l + 256j .. 4l + 256j + 3 (VPL float4 per lane per row). It
- * reduces each row's maximum with DPP, forms e_j in place, then walks the
- * row in 256-column chunks, writing each chunk of its R rows to a
- * wave-private LDS tile where every lane continues the left-to-right sum
- * of row l % R. All 64 lanes run that chain: a wave instruction takes the
- * same issue slot at any lane count, and a full mask keeps the chain in
- * one basic block with its LDS reads. The sum stops after the wave's last
- * column holding something other than -inf: the later terms are +0 and
- * leave a nonnegative F32 sum unchanged, so masked (causal) rows cost
- * half. p_j is formed from the registers and streamed out. No workgroup
- * barrier is needed after the table copy, so the waves of a CU overlap
- * their loads, arithmetic and sums freely. VEC rows (aligned, width a
- * multiple of 4) move in 16-byte (F32) or 8-byte (16-bit) accesses; other
- * rows element by element, with columns past the width read as -inf. */
-template <int VPL, int R, int DEPTH, bool F32IO, bool VEC>
-__device__ __forceinline__ void m3_softmax_rows(const m3_softmax_args &a)
-{
-    __shared__ float tiles[kWaves][R][kLine];
-    __shared__ uint64_t exp_table[32];
-    const uint32_t lane = threadIdx.x & 63U;
-    const uint32_t wave = m3_uniform_u32(threadIdx.x >> 6U);
-    const uint32_t width = a.width;
-    const uint32_t in_dtype = F32IO ? (uint32_t)M3N_F32 : a.in_dtype;
-    const uint32_t out_dtype = F32IO ? (uint32_t)M3N_F32 : a.out_dtype;
-    const uint32_t out_size = out_dtype == M3N_F32 ? 4U : 2U;
-    const uint64_t out_pitch = (uint64_t)width * out_size;
-    const uint64_t tasks = (a.rows + R - 1U) / R;
-    float *tile = &tiles[wave][0][0];
-
-    if (threadIdx.x < 32U) {
-        exp_table[threadIdx.x] = m3_expf_table[threadIdx.x];
-    }
-    __syncthreads();
-    for (uint64_t task = (uint64_t)blockIdx.x * kWaves + wave; task < tasks;
-         task += (uint64_t)gridDim.x * kWaves) {
-        const uint64_t first_row = task * R;
-        /* rows of this task that exist (the last task may be partial) */
-        const uint32_t present =
-            (uint32_t)min((uint64_t)R, a.rows - first_row);
-        float4 v[R][VPL];
-        float maximum[R];
-        uint32_t last = 0U; /* 1 + index of the last float4 not all -inf */
-
-        /* Every load is issued and none is under a branch, so the wave
-         * waits for each row's data alone: row 0 is reduced and
-         * exponentiated while the later rows are still arriving. A row past
-         * the end of the tensor (the last task) reads the task's first row
-         * and is never stored. A VEC column past the width reads four F32
-         * -inf from m3_minus_inf4 (16-bit inputs: column 0, replaced by
-         * -inf). A variant serves widths above 256 * VPL / 2, so its chunks
-         * j < VPL / 2 are always inside the row. */
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const uint8_t *row = m3_softmax_row(
-                a, first_row + ((uint32_t)k < present ? (uint32_t)k : 0U));
-
-#pragma unroll
-            for (int j = 0; j < VPL; ++j) {
-                const uint32_t c = lane * 4U + kChunk * j;
-                const bool inside = (VPL > 1 && j < VPL / 2) || c < width;
-
-                if (!VEC) {
-                    v[k][j] = m3_softmax_load4_masked<F32IO>(row, c, width,
-                                                             in_dtype);
-                } else if (F32IO || in_dtype == M3N_F32) {
-                    const m3_f32x4 *source =
-                        inside ? (const m3_f32x4 *)(row + (uint64_t)c * 4U)
-                               : (const m3_f32x4 *)&m3_minus_inf4;
-                    const m3_f32x4 w = __builtin_nontemporal_load(source);
-
-                    v[k][j] = make_float4(w[0], w[1], w[2], w[3]);
-                } else {
-                    const float4 x = m3_softmax_load4<F32IO>(
-                        row, inside ? c : 0U, in_dtype);
-
-                    v[k][j] = inside ? x
-                                     : make_float4(-INFINITY, -INFINITY,
-                                                   -INFINITY, -INFINITY);
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            float m = -INFINITY;
-
-#pragma unroll
-            for (int j = 0; j < VPL; ++j) {
-                const float t = fmaxf(fmaxf(v[k][j].x, v[k][j].y),
-                                      fmaxf(v[k][j].z, v[k][j].w));
-
-                m = fmaxf(m, t);
-                last = t != -INFINITY ? max(last, lane + 64U * j + 1U) : last;
-            }
-            m = m3_uniform_f32(m3_wave_max(m));
-            maximum[k] = m;
-            if (m != INFINITY && m != -INFINITY) {
-#pragma unroll
-                for (int j = 0; j < VPL; ++j) {
-                    v[k][j].x = m3_expf_with_table(v[k][j].x - m, exp_table);
-                    v[k][j].y = m3_expf_with_table(v[k][j].y - m, exp_table);
-                    v[k][j].z = m3_expf_with_table(v[k][j].z - m, exp_table);
-                    v[k][j].w = m3_expf_with_table(v[k][j].w - m, exp_table);
-                }
-            }
-        }
-        const uint32_t wave_length = m3_uniform_u32(m3_wave_max_u32(last)) * 4U;
-        const float *line = tile + (lane % (uint32_t)R) * kLine;
-        float sum = 0.0F;
-
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            const uint32_t base = kChunk * j;
-
-            if (base >= wave_length) {
-                break;
-            }
-#pragma unroll
-            for (int k = 0; k < R; ++k) {
-                *(float4 *)(tile + k * kLine + lane * 4U) = v[k][j];
-            }
-            m3_wave_sync();
-            sum = m3_chunk_sum<DEPTH>(sum, line,
-                                      min(wave_length - base, kChunk));
-            m3_wave_sync();
-        }
-        const double inverse_of_lane = 1.0 / (double)sum;
-
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            if ((uint32_t)k >= present) {
-                continue;
-            }
-            m3_softmax_emit_row<VPL, F32IO, VEC>(
-                v[k], maximum[k], m3_lane_f64(inverse_of_lane, k),
-                a.output + (first_row + (uint32_t)k) * out_pitch, lane, width,
-                out_dtype);
-        }
-    }
-}
-
-template <int VPL, int R, int DEPTH, bool F32IO, bool VEC>
-__global__ __launch_bounds__(256) void m3_softmax_rows_kernel(
-    m3_softmax_args a)
-{
-    if (m3_gate_closed(a.list_gate)) {
-        return; /* a check earlier in the list failed */
-    }
-    m3_softmax_rows<VPL, R, DEPTH, F32IO, VEC>(a);
-}
-
 /* x of lane CTRL selects within this lane's 16-lane DPP row (`identity`
  * where the control names no lane). */
 template <int CTRL>
@@ -871,33 +470,17 @@ __device__ __forceinline__ uint32_t m3_row16_sum(uint32_t n)
     return n + m3_dpp_u32<0x140>(n);
 }
 
-/* s + (e of lane N of this DPP row): row_newbcast:N hands every lane of
- * the row the addend of lane N, so the 16 lanes carry the same sum. */
-template <int N>
-__device__ __forceinline__ float m3_add_from_lane(float s, float e)
-{
-    return s + m3_dpp_f32<0x150 + N>(0.0F, e);
-}
-
-/* Continues the left-to-right sum over the 64 columns of one block: lane
- * N holds columns 4N..4N+3 of it in e. */
-template <int... N>
-__device__ __forceinline__ float m3_block_sum(float s, float4 e,
-                                              std::integer_sequence<int, N...>)
-{
-    ((s = m3_add_from_lane<N>(s, e.x), s = m3_add_from_lane<N>(s, e.y),
-      s = m3_add_from_lane<N>(s, e.z), s = m3_add_from_lane<N>(s, e.w)),
-     ...);
-    return s;
-}
-
-/* The same sum with the running value passed from lane to lane: step g,
- * the same four instructions in every lane, takes lane g - 1's sum
- * (row_ror:1; lane 0 takes lane 15's, the end of the previous block) and
- * adds lane g's four columns, so that lane g holds the in-order sum after
- * step g and lane 15 after the block. A dependent DPP addition takes about
- * 12 cycles and a plain one 4: 6 cycles per column against 12 for
- * m3_block_sum, whose DPP operand is the addend, not the sum. */
+/* Continues the left-to-right sum over the 64 columns of one block: lane g
+ * of each 16-lane DPP row holds columns 4g..4g+3 of it in e. The running
+ * value passes from lane to lane: step g, the same four instructions in
+ * every lane, takes lane g - 1's sum (row_ror:1; lane 0 takes lane 15's, the
+ * end of the previous block) and adds lane g's four columns, so that lane g
+ * holds the in-order sum after step g and lane 15 after the block. A
+ * dependent DPP addition takes about 12 cycles and a plain one 4: 6 cycles
+ * per column, against 12 with every addend broadcast from its lane
+ * (row_newbcast), and faster at every size measured: 16.7 against 19.2 us
+ * for F32 [8192,1024], 55 against 62 us for [32768,1024], 19.1 against
+ * 23.0 us for BF16 [4096,2048]. */
 __device__ __forceinline__ float m3_block_sum_passed(float s, float4 e)
 {
 #pragma unroll
@@ -910,52 +493,85 @@ __device__ __forceinline__ float m3_block_sum_passed(float s, float4 e)
     return s;
 }
 
-/* Rows of 32Q + 1 .. 64Q columns (VEC: aligned, a multiple of 4 wide),
- * Q = 8 or 16, with the in-order sum carried in registers. A wave takes
- * four consecutive rows, one per 16-lane DPP row (lanes 16k..16k+15 hold
- * row k); lane i of a row holds columns 4i + 64j .. 4i + 64j + 3 (block
- * j = 0..Q-1), so each load instruction reads four runs of 256 bytes (F32)
- * or 128 bytes (16-bit). The maximum is reduced within the 16 lanes and
- * e_j formed in place; then the left-to-right sum is one dependent
- * addition per column, whose addend comes from the lane holding it
- * (m3_add_from_lane), and the four rows advance together. Against the
- * rows kernel this removes the LDS tile: there every lane group reads its
- * row's e_j back from LDS, at a bandwidth cost per CU that set the sum's
- * pace. As there, the sum stops after the wave's last float4 holding
- * something other than -inf (later terms are +0). Rows whose maximum is
- * +-inf are written from their inputs before the exponentials (zeros, or
- * 1/k on their k +inf entries) behind a wave-uniform test. FULL rows are
- * exactly 64Q wide; otherwise blocks of the second half may lie past the
- * width, read -inf there and are not stored. F32IO: F32 in and out, with
- * immediate-offset addressing; otherwise any float dtypes. One task per
- * wave: the grid covers them all (a loop over tasks took 30 more VGPRs and
- * ran slower).
+/* x of the same lane in the other DPP row of its pair (rows 0 and 1, rows
+ * 2 and 3): ds_swizzle, lane index xor 16. */
+__device__ __forceinline__ float m3_other_half(float x)
+{
+    return m3_bits_f32((uint32_t)__builtin_amdgcn_ds_swizzle(
+        (int)m3_f32_bits(x), 0x401F));
+}
+
+/* The running sum at the end of an even DPP row (its lane 15) moved to
+ * every lane of the odd row after it (row_bcast:15); even rows keep
+ * theirs. */
+__device__ __forceinline__ float m3_to_second_half(float x)
+{
+    return m3_bits_f32((uint32_t)__builtin_amdgcn_update_dpp(
+        (int)m3_f32_bits(x), (int)m3_f32_bits(x), 0x142, 0xA, 0xF, false));
+}
+
+/* Rows of 32Q + 1 .. 64Q columns, Q = 8 or 16, with the in-order sum
+ * carried in registers. A wave takes four consecutive rows, one per 16-lane
+ * DPP row (lanes 16k..16k+15 hold row k); lane i of a row holds columns
+ * 4i + 64j .. 4i + 64j + 3 (block j = 0..Q-1), so each load instruction
+ * reads four runs of 256 bytes (F32) or 128 bytes (16-bit), at any
+ * alignment. The maximum is reduced within the 16 lanes and e_j formed in
+ * place; then the left-to-right sum passes from lane to lane
+ * (m3_block_sum_passed), the four rows advancing together, with no LDS
+ * traffic. The sum and, where the class has blocks past the row, the
+ * exponentials stop after the wave's last float4 holding something other
+ * than -inf (later terms are +0). Rows whose maximum is +-inf are written
+ * from their inputs before the exponentials (zeros, or 1/k on their k +inf
+ * entries) behind a wave-uniform test. FULL rows are exactly 64Q wide;
+ * otherwise blocks of the second half may lie past the width, read -inf
+ * there and are not stored. F32IO: F32 in and out, with immediate-offset
+ * addressing; otherwise any float dtypes, the conversions chosen once per
+ * wave. One task per wave: the grid covers them all (a loop over tasks took
+ * 30 more VGPRs and ran slower).
  *
- * All waves issue their loads at once, and the waves whose rows the HBM
- * serves last decide when the kernel ends: by then most SIMDs are idle and
- * the sum's latency is what counts. A wave whose rows arrive more than
- * a.late_ticks after its start (s_memrealtime) therefore sums with
- * m3_block_sum_passed, half the latency per column; the others keep
- * m3_block_sum, which leaves more issue slots to the waves sharing their
- * SIMD. Both perform the same additions in the same order. */
-template <int Q, bool FULL, bool F32IO>
+ * HALVES: rows of 64Q + 1 .. 128Q columns, two per wave, each as two halves
+ * of a multiple of 64 columns in a pair of DPP rows. The sum runs over the
+ * first half in both DPP rows, its end value moves to the second one
+ * (row_bcast:15) and the sum goes on over the second half: as many
+ * additions per row as columns, as with one row per DPP row.
+ *
+ * Bound by HBM for F32 rows that fill the device and by the additions and
+ * exponentials for 16-bit ones. Against the forms it replaced (element by
+ * element for rows not aligned to 16 or 8 bytes; beyond 1024 columns a wave
+ * per two rows with the sums in LDS): BF16 causal [16,777,777] 61 -> 17.2
+ * us, F32 [10796,777] 54 -> 19.5, BF16 [8192,1024] 30.4 -> 15.2, F32
+ * [5588,1501] 77 -> 21.5, [4096,2048] 24.1 -> 21.4, BF16 [4096,2048] 36.3
+ * -> 19.1. */
+template <int Q, bool FULL, bool HALVES, bool F32IO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void m3_softmax_lane_rows_kernel(m3_softmax_args a)
 {
     if (m3_gate_closed(a.list_gate)) {
         return; /* a check earlier in the list failed */
     }
+    static_assert(!(FULL && HALVES), "a halved row is never full");
+    /* blocks wholly inside any row (or half) of the class */
+    constexpr int kInside = FULL ? Q : HALVES ? Q / 2 - 1 : Q / 2;
+    constexpr uint32_t kRows = HALVES ? 2U : 4U; /* rows per wave */
     __shared__ uint64_t exp_table[32];
     const uint32_t lane = threadIdx.x & 63U;
     const uint32_t wave = m3_uniform_u32(threadIdx.x >> 6U);
     const uint32_t sub = lane & 15U;
-    const uint32_t width = a.width;
     const uint32_t in_dtype = F32IO ? (uint32_t)M3N_F32 : a.in_dtype;
     const uint32_t out_dtype = F32IO ? (uint32_t)M3N_F32 : a.out_dtype;
-    const uint64_t out_pitch =
-        (uint64_t)width * (out_dtype == M3N_F32 ? 4U : 2U);
-    const uint64_t tasks = (a.rows + 3U) / 4U;
-    const uint64_t task = (uint64_t)blockIdx.x * kWaves + wave;
+    const uint32_t in_size = in_dtype == M3N_F32 ? 4U : 2U;
+    const uint32_t out_size = out_dtype == M3N_F32 ? 4U : 2U;
+    const uint64_t out_pitch = (uint64_t)a.width * out_size;
+    /* the columns of this lane's DPP row: the row, or with HALVES its first
+     * `split` columns (even DPP rows) and the rest (odd ones); `least`: the
+     * fewer of the two, in every lane */
+    const uint32_t split = HALVES ? ((a.width + 127U) / 128U) * 64U : 0U;
+    const uint32_t least = a.width - split;
+    const bool second = HALVES && (lane & 16U) != 0U;
+    const uint32_t width = HALVES && !second ? split : least;
+    const uint32_t edge = m3_softmax_edge_block(least, 64U);
+    const uint64_t tasks = (a.rows + kRows - 1U) / kRows;
+    const uint64_t task = m3_softmax_block() * kWaves + wave;
     const uint64_t start = __builtin_amdgcn_s_memrealtime();
     /* The expf table's load goes first and the rows' loads right after it,
      * ahead of the barrier that publishes the table in LDS. The barrier's
@@ -965,32 +581,57 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
      * task loads the last task's rows and stops at the barrier. */
     const uint64_t table_word = m3_expf_table[threadIdx.x & 31U];
     const uint64_t mine = task < tasks ? task : tasks - 1U;
-    const uint64_t row = mine * 4U + (lane >> 4U);
+    const uint64_t row = mine * kRows + (lane >> (HALVES ? 5U : 4U));
     const bool present = task < tasks && row < a.rows;
     /* a row past the end of the tensor reads the task's first row */
-    const uint8_t *in = m3_softmax_row(a, row < a.rows ? row : mine * 4U);
+    const uint8_t *in = m3_softmax_row(a, row < a.rows ? row : mine * kRows);
     uint8_t *out = a.output + row * out_pitch;
+
+    if (second) {
+        in += (uint64_t)split * in_size;
+        out += (uint64_t)split * out_size;
+    }
     float4 v[Q];
 
+    if (F32IO || in_dtype == M3N_F32) {
+        /* two loops: a load from a choice of the two addresses becomes two
+         * loads that are no longer nontemporal */
 #pragma unroll
-    for (int j = 0; j < Q; ++j) {
-        const uint32_t c = sub * 4U + 64U * j;
-        const bool inside = FULL || j < Q / 2 || c < width;
+        for (int j = 0; j < kInside; ++j) {
+            v[j] = m3_softmax_load4<true>(in + sub * 16U + 256U * j, M3N_F32);
+        }
+#pragma unroll
+        for (int j = kInside; j < Q; ++j) {
+            v[j] = m3_softmax_load4<true>(
+                m3_softmax_source<true>(in, sub * 4U + 64U * j, width,
+                                        M3N_F32),
+                M3N_F32);
+        }
+    } else {
+        m3_u32x2 raw[Q];
 
-        if (F32IO) {
-            const m3_f32x4 *source =
-                inside ? (const m3_f32x4 *)(in + sub * 16U) + 16 * j
-                       : (const m3_f32x4 *)&m3_minus_inf4;
-            const m3_f32x4 w = __builtin_nontemporal_load(source);
-
-            v[j] = make_float4(w[0], w[1], w[2], w[3]);
+#pragma unroll
+        for (int j = 0; j < kInside; ++j) {
+            raw[j] = __builtin_nontemporal_load(
+                (const m3_u32x2_any *)(in + sub * 8U + 128U * j));
+        }
+#pragma unroll
+        for (int j = kInside; j < Q; ++j) {
+            raw[j] = __builtin_nontemporal_load(
+                (const m3_u32x2_any *)m3_softmax_source<false>(
+                    in, sub * 4U + 64U * j, width, in_dtype));
+        }
+        /* one uniform branch for the whole row, not one per value */
+        if (in_dtype == M3N_F16) {
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+                v[j] = m3_widen4(raw[j], M3N_F16);
+            }
         } else {
-            const float4 x =
-                m3_softmax_load4<false>(in, inside ? c : 0U, in_dtype);
-
-            v[j] = inside ? x
-                          : make_float4(-INFINITY, -INFINITY, -INFINITY,
-                                        -INFINITY);
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+                v[j] = m3_widen4(raw[j], M3N_BF16);
+            }
         }
     }
     if (threadIdx.x < 32U) {
@@ -1004,6 +645,12 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
         uint32_t last = 0U; /* 1 + index of the last float4 not all -inf */
 
 #pragma unroll
+        for (int j = kInside; j < Q; ++j) {
+            if ((uint32_t)j == edge) {
+                v[j] = m3_softmax_edge4(v[j], sub * 4U + 64U * j, width);
+            }
+        }
+#pragma unroll
         for (int j = 0; j < Q; ++j) {
             const float t = fmaxf(fmaxf(v[j].x, v[j].y),
                                   fmaxf(v[j].z, v[j].w));
@@ -1012,24 +659,23 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
             last = t != -INFINITY ? sub + 16U * j + 1U : last;
         }
         m = m3_row16_max(m);
-        const uint32_t length = m3_uniform_u32(m3_wave_max_u32(last));
+        if (HALVES) {
+            m = fmaxf(m, m3_other_half(m));
+        }
+        /* blocks to sum: of the rows, or of their halves */
+        const uint32_t length =
+            m3_uniform_u32(m3_wave_max_u32(second ? 0U : last));
+        const uint32_t length2 =
+            HALVES ? m3_uniform_u32(m3_wave_max_u32(second ? last : 0U)) : 0U;
         const bool finite = m != INFINITY && m != -INFINITY;
-        /* every load has returned here (all were reduced); the wait makes
-         * the clock read follow them */
-        __builtin_amdgcn_s_waitcnt(0);
-        const bool late =
-            __builtin_amdgcn_s_memrealtime() - start > (uint64_t)a.late_ticks;
         /* stores p at block j when the block is inside the row */
-        auto put = [&](int j, float4 p) {
+        auto put = [&](int j, float4 p, uint32_t dtype) {
             const uint32_t c = sub * 4U + 64U * j;
 
-            if (!FULL && j >= Q / 2 && c >= width) {
-                return;
-            }
-            if (F32IO) {
-                m3_stream_store((float4 *)(out + sub * 16U) + 16 * j, p);
-            } else {
-                m3_softmax_store4<false>(out, c, out_dtype, p);
+            if (j < kInside || 64U * (j + 1U) <= least) {
+                m3_softmax_store4<F32IO>(out, c, dtype, p);
+            } else if (c < width) {
+                m3_softmax_put4<F32IO>(out, c, width, dtype, p);
             }
         };
 
@@ -1041,7 +687,11 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
                 count += (v[j].x == INFINITY) + (v[j].y == INFINITY) +
                          (v[j].z == INFINITY) + (v[j].w == INFINITY);
             }
-            const float one_over_count = 1.0F / (float)m3_row16_sum(count);
+            count = m3_row16_sum(count);
+            if (HALVES) {
+                count += m3_f32_bits(m3_other_half(m3_bits_f32(count)));
+            }
+            const float one_over_count = 1.0F / (float)count;
 
             if (!finite && present) {
 #pragma unroll
@@ -1052,7 +702,7 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
                     p.y = v[j].y == INFINITY ? one_over_count : 0.0F;
                     p.z = v[j].z == INFINITY ? one_over_count : 0.0F;
                     p.w = v[j].w == INFINITY ? one_over_count : 0.0F;
-                    put(j, p);
+                    put(j, p, out_dtype);
                 }
             }
         }
@@ -1065,6 +715,10 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
 
 #pragma unroll
         for (int j = 0; j < Q; ++j) {
+            if (!(FULL && F32IO) && 16U * j >= max(length, length2)) {
+                v[j] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+                continue;
+            }
             v[j].x = m3_expf_with_table(v[j].x - shift, exp_table);
             v[j].y = m3_expf_with_table(v[j].y - shift, exp_table);
             v[j].z = m3_expf_with_table(v[j].z - shift, exp_table);
@@ -1075,22 +729,27 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
         }
         float sum = 0.0F;
 
-        if (late) {
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+            if (16U * j < length) {
+                sum = m3_block_sum_passed(sum, v[j]);
+            }
+        }
+        if (HALVES) {
+            sum = m3_to_second_half(sum);
 #pragma unroll
             for (int j = 0; j < Q; ++j) {
-                if (16U * j < length) {
+                if (16U * j < length2) {
                     sum = m3_block_sum_passed(sum, v[j]);
                 }
             }
-            sum = m3_dpp_f32<0x15F>(0.0F, sum); /* lane 15's, to the row */
-        } else {
-#pragma unroll
-            for (int j = 0; j < Q; ++j) {
-                if (16U * j < length) {
-                    sum = m3_block_sum(sum, v[j],
-                                       std::make_integer_sequence<int, 16>());
-                }
-            }
+        }
+        sum = m3_dpp_f32<0x15F>(0.0F, sum); /* lane 15's, to the row */
+        if (HALVES) {
+            /* the whole row's sum, which the second half holds */
+            const float other = m3_other_half(sum);
+
+            sum = second ? sum : other;
         }
         /* A wave whose rows arrived early waits, up to a.hold_ticks after
          * its start, before it stores: its writes then do not compete with
@@ -1103,11 +762,171 @@ void m3_softmax_lane_rows_kernel(m3_softmax_args a)
         if (finite && present) {
             const double inverse = 1.0 / (double)sum;
 
+            if (F32IO || out_dtype == M3N_F32) {
 #pragma unroll
-            for (int j = 0; j < Q; ++j) {
-                put(j, m3_softmax_scale4(v[j], inverse));
+                for (int j = 0; j < Q; ++j) {
+                    put(j, m3_softmax_scale4(v[j], inverse), M3N_F32);
+                }
+            } else if (out_dtype == M3N_F16) {
+#pragma unroll
+                for (int j = 0; j < Q; ++j) {
+                    put(j, m3_softmax_scale4(v[j], inverse), M3N_F16);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < Q; ++j) {
+                    put(j, m3_softmax_scale4(v[j], inverse), M3N_BF16);
+                }
             }
         }
+    }
+}
+
+/* e_j of four inputs against the row maximum m. */
+__device__ __forceinline__ float4 m3_exp4(float4 v, float m,
+                                          const uint64_t *table)
+{
+    return make_float4(m3_expf_with_table(v.x - m, table),
+                       m3_expf_with_table(v.y - m, table),
+                       m3_expf_with_table(v.z - m, table),
+                       m3_expf_with_table(v.w - m, table));
+}
+
+/* Rows of up to 64Q columns, Q = 1, 2 or 4: the lane-row layout (a wave
+ * takes four rows, one per 16-lane DPP row, lane i at columns 4i + 64j ..
+ * +3), so that all lanes work on short rows too. What bounds it is the
+ * latency of one wave's load, exponentials and sum, hidden by the other
+ * waves of its SIMD (at most 56 VGPRs: eight), so a wave takes no more than
+ * four rows and passes the running sum from lane to lane
+ * (m3_block_sum_passed, half the latency of m3_block_sum). The sum stops
+ * after the block that holds the last column other than -inf in any of the
+ * four rows. Measured against a wave of eight rows with lane l at columns
+ * 4l .. 4l + 3 and the sums in LDS: F32 [254200,33] 83 -> 28 us,
+ * [83886,100] 27.3 -> 18.2, [32896,255] 54 -> 19, [32768,256] 14.2 -> 14.0;
+ * BF16 [32768,256] 22.2 -> 15.3; two or four groups of four rows per wave
+ * with their sums side by side: 16.0 and 19.0 for [32768,256].
+ * ELEMENTS: rows of fewer than four columns, element by element. */
+template <int Q, bool F32IO, bool ELEMENTS>
+__global__ __launch_bounds__(256) void m3_softmax_short_rows_kernel(
+    m3_softmax_args a)
+{
+    if (m3_gate_closed(a.list_gate)) {
+        return; /* a check earlier in the list failed */
+    }
+    __shared__ uint64_t exp_table[32];
+    const uint32_t lane = threadIdx.x & 63U;
+    const uint32_t wave = m3_uniform_u32(threadIdx.x >> 6U);
+    const uint32_t sub = lane & 15U;
+    const uint32_t width = a.width;
+    const uint32_t in_dtype = F32IO ? (uint32_t)M3N_F32 : a.in_dtype;
+    const uint32_t out_dtype = F32IO ? (uint32_t)M3N_F32 : a.out_dtype;
+    const uint64_t out_pitch =
+        (uint64_t)width * (out_dtype == M3N_F32 ? 4U : 2U);
+    const uint32_t edge = m3_softmax_edge_block(width, 64U);
+    const uint64_t row =
+        (m3_softmax_block() * kWaves + wave) * 4U + (lane >> 4U);
+    const uint64_t table_word = m3_expf_table[threadIdx.x & 31U];
+    /* rows past the end of the tensor read its last row, store nothing */
+    const uint8_t *in = m3_softmax_row(a, min(row, a.rows - 1U));
+    float4 v[Q];
+
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+        const uint32_t c = sub * 4U + 64U * j;
+
+        v[j] = ELEMENTS
+                   ? m3_softmax_load4_elements(in, c, width, in_dtype)
+                   : m3_softmax_load4<F32IO>(
+                         m3_softmax_source<F32IO>(in, c, width, in_dtype),
+                         in_dtype);
+    }
+    if (threadIdx.x < 32U) {
+        exp_table[threadIdx.x] = table_word;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    float m = -INFINITY;
+    uint32_t last = 0U; /* 1 + index of the last float4 not all -inf */
+
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+        if (!ELEMENTS && (uint32_t)j == edge) {
+            v[j] = m3_softmax_edge4(v[j], sub * 4U + 64U * j, width);
+        }
+        const float t =
+            fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w));
+
+        m = fmaxf(m, t);
+        last = t != -INFINITY ? sub + 16U * j + 1U : last;
+    }
+    m = m3_row16_max(m);
+    const uint32_t length = m3_uniform_u32(m3_wave_max_u32(last));
+    const bool finite = m != INFINITY && m != -INFINITY;
+    auto put = [&](int j, float4 p, uint32_t dtype) {
+        const uint32_t c = sub * 4U + 64U * j;
+
+        if (row < a.rows && c < width) {
+            m3_softmax_put4<F32IO>(a.output + row * out_pitch, c, width,
+                                   dtype, p);
+        }
+    };
+
+    if (M3_ANY_LANE(!finite)) {
+        /* rows whose maximum is +-inf: zeros, or 1/k on k +inf entries */
+        uint32_t count = 0U;
+
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+            count += (v[j].x == INFINITY) + (v[j].y == INFINITY) +
+                     (v[j].z == INFINITY) + (v[j].w == INFINITY);
+        }
+        const float one_over_count = 1.0F / (float)m3_row16_sum(count);
+
+        if (!finite) {
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+                put(j,
+                    make_float4(v[j].x == INFINITY ? one_over_count : 0.0F,
+                                v[j].y == INFINITY ? one_over_count : 0.0F,
+                                v[j].z == INFINITY ? one_over_count : 0.0F,
+                                v[j].w == INFINITY ? one_over_count : 0.0F),
+                    out_dtype);
+            }
+        }
+    }
+    /* e_j against a finite maximum (what the other rows get is not used) */
+    const float shift = finite ? m : 0.0F;
+    float sum = 0.0F;
+
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+        if (16U * j >= length) {
+            v[j] = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+            continue;
+        }
+        v[j] = m3_exp4(v[j], shift, exp_table);
+        sum = m3_block_sum_passed(sum, v[j]);
+    }
+    sum = m3_dpp_f32<0x15F>(0.0F, sum); /* lane 15's, to the row */
+    const double inverse = 1.0 / (double)sum;
+    auto emit = [&](uint32_t dtype) {
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+            const float4 p = m3_softmax_scale4(v[j], inverse);
+
+            if (finite) {
+                put(j, p, dtype);
+            }
+        }
+    };
+
+    if (F32IO || out_dtype == M3N_F32) {
+        emit(M3N_F32);
+    } else if (out_dtype == M3N_F16) {
+        emit(M3N_F16);
+    } else {
+        emit(M3N_BF16);
     }
 }
 
@@ -1121,6 +940,15 @@ __device__ __forceinline__ uint32_t m3_ring_slot(uint32_t f)
     const uint32_t i = f >> 2U;
 
     return (i << 2U) | (((f & 3U) + (i >> 1U) + (i >> 3U)) & 3U);
+}
+
+/* Adds four floats to s in order. */
+__device__ __forceinline__ float m3_add4(float s, float4 e)
+{
+    s = s + e.x;
+    s = s + e.y;
+    s = s + e.z;
+    return s + e.w;
 }
 
 /* Continues the left-to-right sum over one 256-column chunk of a ring line.
@@ -1156,16 +984,6 @@ __device__ __forceinline__ float4 m3_keep4(float4 x, uint32_t mask)
                        m3_bits_f32(m3_f32_bits(x.w) & mask));
 }
 
-/* e_j of four inputs against the row maximum m. */
-__device__ __forceinline__ float4 m3_exp4(float4 v, float m,
-                                          const uint64_t *table)
-{
-    return make_float4(m3_expf_with_table(v.x - m, table),
-                       m3_expf_with_table(v.y - m, table),
-                       m3_expf_with_table(v.z - m, table),
-                       m3_expf_with_table(v.w - m, table));
-}
-
 /* Rows of any width, streamed by a workgroup of four waves that owns R
  * consecutive rows and reads them three times in 256-column chunks, lane l
  * at columns 4l..4l+3 of a chunk:
@@ -1184,7 +1002,7 @@ __device__ __forceinline__ float4 m3_exp4(float4 v, float m,
  * in a row with a finite maximum (later terms are +0). Rows past the end
  * of the tensor repeat the task's first row and store its values again.
  * Rows whose starts are not evenly spaced come from the outer axes. */
-template <bool F32IO, bool VEC>
+template <bool F32IO>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
     m3_softmax_args a)
@@ -1250,7 +1068,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
             for (int k = 0; k < R; ++k) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    x[k][h] = m3_softmax_get4<F32IO, VEC, false>(
+                    x[k][h] = m3_softmax_get4<F32IO, false>(
                         rows[k], chunk[h] * kChunk + lane * 4U, width,
                         in_dtype);
                 }
@@ -1323,7 +1141,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
             for (int k = 0; k < R; ++k) {
-                x[h][k] = m3_softmax_get4<F32IO, VEC, false>(
+                x[h][k] = m3_softmax_get4<F32IO, false>(
                     rows[k], (h * P + producer) * kChunk + lane * 4U, seen,
                     in_dtype);
             }
@@ -1346,7 +1164,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
                 }
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    const float4 v = m3_softmax_get4<F32IO, VEC, false>(
+                    const float4 v = m3_softmax_get4<F32IO, false>(
                         rows[k], ahead * kChunk + lane * 4U, seen, in_dtype);
 
                     if ((step & 1U) != 0U) {
@@ -1400,7 +1218,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
 
 #pragma unroll
             for (int k = 0; k < R; ++k) {
-                x[k] = m3_softmax_get4<F32IO, VEC, false>(
+                x[k] = m3_softmax_get4<F32IO, false>(
                     rows[k], j * kChunk + lane * 4U, width, in_dtype);
             }
 #pragma unroll
@@ -1424,8 +1242,8 @@ __attribute__((amdgpu_waves_per_eu(4))) void m3_softmax_stream_kernel(
                                 (m3_f32_bits(q.z) & ~finite[k])),
                     m3_bits_f32((m3_f32_bits(p.w) & finite[k]) |
                                 (m3_f32_bits(q.w) & ~finite[k])));
-                m3_softmax_put4<F32IO, VEC>(outs[k], j * kChunk + lane * 4U,
-                                            width, out_dtype, q);
+                m3_softmax_put4<F32IO>(outs[k], j * kChunk + lane * 4U, width,
+                                       out_dtype, q);
             }
         }
         /* the LDS of this task is reused by the next */
@@ -1465,10 +1283,9 @@ __device__ __forceinline__ uint32_t m3_wave_scan_u32(uint32_t x)
     return x;
 }
 
-/* Rows of up to 256 NW Q columns (VEC: aligned, a multiple of 4 wide),
- * read once and written once (m3_softmax_wide_kernel): a workgroup of NW
- * waves holds one row in VGPRs, wave w the contiguous columns [256Qw,
- * 256Q(w+1)); lane l of a wave holds columns 256j + 4l .. +3 of them in
+/* Rows of up to 256 NW Q columns, at any alignment, read once and written
+ * once (m3_softmax_wide_kernel): a workgroup of NW waves holds one row in
+ * VGPRs, wave w the contiguous columns [256Qw, 256Q(w+1)); lane l of a wave holds columns 256j + 4l .. +3 of them in
  * block j (j < Q), and DPP row r of the wave (lanes 16r..16r+15) holds the
  * 64 columns 256j + 64r .. of block j, a "segment". Columns past the width
  * read -inf and give e = +0.
@@ -1500,26 +1317,18 @@ __device__ __forceinline__ uint32_t m3_wave_scan_u32(uint32_t x)
  * exponentials. Rows whose maximum is +-inf are written from their inputs
  * (zeros, or 1/k on their k +inf entries). p = e / sum as in the other
  * kernels (m3_softmax_scale4), stored once. */
-/* Loads one row's block j of this lane as F32 (columns past the width
- * read -inf). */
-template <bool F32IO>
+/* Columns c..c+3 of a row; columns past the width read as -inf. A row that
+ * is not RAGGED has a multiple of four columns. */
+template <bool F32IO, bool RAGGED>
 __device__ __forceinline__ float4 m3_wide_load(const uint8_t *in, uint32_t c,
                                                uint32_t width,
                                                uint32_t in_dtype)
 {
-    if (F32IO) {
-        const m3_f32x4 *source =
-            c < width ? (const m3_f32x4 *)(in + 4U * (uint64_t)c)
-                      : (const m3_f32x4 *)&m3_minus_inf4;
-        const m3_f32x4 w = __builtin_nontemporal_load(source);
-
-        return make_float4(w[0], w[1], w[2], w[3]);
+    if (RAGGED) {
+        return m3_softmax_get4<F32IO>(in, c, width, in_dtype);
     }
-    const float4 x = m3_softmax_load4<false>(in, c < width ? c : 0U, in_dtype);
-
-    return c < width ? x
-                     : make_float4(-INFINITY, -INFINITY, -INFINITY,
-                                   -INFINITY);
+    return m3_softmax_load4<F32IO>(
+        m3_softmax_source<F32IO, false>(in, c, width, in_dtype), in_dtype);
 }
 
 /* One wave's share of a row's reductions for the wide kernel: maximum,
@@ -1584,10 +1393,11 @@ constexpr uint32_t kWideSlots = 48U;
 /* Relative distance from a power of two within which an estimated running
  * sum counts as possibly on the other side of it. The in-order F32 sum of
  * n non-negative terms is within (n - 1) 2^-24 of the exact sum, relative,
- * at most 2^-9 for n <= 32768; the estimates (F32 sums of F32 segment
- * totals, fewer than 100 dependent additions) are within 2^-17 of it. So
- * every segment where s crosses a power of two, or whose guessed binade
- * differs from that of s, has an estimate within this margin of one. */
+ * at most 2^-8 for n <= 65536 (and far closer in practice); the estimates
+ * (F32 sums of F32 segment totals, fewer than 100 dependent additions) are
+ * within 2^-17 of it. So every segment where s crosses a power of two, or
+ * whose guessed binade differs from that of s, has an estimate within this
+ * margin of one (a segment that did not would be summed from its input). */
 constexpr float kWideMargin = 1.0F / 256.0F;
 
 /* Sum of x over the lanes below this one (lane 0: +0), in any order: the
@@ -1668,7 +1478,7 @@ __device__ __forceinline__ uint32_t m3_binade(float x)
  * candidates in the row) has its exponentials formed again from the input
  * by the walking wave, the same expf of the same operands, so that the
  * bits never depend on the prediction. */
-template <int Q, int NW, bool F32IO, int WAVES_PER_EU>
+template <int Q, int NW, bool F32IO, bool RAGGED, int WAVES_PER_EU>
 __global__ __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
     m3_softmax_args a)
@@ -1733,7 +1543,23 @@ __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
         ++tag;
 #pragma unroll
         for (int j = 0; j < Q; ++j) {
-            v[j] = m3_wide_load<F32IO>(in, first + 256U * j, width, in_dtype);
+            const uint32_t c = first + 256U * j;
+
+            v[j] = m3_softmax_load4<F32IO>(
+                m3_softmax_source<F32IO, RAGGED>(in, c, width, in_dtype),
+                in_dtype);
+        }
+        if (RAGGED) {
+            /* the block that holds the row's end */
+            const uint32_t edge =
+                m3_softmax_edge_block(width, 256U) - wave * Q;
+
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+                if ((uint32_t)j == edge) {
+                    v[j] = m3_softmax_edge4(v[j], first + 256U * j, width);
+                }
+            }
         }
         /* maximum, +inf count and 1 + the last column that is not -inf
          * (counting the +inf entries of every row, not only of rows whose
@@ -1775,7 +1601,9 @@ __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
                 p.y = v[j].y == INFINITY ? one_over_count : 0.0F;
                 p.z = v[j].z == INFINITY ? one_over_count : 0.0F;
                 p.w = v[j].w == INFINITY ? one_over_count : 0.0F;
-                if (c < width) {
+                if (RAGGED && c < width) {
+                    m3_softmax_put4<F32IO>(out, c, width, out_dtype, p);
+                } else if (c < width) {
                     m3_softmax_store4<F32IO>(out, c, out_dtype, p);
                 }
             }
@@ -2016,7 +1844,8 @@ __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
                     } else {
                         const uint32_t c = 64U * t + 4U * (wl & 15U);
 
-                        e = m3_wide_load<F32IO>(in, c, width, in_dtype);
+                        e = m3_wide_load<F32IO, RAGGED>(in, c, width,
+                                                        in_dtype);
                         if (64U * t < last) {
                             e.x = m3_expf_with_table(e.x - m, exp_table);
                             e.y = m3_expf_with_table(e.y - m, exp_table);
@@ -2054,9 +1883,37 @@ __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
         for (int j = 0; j < Q; ++j) {
             const uint32_t c = column + 256U * j;
 
-            if (c < width) {
+            if (RAGGED ? c + 4U <= width : c < width) {
                 m3_softmax_store4<F32IO>(out, c, out_dtype,
                                          m3_softmax_scale4(v[j], inverse));
+            }
+        }
+        /* the one to three columns after the last whole float4: formed
+         * again from the input (a lane each, the same expf of the same
+         * operands), because picking them out of v costs registers that
+         * the walk needs. In place they are still the input: nothing
+         * above stores them. */
+        if (RAGGED) {
+            const uint32_t tail = m3_lane_index();
+
+            if (wave == 0U && tail < (width & 3U)) {
+                const uint32_t c = (width & ~3U) + tail;
+                const uint32_t raw =
+                    in_dtype == M3N_F32
+                        ? *(const uint32_t *)(in + (uint64_t)c * 4U)
+                        : (uint32_t) *
+                              (const uint16_t *)(in + (uint64_t)c * 2U);
+                const float e = m3_expf_with_table(
+                    m3_bits_f32(m3_load_as_f32_bits(raw, in_dtype)) - m,
+                    exp_table);
+                const uint32_t bits = m3_store_from_f32_bits(
+                    m3_f32_bits(m3_softmax_scale(e, inverse)), out_dtype);
+
+                if (out_dtype == M3N_F32) {
+                    *(uint32_t *)(out + (uint64_t)c * 4U) = bits;
+                } else {
+                    *(uint16_t *)(out + (uint64_t)c * 2U) = (uint16_t)bits;
+                }
             }
         }
         /* the next row writes part_* and totals (read before the last
@@ -2068,21 +1925,22 @@ __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void m3_softmax_wide_kernel(
 typedef void (*m3_softmax_launcher)(dim3, hipStream_t, hipEvent_t,
                                     hipEvent_t, m3_softmax_args);
 
-template <int VPL, int R, int DEPTH, bool F32IO, bool VEC>
-void m3_launch_rows(dim3 grid, hipStream_t stream, hipEvent_t start,
-                    hipEvent_t stop, m3_softmax_args args)
+template <int Q, bool F32IO, bool ELEMENTS>
+void m3_launch_short_rows(dim3 grid, hipStream_t stream, hipEvent_t start,
+                          hipEvent_t stop, m3_softmax_args args)
 {
-    hipExtLaunchKernelGGL((m3_softmax_rows_kernel<VPL, R, DEPTH, F32IO, VEC>),
-                          grid, dim3(kThreads), 0, stream, start, stop, 0U,
-                          args);
+    hipExtLaunchKernelGGL(
+        (m3_softmax_short_rows_kernel<Q, F32IO, ELEMENTS>), grid,
+        dim3(kThreads), 0, stream, start, stop, 0U, args);
 }
 
-template <int Q, bool FULL, bool F32IO>
+template <int Q, bool FULL, bool HALVES, bool F32IO>
 void m3_launch_lane_rows(dim3 grid, hipStream_t stream, hipEvent_t start,
                          hipEvent_t stop, m3_softmax_args args)
 {
-    hipExtLaunchKernelGGL((m3_softmax_lane_rows_kernel<Q, FULL, F32IO>), grid,
-                          dim3(kThreads), 0, stream, start, stop, 0U, args);
+    hipExtLaunchKernelGGL(
+        (m3_softmax_lane_rows_kernel<Q, FULL, HALVES, F32IO>), grid,
+        dim3(kThreads), 0, stream, start, stop, 0U, args);
 }
 
 /* Waves per SIMD the wide kernel is built for: seven (at most 72 VGPRs;
@@ -2095,60 +1953,34 @@ void m3_launch_lane_rows(dim3 grid, hipStream_t stream, hipEvent_t start,
  * workgroups of 64 values per lane with F32 I/O (ten and five per CU),
  * four-wave ones of 48 with 16-bit I/O and eight-wave ones of 40; four
  * (128 VGPRs) for the rest, which would spill registers at 96. */
-template <int Q, int NW, bool F32IO>
+template <int Q, int NW, bool F32IO, bool RAGGED>
 constexpr int m3_wide_waves_per_eu()
 {
     return NW == 2 && Q == 8 ? 7
            : Q == 12 && F32IO ? 6
+           : Q == 16 && RAGGED ? 4
            : (NW <= 4 && (F32IO || Q <= 12)) || (NW == 8 && Q <= 10) ? 5
                                                                     : 4;
 }
 
-template <int Q, int NW, bool F32IO>
+template <int Q, int NW, bool F32IO, bool RAGGED>
 void m3_launch_wide(dim3 grid, hipStream_t stream, hipEvent_t start,
                     hipEvent_t stop, m3_softmax_args args)
 {
-    hipExtLaunchKernelGGL((m3_softmax_wide_kernel<Q, NW, F32IO,
-                                                  m3_wide_waves_per_eu<Q, NW, F32IO>()>),
-                          grid, dim3(64 * NW), 0, stream, start, stop, 0U,
-                          args);
+    hipExtLaunchKernelGGL(
+        (m3_softmax_wide_kernel<Q, NW, F32IO, RAGGED,
+                                m3_wide_waves_per_eu<Q, NW, F32IO,
+                                                     RAGGED>()>),
+        grid, dim3(64 * NW), 0, stream, start, stop, 0U, args);
 }
 
-template <bool F32IO, bool VEC>
+template <bool F32IO>
 void m3_launch_stream(dim3 grid, hipStream_t stream, hipEvent_t start,
                       hipEvent_t stop, m3_softmax_args args)
 {
-    hipExtLaunchKernelGGL((m3_softmax_stream_kernel<F32IO, VEC>), grid,
+    hipExtLaunchKernelGGL((m3_softmax_stream_kernel<F32IO>), grid,
                           dim3(kThreads), 0, stream, start, stop, 0U, args);
 }
-
-struct m3_rows_variant {
-    uint32_t vectors_per_lane;
-    uint32_t rows_per_wave;
-    m3_softmax_launcher f32;      /* F32 in and out, VEC rows */
-    m3_softmax_launcher other;    /* any dtypes, VEC rows */
-    m3_softmax_launcher elements; /* any dtypes, element-wise rows */
-};
-
-/* Wave-independent variants; the first whose width class fits is used.
- * Rows per wave and sum prefetch depth are chosen for four waves per SIMD
- * at widths up to 1024 with F32 in and out; the width-2048 instance and
- * the 16-bit-IO instances from width 1024 take more VGPRs and run three
- * waves per SIMD. */
-const m3_rows_variant m3_rows_variants[] = {
-    {1U, 8U, &m3_launch_rows<1, 8, 8, true, true>,
-     &m3_launch_rows<1, 8, 8, false, true>,
-     &m3_launch_rows<1, 8, 8, false, false>},
-    {2U, 4U, &m3_launch_rows<2, 4, 8, true, true>,
-     &m3_launch_rows<2, 4, 8, false, true>,
-     &m3_launch_rows<2, 4, 8, false, false>},
-    {4U, 4U, &m3_launch_rows<4, 4, 4, true, true>,
-     &m3_launch_rows<4, 4, 4, false, true>,
-     &m3_launch_rows<4, 4, 4, false, false>},
-    {8U, 2U, &m3_launch_rows<8, 2, 4, true, true>,
-     &m3_launch_rows<8, 2, 4, false, true>,
-     &m3_launch_rows<8, 2, 4, false, false>},
-};
 
 struct m3_softmax_general_args {
     const uint8_t *input;
@@ -2276,7 +2108,6 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
     const uint8_t *in = (const uint8_t *)input->base + input->byte_offset;
     uint8_t *out = (uint8_t *)output->base + output->byte_offset;
     uint32_t in_size = (uint32_t)m3_dtype_bytes(input->dtype);
-    uint32_t out_size = (uint32_t)m3_dtype_bytes(output->dtype);
 
     /* Outer axes (all but the last) of the input, coalesced. */
     m3_hip_view outer = *input;
@@ -2297,10 +2128,6 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
 
     if (columns_contiguous) {
         m3_softmax_args args;
-        /* VEC rows: every row start aligned for 4-element accesses */
-        bool vec = width % 4U == 0U &&
-                   ((uintptr_t)in % (4U * in_size)) == 0U &&
-                   ((uintptr_t)out % (4U * out_size)) == 0U;
         const bool f32 =
             input->dtype == M3_HIP_F32 && output->dtype == M3_HIP_F32;
 
@@ -2315,64 +2142,67 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
         if (uniform_rows) {
             args.outer_rank = 1U;
             args.row_stride = rows == 1U ? 0U : (uint64_t)plan.strides[0][0];
-            vec = vec && args.row_stride % (4U * in_size) == 0U;
         } else {
             args.outer_rank = plan.rank;
             for (uint32_t axis = 0U; axis < plan.rank; ++axis) {
                 args.outer_shape[axis] = plan.shape[axis];
                 args.outer_strides[axis] = plan.strides[0][axis];
-                vec = vec && (uint64_t)plan.strides[0][axis] %
-                                     (4U * in_size) ==
-                                 0U;
             }
         }
-        /* VEC rows of 513..1024 columns, and of 257..512 columns with a
-         * 16-bit input or output: the lane-row kernel, 16 or 8 float4 per
-         * lane (index: [wide][full][f32]). F32 rows of 257..512 columns
-         * measured the same or faster on the rows kernel (49.5 against
-         * 49.6 us for [65536,512], 23.4 against 22.2 us for [32768,300]);
-         * with 16-bit I/O the lane-row kernel is faster at every width
-         * (56.6 against 73.3 us for [65536,512] BF16, 38.5 against 58.1 us
-         * for [16384,1024] BF16). */
-        static const m3_softmax_launcher lane_launchers[2][2][2] = {
-            {{&m3_launch_lane_rows<8, false, false>,
-              &m3_launch_lane_rows<8, false, true>},
-             {&m3_launch_lane_rows<8, true, false>,
-              &m3_launch_lane_rows<8, true, true>}},
-            {{&m3_launch_lane_rows<16, false, false>,
-              &m3_launch_lane_rows<16, false, true>},
-             {&m3_launch_lane_rows<16, true, false>,
-              &m3_launch_lane_rows<16, true, true>}}};
+        /* Rows of up to 256 columns: the narrowest class that holds them
+         * (index: [Q = 1, 2, 4][F32 I/O]) */
+        if (width <= 256U) {
+            static const m3_softmax_launcher launchers[3][2] = {
+                {&m3_launch_short_rows<1, false, false>,
+                 &m3_launch_short_rows<1, true, false>},
+                {&m3_launch_short_rows<2, false, false>,
+                 &m3_launch_short_rows<2, true, false>},
+                {&m3_launch_short_rows<4, false, false>,
+                 &m3_launch_short_rows<4, true, false>}};
+            const uint32_t which = width <= 64U ? 0U : width <= 128U ? 1U : 2U;
+            const dim3 grid = m3_softmax_grid((rows + 4U * kWaves - 1U) /
+                                              (4U * kWaves));
+            const m3_softmax_launcher launcher =
+                width < 4U ? &m3_launch_short_rows<1, false, true>
+                           : launchers[which][f32];
+
+            return m3_hip_launch(
+                device, "m3_softmax_rows",
+                [&](hipEvent_t start, hipEvent_t stop) {
+                    launcher(grid, device->stream, start, stop, args);
+                },
+                message, capacity);
+        }
+        /* Rows of 257..2048 columns: the lane-row kernel, 8 or 16 float4
+         * per lane and, beyond 1024 columns, a row in two halves
+         * (index: [class][full][F32 I/O]). */
+        static const m3_softmax_launcher lane_launchers[3][2][2] = {
+            {{&m3_launch_lane_rows<8, false, false, false>,
+              &m3_launch_lane_rows<8, false, false, true>},
+             {&m3_launch_lane_rows<8, true, false, false>,
+              &m3_launch_lane_rows<8, true, false, true>}},
+            {{&m3_launch_lane_rows<16, false, false, false>,
+              &m3_launch_lane_rows<16, false, false, true>},
+             {&m3_launch_lane_rows<16, true, false, false>,
+              &m3_launch_lane_rows<16, true, false, true>}},
+            {{&m3_launch_lane_rows<16, false, true, false>,
+              &m3_launch_lane_rows<16, false, true, true>},
+             {&m3_launch_lane_rows<16, false, true, false>,
+              &m3_launch_lane_rows<16, false, true, true>}}};
+        const uint32_t lane_class = width <= 512U    ? 0U
+                                    : width <= 1024U ? 1U
+                                                     : 2U;
+        const uint32_t lane_rows = lane_class == 2U ? 2U : 4U; /* per wave */
         const uint64_t lane_blocks =
-            (rows + 4U * kWaves - 1U) / (4U * kWaves);
-        const uint32_t lane_q = width > 1024U           ? 0U
-                                : width > 512U          ? 16U
-                                : width > 256U && !f32 ? 8U
-                                                        : 0U;
+            (rows + lane_rows * kWaves - 1U) / (lane_rows * kWaves);
 
-        if (vec && lane_q != 0U && lane_blocks <= kMaxLaneGrid) {
-            const dim3 grid((uint32_t)lane_blocks);
-            /* late: 0.95 times the time the launch's reads take at peak
-             * HBM bandwidth (8.0 us for [16,1024,1024] F32; in bench.py on
-             * one box with the store hold, three rounds: 6.0 us 22.8-23.5,
-             * 7.1 us 22.8-23.7, 8.0 us 22.7-22.9, 9.0 us 23.5), at least 3 us
-             * (about the latency of a first load), unless
-             * M3_HIP_SOFTMAX_LATE_US sets it */
-            const double late_us =
-                device->softmax_late_us >= 0.0F
-                    ? (double)device->softmax_late_us
-                    : std::max(kLateFloorUs,
-                               kLateFactor * (double)rows * (double)width *
-                                   in_size / kHbmBytesPerUs);
-            const double ticks = late_us * device->wall_clock_khz / 1000.0;
-
-            args.late_ticks = device->wall_clock_khz == 0U || ticks >= 4.0e9
-                                  ? 0xffffffffU
-                                  : (uint32_t)ticks;
-            /* hold: 1.25 times the time the launch's reads take at peak
-             * HBM bandwidth (10.5 us for [16,1024,1024] F32; in bench.py on
-             * one box, three rounds: 9.0 us 23.1-23.4, 10.0 us 23.0-23.2,
-             * 10.5 us 22.7-23.0, 11.0 us 23.5-23.9), when every
+        if (width <= 2048U) {
+            const dim3 grid = m3_softmax_grid(lane_blocks);
+            /* hold: 1.07 times the time the launch's reads take at peak
+             * HBM bandwidth (9.0 us for [16,1024,1024] F32, a pass among
+             * others on one box: no hold 22.8 us causal and 27.0 not, 9.0 us
+             * 22.4 and 27.2, 10.0 us 23.6 and 27.5, 10.5 us 24.3 and 27.5;
+             * causal [16,1000,1000]: 31.6 without, 28.9 at 9.0), when every
              * wave of the launch is resident at once so that all its reads
              * are issued at the start; otherwise none. M3_HIP_SOFTMAX_HOLD_US
              * sets it. */
@@ -2381,7 +2211,7 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
             const double hold_us =
                 device->softmax_hold_us >= 0.0F
                     ? (double)device->softmax_hold_us
-                : (rows + 3U) / 4U <= resident
+                : (rows + lane_rows - 1U) / lane_rows <= resident
                     ? kHoldFactor * (double)rows * (double)width * in_size /
                           kHbmBytesPerUs
                     : 0.0;
@@ -2391,7 +2221,8 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                                   ? 0U
                                   : (uint32_t)hold;
             const m3_softmax_launcher launcher =
-                lane_launchers[lane_q == 16U][width == 64U * lane_q][f32];
+                lane_launchers[lane_class][width == 512U || width == 1024U]
+                              [f32];
 
             return m3_hip_launch(
                 device, "m3_softmax_rows",
@@ -2400,41 +2231,27 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                 },
                 message, capacity);
         }
-        for (const m3_rows_variant &variant : m3_rows_variants) {
-            if (width > kChunk * variant.vectors_per_lane) {
-                continue;
-            }
-            uint64_t tasks =
-                (rows + variant.rows_per_wave - 1U) / variant.rows_per_wave;
-            uint64_t blocks = (tasks + kWaves - 1U) / kWaves;
-            dim3 grid((uint32_t)(blocks < kMaxGrid ? blocks : kMaxGrid));
-            m3_softmax_launcher launcher =
-                !vec ? variant.elements : f32 ? variant.f32 : variant.other;
-
-            return m3_hip_launch(
-                device, "m3_softmax_rows",
-                [&](hipEvent_t start, hipEvent_t stop) {
-                    launcher(grid, device->stream, start, stop, args);
-                },
-                message, capacity);
-        }
-        /* VEC rows of 2049..32768 columns: a workgroup per row at a time,
-         * each row read once, the in-order sum in parallel. */
-        if (vec && width > 2048U && width <= 32768U) {
+        /* Rows of 2049..65536 columns: a workgroup per row at a time, each
+         * row read once, the in-order sum in parallel. */
+        if (width <= 65536U) {
             /* the smallest row class that holds the width: NW waves of Q
              * float4 per lane, 256 NW Q columns; one workgroup per row (the
              * hardware hands a CU's next row to whichever of its workgroups
              * ends first) */
 #define M3_WIDE_ENTRY(Q, NW)                                                  \
     {1024U * (Q) * (NW) / 4U,                                                 \
-     {&m3_launch_wide<Q, NW, false>, &m3_launch_wide<Q, NW, true>}}
+     {{&m3_launch_wide<Q, NW, false, false>,                                  \
+       &m3_launch_wide<Q, NW, true, false>},                                  \
+      {&m3_launch_wide<Q, NW, false, true>,                                   \
+       &m3_launch_wide<Q, NW, true, true>}}}
             static const struct {
                 uint32_t columns;
-                m3_softmax_launcher launch[2];
+                m3_softmax_launcher launch[2][2]; /* [ragged][F32 I/O] */
             } classes[] = {M3_WIDE_ENTRY(8, 2),  M3_WIDE_ENTRY(16, 2),
                            M3_WIDE_ENTRY(12, 4), M3_WIDE_ENTRY(16, 4),
                            M3_WIDE_ENTRY(10, 8), M3_WIDE_ENTRY(12, 8),
-                           M3_WIDE_ENTRY(16, 8)};
+                           M3_WIDE_ENTRY(16, 8),  M3_WIDE_ENTRY(12, 16),
+                           M3_WIDE_ENTRY(16, 16)};
 #undef M3_WIDE_ENTRY
             uint32_t which = 0U;
 
@@ -2447,7 +2264,7 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                     ? device->softmax_wide_grid
                     : kMaxGrid;
             const dim3 grid((uint32_t)(rows < cap ? rows : cap));
-            const m3_softmax_launcher launcher = classes[which].launch[f32];
+            const m3_softmax_launcher launcher = classes[which].launch[width % 4U != 0U][f32];
 
             return m3_hip_launch(
                 device, "m3_softmax_rows_wide",
@@ -2456,50 +2273,12 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                 },
                 message, capacity);
         }
-        /* Rows wider than the register variants: whole rows in LDS when
-         * they fit the dynamic LDS a launch gets without opting in. */
-        uint32_t pitch_bytes = ((uint32_t)width + kPad) * 4U;
-        uint32_t budget = device->lds_per_block > kStaticLds
-                              ? device->lds_per_block - kStaticLds
-                              : 0U;
-
-        budget = budget > kTiledLdsCap ? kTiledLdsCap : budget;
-        uint32_t tile_rows = width <= kMaxWidth ? budget / pitch_bytes : 0U;
-
-        tile_rows = tile_rows > kMaxTileRows ? kMaxTileRows : tile_rows;
-        if (vec && uniform_rows && tile_rows != 0U) {
-            args.tile_rows = tile_rows;
-            uint64_t tiles = (rows + tile_rows - 1U) / tile_rows;
-            uint32_t blocks =
-                (uint32_t)(tiles < (uint64_t)device->compute_units * 8U
-                               ? tiles
-                               : (uint64_t)device->compute_units * 8U);
-            size_t lds_bytes = (size_t)tile_rows * pitch_bytes;
-
-            return m3_hip_launch(
-                device, "m3_softmax_rows_lds",
-                [&](hipEvent_t start, hipEvent_t stop) {
-                    if (f32) {
-                        hipExtLaunchKernelGGL((m3_softmax_tiled_kernel<true>),
-                                              dim3(blocks), dim3(kThreads),
-                                              lds_bytes, device->stream, start,
-                                              stop, 0U, args);
-                    } else {
-                        hipExtLaunchKernelGGL((m3_softmax_tiled_kernel<false>),
-                                              dim3(blocks), dim3(kThreads),
-                                              lds_bytes, device->stream, start,
-                                              stop, 0U, args);
-                    }
-                },
-                message, capacity);
-        }
         /* Any other row: streamed through three passes, a workgroup per
          * kStreamRows rows. */
         uint64_t tasks = (rows + kStreamRows - 1U) / kStreamRows;
         dim3 grid((uint32_t)(tasks < kMaxGrid ? tasks : kMaxGrid));
-        m3_softmax_launcher launcher = !vec ? &m3_launch_stream<false, false>
-                                       : f32 ? &m3_launch_stream<true, true>
-                                             : &m3_launch_stream<false, true>;
+        m3_softmax_launcher launcher =
+            f32 ? &m3_launch_stream<true> : &m3_launch_stream<false>;
 
         return m3_hip_launch(
             device, "m3_softmax_rows_streamed",
