@@ -15,10 +15,13 @@
  * written with streaming stores), or, for the cheap conversions of a
  * tensor whose lanes are all resident at once, its held form (all loads,
  * then the stores after a timed wait);
+ * an input whose unit-stride axis is another than the output's innermost
+ * one (a permuted view) goes through transposing tiles in LDS; other
  * strided inputs run a per-element kernel over the coalesced index space.
  */
 #include "m3_hip_internal.h"
 
+#include <algorithm>
 #include <cstring>
 
 namespace {
@@ -228,6 +231,210 @@ __global__ __launch_bounds__(256) void m3_copy_bytes_kernel(
     }
 }
 
+/* ---- transposing tiles ------------------------------------------------------ */
+
+/* An input whose consecutive elements lie along another axis (u) than the
+ * output's (n): the output's innermost axis n steps by n_stride bytes in
+ * the input, and axis u, whose consecutive elements are out_u_stride
+ * elements apart in the output, is the input's unit-stride one. */
+struct m3_transpose_args {
+    const uint8_t *input;
+    uint8_t *output;
+    uint32_t n;
+    uint32_t u;
+    int64_t n_stride;
+    uint64_t out_u_stride;
+    uint32_t tiles; /* tiles_n * tiles_u * the outer axes' extents */
+    m3_fast_div tiles_n;
+    m3_fast_div tiles_u;
+    uint32_t outer_rank;
+    uint64_t outer_shape[M3_HIP_MAX_RANK];
+    int64_t outer_in[M3_HIP_MAX_RANK];   /* bytes */
+    uint64_t outer_out[M3_HIP_MAX_RANK]; /* elements */
+    m3_hip_gate list_gate;
+};
+
+/* The smallest extent of both axes for which tiles are used: at 16 a tile's
+ * lanes are a quarter (u) or an eighth (n) full, and [1,50000,33], half
+ * full, takes 6 us against 20 for one element per lane; below it the
+ * kernel would mostly read and write nothing. */
+constexpr uint32_t kTransposeLeast = 16U;
+constexpr uint32_t kTileU = 64U;
+constexpr uint32_t kTileN = 128U;
+constexpr uint32_t kXcds = 8U;
+constexpr uint32_t kMaxTransposeGrid = 1U << 20; /* workgroups; they loop */
+
+/* Four consecutive elements at any alignment, zero-extended. */
+template <uint32_t SIZE>
+__device__ __forceinline__ uint4 m3_load4_any(const uint8_t *p)
+{
+    if (SIZE == 4U) {
+        const m3_u32x4_any w = *(const m3_u32x4_any *)p;
+
+        return make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    const m3_u32x2_any h = *(const m3_u32x2_any *)p;
+
+    return make_uint4(h[0] & 0xffffU, h[0] >> 16U, h[1] & 0xffffU,
+                      h[1] >> 16U);
+}
+
+__device__ __forceinline__ void m3_store4_any(uint8_t *p, uint4 v)
+{
+    const m3_u32x4_any w = {v.x, v.y, v.z, v.w};
+
+    __builtin_nontemporal_store(w, (m3_u32x4_any *)p);
+}
+
+__device__ __forceinline__ void m3_store4_any(uint8_t *p, uint2 v)
+{
+    const m3_u32x2_any w = {v.x, v.y};
+
+    __builtin_nontemporal_store(w, (m3_u32x2_any *)p);
+}
+
+/* A tile of 64 (u) by 128 (n) elements through LDS: each lane reads four
+ * elements along u at four consecutive n, transposes the 4 x 4 block in
+ * registers, converts it and writes it as four vectors along n; the tile is
+ * then stored along n. Both sides of memory move whole runs (256 bytes and
+ * 512 for 4-byte elements), at any alignment. The vector slot of a row in
+ * LDS is rotated by an exclusive or with the row's group of four, so that
+ * the lanes of a write (consecutive u) and of a read (consecutive n) both
+ * fall on distinct banks. IN == OUT copies raw elements.
+ *
+ * Bound by HBM; against one element per lane with 64-bit divisions and
+ * strided reads: F32 [2,8191,512] 36.5 -> 13.9 us (4.8 TB/s; 9.9 us at
+ * length 8192, whose stores are aligned), F32 [1,32000,1024] 610 -> 40.5,
+ * BF16 [2,8191,512] 37.4 -> 7.8, BF16 to F32 [4,8000,1001] 283 -> 31.
+ * Nontemporal stores against ordinary ones: 9.9 against 11.9 us at length
+ * 8192, 31 against 36 for [4,8000,1001], 13.0 against 12.4 at 8191. Tiles
+ * of 64 along n: 14.5 at 8191, 64 against 49 for F32 [1,31999,1024];
+ * neighbouring tiles dealt to different XCDs: 47 against 40.5. */
+template <uint32_t IN, uint32_t OUT>
+__global__ __launch_bounds__(256) void m3_transpose_kernel(m3_transpose_args a)
+{
+    if (m3_gate_closed(a.list_gate)) {
+        return; /* a check earlier in the list failed */
+    }
+    constexpr uint32_t in_size = m3_size_of(IN);
+    constexpr uint32_t out_size = m3_size_of(OUT);
+    using out_io = m3_vec_io<out_size>;
+    using slot_type = typename out_io::type;
+    constexpr uint32_t kSlots = kTileN / 4U; /* vectors per tile row */
+    __shared__ slot_type lds[kTileU][kSlots];
+    const uint32_t ul = threadIdx.x & 15U;
+    const uint32_t nl = threadIdx.x >> 4U;
+
+    for (uint32_t block = blockIdx.x; block < a.tiles; block += gridDim.x) {
+        uint32_t tile = block;
+
+        if (gridDim.x == a.tiles) {
+            /* neighbouring tiles, which share lines at their edges, on one
+             * XCD (workgroups go round the XCDs) */
+            const uint32_t xcd = block % kXcds;
+            const uint32_t share = a.tiles / kXcds;
+            const uint32_t rest = a.tiles % kXcds;
+
+            tile = xcd * share + min(xcd, rest) + block / kXcds;
+        }
+        const uint32_t q = m3_fast_div_q(a.tiles_n, tile);
+        const uint32_t tile_n = (tile - q * a.tiles_n.divisor) * kTileN;
+        uint64_t outer = m3_fast_div_q(a.tiles_u, q);
+        const uint32_t tile_u =
+            (q - (uint32_t)outer * a.tiles_u.divisor) * kTileU;
+        const uint8_t *in = a.input;
+        uint8_t *out = a.output;
+
+        for (int axis = (int)a.outer_rank - 1; axis >= 0; --axis) {
+            const uint64_t dim = a.outer_shape[axis];
+            const uint64_t rest = outer / dim;
+            const uint64_t c = outer - rest * dim;
+
+            in += (int64_t)c * a.outer_in[axis];
+            out += c * a.outer_out[axis] * out_size;
+            outer = rest;
+        }
+        /* the tile's last partial vector along u is read from the row's
+         * last four elements (u >= 4), which repeat the lanes before it */
+        const uint32_t u0 = min(tile_u + 4U * ul, a.u - 4U);
+        const bool inside = tile_u + 4U * ul < a.u;
+        uint4 v[kSlots / 16U][4];
+
+#pragma unroll
+        for (uint32_t k = 0U; k < kSlots / 16U; ++k) {
+#pragma unroll
+            for (uint32_t i = 0U; i < 4U; ++i) {
+                const uint32_t n = tile_n + 64U * k + 4U * nl + i;
+
+                v[k][i] = m3_load4_any<in_size>(
+                    in + (int64_t)min(n, a.n - 1U) * a.n_stride +
+                    (uint64_t)u0 * in_size);
+            }
+        }
+#pragma unroll
+        for (uint32_t k = 0U; k < kSlots / 16U; ++k) {
+            const uint4 t[4] = {
+                make_uint4(v[k][0].x, v[k][1].x, v[k][2].x, v[k][3].x),
+                make_uint4(v[k][0].y, v[k][1].y, v[k][2].y, v[k][3].y),
+                make_uint4(v[k][0].z, v[k][1].z, v[k][2].z, v[k][3].z),
+                make_uint4(v[k][0].w, v[k][1].w, v[k][2].w, v[k][3].w)};
+
+#pragma unroll
+            for (uint32_t e = 0U; e < 4U; ++e) {
+                /* rows before the tile wrap and are dropped */
+                const uint32_t r = u0 + e - tile_u;
+                uint4 w = t[e];
+
+                if (IN != OUT) {
+                    w = make_uint4(m3_convert<IN, OUT>(w.x),
+                                   m3_convert<IN, OUT>(w.y),
+                                   m3_convert<IN, OUT>(w.z),
+                                   m3_convert<IN, OUT>(w.w));
+                }
+                if (inside && r < kTileU) {
+                    lds[r][(16U * k + nl) ^ ((r >> 2U) & 15U)] =
+                        out_io::pack(w);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t s = 0U; s < kTileU * kSlots / kThreads; ++s) {
+            const uint32_t index = s * kThreads + threadIdx.x;
+            const uint32_t r = index / kSlots;
+            const uint32_t slot = index % kSlots;
+            const uint32_t n = tile_n + 4U * slot;
+
+            if (tile_u + r >= a.u || n >= a.n) {
+                continue;
+            }
+            const slot_type w = lds[r][slot ^ ((r >> 2U) & 15U)];
+            uint8_t *p =
+                out + ((tile_u + r) * a.out_u_stride + n) * out_size;
+
+            if (n + 4U <= a.n) {
+                m3_store4_any(p, w);
+                continue;
+            }
+            const uint4 x = out_io::unpack(w);
+            const uint32_t rest[3] = {x.x, x.y, x.z};
+
+#pragma unroll
+            for (uint32_t i = 0U; i < 3U; ++i) {
+                if (n + i >= a.n) {
+                    continue;
+                }
+                if (out_size == 4U) {
+                    ((uint32_t *)p)[i] = rest[i];
+                } else {
+                    ((uint16_t *)p)[i] = (uint16_t)rest[i];
+                }
+            }
+        }
+        __syncthreads(); /* the next tile overwrites the LDS */
+    }
+}
+
 /* Groups of four elements per lane of the held form. */
 constexpr int kHeldGroups = 8;
 /* Workgroups per CU that are all resident at once in the held form (its
@@ -369,6 +576,95 @@ m3_cast_launcher m3_cast_vec_launcher(uint32_t in, uint32_t out)
     return nullptr;
 }
 
+typedef void (*m3_transpose_launcher)(dim3, hipStream_t, hipEvent_t,
+                                      hipEvent_t, m3_transpose_args);
+
+template <uint32_t IN, uint32_t OUT>
+void m3_launch_transpose(dim3 grid, hipStream_t stream, hipEvent_t start,
+                         hipEvent_t stop, m3_transpose_args args)
+{
+    hipExtLaunchKernelGGL((m3_transpose_kernel<IN, OUT>), grid,
+                          dim3(kThreads), 0, stream, start, stop, 0U, args);
+}
+
+/* The transposing kernel of a conversion; copies of one element size share
+ * one. */
+m3_transpose_launcher m3_transpose_of(uint32_t in, uint32_t out)
+{
+    static const m3_transpose_launcher launchers[4][4] = {
+        {&m3_launch_transpose<M3N_F32, M3N_F32>,
+         &m3_launch_transpose<M3N_F32, M3N_F16>,
+         &m3_launch_transpose<M3N_F32, M3N_BF16>,
+         &m3_launch_transpose<M3N_F32, M3N_I32>},
+        {&m3_launch_transpose<M3N_F16, M3N_F32>,
+         &m3_launch_transpose<M3N_F16, M3N_F16>,
+         &m3_launch_transpose<M3N_F16, M3N_BF16>,
+         &m3_launch_transpose<M3N_F16, M3N_I32>},
+        {&m3_launch_transpose<M3N_BF16, M3N_F32>,
+         &m3_launch_transpose<M3N_BF16, M3N_F16>,
+         &m3_launch_transpose<M3N_F16, M3N_F16>,
+         &m3_launch_transpose<M3N_BF16, M3N_I32>},
+        {&m3_launch_transpose<M3N_I32, M3N_F32>,
+         &m3_launch_transpose<M3N_I32, M3N_F16>,
+         &m3_launch_transpose<M3N_I32, M3N_BF16>,
+         &m3_launch_transpose<M3N_F32, M3N_F32>}};
+
+    return launchers[in][out];
+}
+
+/* Fills `args` when the plan (operand 1 the input) is one that the
+ * transposing kernel takes: the innermost axis strided in the input, some
+ * other axis of unit stride there, both of at least kTransposeLeast. */
+bool m3_plan_transpose(const m3_index_plan &plan, uint32_t in_size,
+                       m3_transpose_args *args)
+{
+    const uint32_t inner = plan.rank - 1U;
+    uint64_t out_strides[M3_HIP_MAX_RANK];
+    uint64_t elements = 1U;
+    uint64_t outer = 1U;
+    uint32_t unit = plan.rank;
+
+    for (int axis = (int)inner; axis >= 0; --axis) {
+        out_strides[axis] = elements;
+        elements *= plan.shape[axis];
+        if (plan.strides[1][axis] == (int64_t)in_size) {
+            unit = (uint32_t)axis;
+        }
+    }
+    if (unit >= inner || plan.shape[inner] < kTransposeLeast ||
+        plan.shape[unit] < kTransposeLeast ||
+        plan.shape[inner] > 0x7fffffffULL ||
+        plan.shape[unit] > 0x7fffffffULL) {
+        return false;
+    }
+    for (uint32_t axis = 0U; axis < inner; ++axis) {
+        if (axis == unit) {
+            continue;
+        }
+        args->outer_shape[args->outer_rank] = plan.shape[axis];
+        args->outer_in[args->outer_rank] = plan.strides[1][axis];
+        args->outer_out[args->outer_rank] = out_strides[axis];
+        args->outer_rank += 1U;
+        outer *= plan.shape[axis];
+    }
+    const uint64_t tiles_n = (plan.shape[inner] + kTileN - 1U) / kTileN;
+    const uint64_t tiles_u = (plan.shape[unit] + kTileU - 1U) / kTileU;
+
+    /* two factors below 2^32 each, checked before the third */
+    if (tiles_n * tiles_u > 0x7fffffffULL ||
+        outer > 0x7fffffffULL / (tiles_n * tiles_u)) {
+        return false;
+    }
+    args->n = (uint32_t)plan.shape[inner];
+    args->u = (uint32_t)plan.shape[unit];
+    args->n_stride = plan.strides[1][inner];
+    args->out_u_stride = out_strides[unit];
+    args->tiles = (uint32_t)(tiles_n * tiles_u * outer);
+    args->tiles_n = m3_fast_div_make((uint32_t)tiles_n);
+    args->tiles_u = m3_fast_div_make((uint32_t)tiles_u);
+    return true;
+}
+
 const char *m3_cast_kernel_name(uint32_t in, uint32_t out)
 {
     static const char *const names[4][4] = {
@@ -441,6 +737,25 @@ int m3_launch_unary(m3_hip_device *device, const m3_hip_view *input,
                 },
                 message, capacity);
         }
+    }
+    m3_transpose_args transpose;
+
+    std::memset(&transpose, 0, sizeof(transpose));
+    if (m3_plan_transpose(plan, (uint32_t)m3_dtype_bytes(input->dtype),
+                          &transpose)) {
+        const m3_transpose_launcher launcher =
+            m3_transpose_of(input->dtype, output->dtype);
+        const dim3 grid(std::min(transpose.tiles, kMaxTransposeGrid));
+
+        transpose.list_gate = device->gate;
+        transpose.input = in;
+        transpose.output = out;
+        return m3_hip_launch(
+            device, name,
+            [&](hipEvent_t start, hipEvent_t stop) {
+                launcher(grid, device->stream, start, stop, transpose);
+            },
+            message, capacity);
     }
     m3_strided_args args;
 

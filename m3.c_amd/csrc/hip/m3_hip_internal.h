@@ -210,6 +210,12 @@ int m3_hip_launch(m3_hip_device *device, const char *name, Launch launch,
 typedef uint32_t m3_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t m3_u32x2 __attribute__((ext_vector_type(2)));
 typedef float m3_f32x4 __attribute__((ext_vector_type(4)));
+/* The same read and written at any element alignment: gfx950 serves global
+ * accesses of 8 and 16 bytes at any address. (A typedef's alignment is lost
+ * through a template parameter.) */
+typedef uint32_t m3_u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t m3_u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef float m3_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ void m3_stream_store(uint4 *p, uint4 v)
 {
