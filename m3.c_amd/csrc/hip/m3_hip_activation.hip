@@ -12,8 +12,9 @@
  *
  * Both are elementwise and bound by HBM traffic at large sizes: TANH moves
  * 8 bytes per F32 element, GATED_SILU 12 (F32) or 6 (16-bit operands).
- * The vector kernels take contiguous, 16-byte (F32) or 8-byte (16-bit)
- * aligned operands of one dtype: a lane handles four consecutive elements
+ * The vector kernels take contiguous operands of one dtype at any
+ * alignment, and for GATED_SILU also a gate and up whose rows are
+ * contiguous and evenly spaced (both halves of one projection): a lane handles four consecutive elements
  * per group, kUnroll groups in flight, loads and stores streaming (every
  * element is read and written once). The last count % 4 elements are done
  * by the first lanes of block 0. Every other layout (strided inputs, mixed
@@ -34,6 +35,7 @@
 #include "m3_hip_internal.h"
 #include "m3_libm.h"
 
+#include <algorithm>
 #include <cstring>
 
 namespace {
@@ -52,29 +54,6 @@ constexpr uint32_t kTanhUnroll = 2U;
  * process: GATED_SILU [16384, 3072] 94.5 against 100.5 us in F32 and 68.5
  * against 72.3 us in BF16; TANH x[2,1536,65536] 484 against 506 us. */
 constexpr uint32_t kBlocksPerCu = 1024U;
-
-/* Four consecutive elements of dtype D at group g of a contiguous array,
- * as F32. */
-template <uint32_t D>
-__device__ __forceinline__ void m3_load4(const uint8_t *base, uint32_t g,
-                                         float v[4])
-{
-    if (D == M3N_F32) {
-        uint4 w = m3_stream_load((const uint4 *)base + g);
-
-        v[0] = m3_bits_f32(w.x);
-        v[1] = m3_bits_f32(w.y);
-        v[2] = m3_bits_f32(w.z);
-        v[3] = m3_bits_f32(w.w);
-    } else {
-        uint2 w = m3_stream_load((const uint2 *)base + g);
-
-        v[0] = m3_bits_f32(m3_load_as_f32_bits(w.x & 0xffffU, D));
-        v[1] = m3_bits_f32(m3_load_as_f32_bits(w.x >> 16U, D));
-        v[2] = m3_bits_f32(m3_load_as_f32_bits(w.y & 0xffffU, D));
-        v[3] = m3_bits_f32(m3_load_as_f32_bits(w.y >> 16U, D));
-    }
-}
 
 /* Stores four F32 results (as bits) rounded to dtype D at group g. */
 template <uint32_t D>
@@ -133,27 +112,25 @@ __global__ __launch_bounds__(256) void m3_tanh_vec_kernel(m3_tanh_vec_args a)
 
     for (uint32_t first = blockIdx.x * kThreads * kTanhUnroll + threadIdx.x;
          first < a.groups; first += step) {
-        float x[kTanhUnroll][4];
+        float4 x[kTanhUnroll];
 
         /* unconditional loads (groups past the end re-read the last one)
          * so that all of them are in flight before the first use */
 #pragma unroll
         for (uint32_t u = 0U; u < kTanhUnroll; ++u) {
-            m3_load4<M3N_F32>(a.input, min(first + u * kThreads,
-                                            a.groups - 1U), x[u]);
+            x[u] = m3_stream_load((const float4 *)a.input +
+                                  min(first + u * kThreads, a.groups - 1U));
         }
 #pragma unroll
         for (uint32_t u = 0U; u < kTanhUnroll; ++u) {
             uint32_t g = first + u * kThreads;
 
             if (g < a.groups) {
-                uint32_t r[4];
-
-#pragma unroll
-                for (uint32_t k = 0U; k < 4U; ++k) {
-                    r[k] = m3_f32_bits(m3_tanhf_uniform(x[u][k]));
-                }
-                m3_store4<M3N_F32>(a.output, g, r);
+                m3_stream_store((float4 *)a.output + g,
+                                make_float4(m3_tanhf_uniform(x[u].x),
+                                            m3_tanhf_uniform(x[u].y),
+                                            m3_tanhf_uniform(x[u].z),
+                                            m3_tanhf_uniform(x[u].w)));
             }
         }
     }
@@ -223,8 +200,59 @@ struct m3_silu_vec_args {
     uint8_t *output;
     uint32_t groups;
     uint32_t tail;
+    /* rows of `width` (at least 4) elements whose starts are this many
+     * elements apart; unused when gate and up are contiguous */
+    m3_fast_div width;
+    uint64_t gate_pitch;
+    uint64_t up_pitch;
     m3_hip_gate list_gate;
 };
+
+/* Element `e` of an operand in rows of a.width elements, `pitch` apart. */
+__device__ __forceinline__ uint64_t m3_silu_row_offset(
+    const m3_silu_vec_args &a, uint64_t pitch, uint32_t e)
+{
+    const uint32_t row = m3_fast_div_q(a.width, e);
+
+    return row * pitch + (e - row * a.width.divisor);
+}
+
+/* Four consecutive elements of dtype D at group g, raw (zero-extended);
+ * ROWS: from rows, four elements that a row's end cuts one by one. Packed
+ * [3001, 2 x 3072] took 47 (BF16), 46 (F32) and 57 us (F16) in the general
+ * kernel, one element per lane, and takes 18.8, 20 and 32 in this one. */
+template <uint32_t D, bool ROWS>
+__device__ __forceinline__ uint4 m3_silu_load4(const m3_silu_vec_args &a,
+                                               const uint8_t *base,
+                                               uint64_t pitch, uint32_t g)
+{
+    constexpr uint32_t size = D == M3N_F32 ? 4U : 2U;
+    const uint32_t e = 4U * g;
+    uint64_t offset = e;
+
+    if (ROWS) {
+        offset = m3_silu_row_offset(a, pitch, e);
+        if (m3_fast_div_q(a.width, e) != m3_fast_div_q(a.width, e + 3U)) {
+            uint32_t x[4];
+
+#pragma unroll
+            for (uint32_t i = 0U; i < 4U; ++i) {
+                const uint8_t *p =
+                    base + m3_silu_row_offset(a, pitch, e + i) * size;
+
+                x[i] = size == 4U ? *(const uint32_t *)p
+                                  : (uint32_t) * (const uint16_t *)p;
+            }
+            return make_uint4(x[0], x[1], x[2], x[3]);
+        }
+    }
+    if (size == 4U) {
+        return m3_stream_load((const uint4 *)(base + offset * 4U));
+    }
+    const uint2 h = m3_stream_load((const uint2 *)(base + offset * 2U));
+
+    return make_uint4(h.x & 0xffffU, h.x >> 16U, h.y & 0xffffU, h.y >> 16U);
+}
 
 /* Four GATED_SILU elements with a gate of dtype D, as F32 bits; `table`
  * is the expf table in LDS. */
@@ -312,6 +340,7 @@ __device__ __forceinline__ uint32_t m3_silu_table_lookup(
                   : 0U;
 }
 
+template <bool ROWS>
 __global__ __launch_bounds__(256) void m3_gated_silu_bf16_kernel(
     m3_silu_vec_args a, const uint4 *source)
 {
@@ -331,8 +360,8 @@ __global__ __launch_bounds__(256) void m3_gated_silu_bf16_kernel(
     __syncthreads();
     for (uint32_t first = blockIdx.x * kThreads * kUnroll + threadIdx.x;
          first < a.groups; first += step) {
-        uint2 gate[kUnroll];
-        uint2 up[kUnroll];
+        uint4 gate[kUnroll];
+        uint4 up[kUnroll];
 
         /* unconditional loads (groups past the end re-read the last one)
          * so that all of them are in flight before the first use */
@@ -340,20 +369,21 @@ __global__ __launch_bounds__(256) void m3_gated_silu_bf16_kernel(
         for (uint32_t k = 0U; k < kUnroll; ++k) {
             const uint32_t index = min(first + k * kThreads, a.groups - 1U);
 
-            gate[k] = m3_stream_load((const uint2 *)a.gate + index);
-            up[k] = m3_stream_load((const uint2 *)a.up + index);
+            gate[k] = m3_silu_load4<M3N_BF16, ROWS>(a, a.gate, a.gate_pitch,
+                                                    index);
+            up[k] = m3_silu_load4<M3N_BF16, ROWS>(a, a.up, a.up_pitch, index);
         }
 #pragma unroll
         for (uint32_t k = 0U; k < kUnroll; ++k) {
             const uint32_t index = first + k * kThreads;
 
             if (index < a.groups) {
-                const uint32_t raw[4] = {gate[k].x & 0xffffU, gate[k].x >> 16U,
-                                         gate[k].y & 0xffffU, gate[k].y >> 16U};
+                const uint32_t raw[4] = {gate[k].x, gate[k].y, gate[k].z,
+                                         gate[k].w};
                 const float u[4] = {m3_bits_f32(up[k].x << 16U),
-                                    m3_bits_f32(up[k].x & 0xffff0000U),
                                     m3_bits_f32(up[k].y << 16U),
-                                    m3_bits_f32(up[k].y & 0xffff0000U)};
+                                    m3_bits_f32(up[k].z << 16U),
+                                    m3_bits_f32(up[k].w << 16U)};
                 uint32_t activation[4];
                 bool miss[4];
                 float p[4];
@@ -399,16 +429,20 @@ __global__ __launch_bounds__(256) void m3_gated_silu_bf16_kernel(
     }
     if (blockIdx.x == 0U && threadIdx.x < a.tail) {
         const uint64_t e = 4ULL * a.groups + threadIdx.x;
-        float g = m3_bits_f32(m3_load_element(a.gate + 2U * e, M3N_BF16));
-        float u = m3_bits_f32(m3_load_element(a.up + 2U * e, M3N_BF16));
+        const uint64_t ge =
+            ROWS ? m3_silu_row_offset(a, a.gate_pitch, (uint32_t)e) : e;
+        const uint64_t ue =
+            ROWS ? m3_silu_row_offset(a, a.up_pitch, (uint32_t)e) : e;
+        float g = m3_bits_f32(m3_load_element(a.gate + 2U * ge, M3N_BF16));
+        float u = m3_bits_f32(m3_load_element(a.up + 2U * ue, M3N_BF16));
 
         m3_store_element(a.output + 2U * e, M3N_BF16,
                          m3_gated_silu_bits(g, u, M3N_BF16));
     }
 }
 
-/* Gate, up and output all of dtype D, contiguous and aligned. */
-template <uint32_t D>
+/* Gate, up and output all of dtype D. */
+template <uint32_t D, bool ROWS>
 __global__ __launch_bounds__(256) void m3_gated_silu_vec_kernel(
     m3_silu_vec_args a)
 {
@@ -434,8 +468,19 @@ __global__ __launch_bounds__(256) void m3_gated_silu_vec_kernel(
         for (uint32_t k = 0U; k < kUnroll; ++k) {
             const uint32_t index = min(first + k * kThreads, a.groups - 1U);
 
-            m3_load4<D>(a.gate, index, g[k]);
-            m3_load4<D>(a.up, index, u[k]);
+            const uint4 gr =
+                m3_silu_load4<D, ROWS>(a, a.gate, a.gate_pitch, index);
+            const uint4 ur =
+                m3_silu_load4<D, ROWS>(a, a.up, a.up_pitch, index);
+
+            g[k][0] = m3_bits_f32(m3_load_as_f32_bits(gr.x, D));
+            g[k][1] = m3_bits_f32(m3_load_as_f32_bits(gr.y, D));
+            g[k][2] = m3_bits_f32(m3_load_as_f32_bits(gr.z, D));
+            g[k][3] = m3_bits_f32(m3_load_as_f32_bits(gr.w, D));
+            u[k][0] = m3_bits_f32(m3_load_as_f32_bits(ur.x, D));
+            u[k][1] = m3_bits_f32(m3_load_as_f32_bits(ur.y, D));
+            u[k][2] = m3_bits_f32(m3_load_as_f32_bits(ur.z, D));
+            u[k][3] = m3_bits_f32(m3_load_as_f32_bits(ur.w, D));
         }
 #pragma unroll
         for (uint32_t k = 0U; k < kUnroll; ++k) {
@@ -451,8 +496,12 @@ __global__ __launch_bounds__(256) void m3_gated_silu_vec_kernel(
     }
     if (blockIdx.x == 0U && threadIdx.x < a.tail) {
         const uint64_t e = 4ULL * a.groups + threadIdx.x;
-        float g = m3_bits_f32(m3_load_element(a.gate + size * e, D));
-        float u = m3_bits_f32(m3_load_element(a.up + size * e, D));
+        const uint64_t ge =
+            ROWS ? m3_silu_row_offset(a, a.gate_pitch, (uint32_t)e) : e;
+        const uint64_t ue =
+            ROWS ? m3_silu_row_offset(a, a.up_pitch, (uint32_t)e) : e;
+        float g = m3_bits_f32(m3_load_element(a.gate + size * ge, D));
+        float u = m3_bits_f32(m3_load_element(a.up + size * ue, D));
 
         m3_store_element(a.output + size * e, D, m3_gated_silu_bits(g, u, D));
     }
@@ -533,27 +582,37 @@ void m3_general_args(const m3_hip_view *output, const m3_hip_view *first,
     }
 }
 
-/* True when `view` is contiguous and its first element is aligned to
- * `alignment` bytes. */
-bool m3_vector_ready(const m3_hip_view *view, uintptr_t alignment)
+/* True when `view`, of the output's element count, is rows of *width
+ * contiguous elements, *pitch elements apart (a contiguous view: one row),
+ * after merging its axes. */
+bool m3_silu_rows(const m3_hip_view *view, uint64_t *width, uint64_t *pitch)
 {
-    uintptr_t address = (uintptr_t)view->base + view->byte_offset;
+    const uint64_t size = m3_dtype_bytes(view->dtype);
+    const m3_hip_view *operands[1] = {view};
+    m3_index_plan plan;
 
-    return m3_view_is_contiguous(view) && address % alignment == 0U;
+    m3_plan_index_space(view, operands, 1U, &plan);
+    if (plan.rank > 2U || plan.strides[0][plan.rank - 1U] != (int64_t)size) {
+        return false;
+    }
+    *width = plan.shape[plan.rank - 1U];
+    *pitch = plan.rank == 1U ? *width
+                             : (uint64_t)plan.strides[0][0] / size;
+    return plan.rank == 1U || (uint64_t)plan.strides[0][0] % size == 0U;
 }
 
-template <uint32_t D>
+template <uint32_t D, bool ROWS>
 void m3_launch_silu_vec(m3_hip_device *device, const m3_silu_vec_args &args,
                         uint32_t blocks, hipEvent_t start, hipEvent_t stop)
 {
     if (D == M3N_BF16) {
-        hipExtLaunchKernelGGL(m3_gated_silu_bf16_kernel, dim3(blocks),
+        hipExtLaunchKernelGGL((m3_gated_silu_bf16_kernel<ROWS>), dim3(blocks),
                               dim3(kThreads), 0, device->stream, start, stop,
                               0U, args,
                               (const uint4 *)device->silu_bf16_table);
         return;
     }
-    hipExtLaunchKernelGGL((m3_gated_silu_vec_kernel<D>), dim3(blocks),
+    hipExtLaunchKernelGGL((m3_gated_silu_vec_kernel<D, ROWS>), dim3(blocks),
                           dim3(kThreads), 0, device->stream, start, stop, 0U,
                           args);
 }
@@ -605,8 +664,7 @@ extern "C" int m3_hip_launch_tanh(m3_hip_device *device,
     }
     /* below 2^32 elements the vector kernel's 32-bit group indices, plus
      * one grid stride (at most 2^28), stay below 2^32 */
-    if (m3_vector_ready(input, 16U) && m3_vector_ready(output, 16U) &&
-        count < (1ULL << 32U)) {
+    if (m3_view_is_contiguous(input) && count < (1ULL << 32U)) {
         m3_tanh_vec_args args;
 
         args.list_gate = device->gate;
@@ -663,28 +721,53 @@ extern "C" int m3_hip_launch_gated_silu(m3_hip_device *device,
         return M3_HIP_OK;
     }
     const uint32_t dtype = output->dtype;
-    const uintptr_t alignment = dtype == M3_HIP_F32 ? 16U : 8U;
+    uint64_t gate_width = 0U;
+    uint64_t up_width = 0U;
+    uint64_t gate_pitch = 0U;
+    uint64_t up_pitch = 0U;
+    const bool contiguous =
+        m3_view_is_contiguous(gate) && m3_view_is_contiguous(up);
+    /* rows: each operand contiguous or in rows, the same ones; four
+     * consecutive elements then lie in at most two rows */
+    const bool in_rows =
+        !contiguous && m3_silu_rows(gate, &gate_width, &gate_pitch) &&
+        m3_silu_rows(up, &up_width, &up_pitch) &&
+        (gate_width == up_width || gate_width == count ||
+         up_width == count) &&
+        std::min(gate_width, up_width) >= 4U;
 
     if (gate->dtype == dtype && up->dtype == dtype &&
-        m3_vector_ready(gate, alignment) && m3_vector_ready(up, alignment) &&
-        m3_vector_ready(output, alignment) &&
+        (contiguous || in_rows) &&
         count < (1ULL << 32U)) { /* 32-bit group indices, as for TANH */
         m3_silu_vec_args args;
 
+        std::memset(&args, 0, sizeof(args));
         args.list_gate = device->gate;
         args.gate = (const uint8_t *)gate->base + gate->byte_offset;
         args.up = (const uint8_t *)up->base + up->byte_offset;
         args.output = (uint8_t *)output->base + output->byte_offset;
         args.groups = (uint32_t)(count / 4U);
         args.tail = (uint32_t)(count % 4U);
+        if (in_rows) {
+            const uint64_t width = std::min(gate_width, up_width);
+
+            args.width = m3_fast_div_make((uint32_t)width);
+            args.gate_pitch = gate_width == width ? gate_pitch : width;
+            args.up_pitch = up_width == width ? up_pitch : width;
+        }
         uint32_t blocks = m3_grid_blocks(
             device, args.groups == 0U ? 1U : args.groups,
             kThreads * kUnroll, kBlocksPerCu);
         void (*launch)(m3_hip_device *, const m3_silu_vec_args &, uint32_t,
                        hipEvent_t, hipEvent_t) =
-            dtype == M3_HIP_F32   ? &m3_launch_silu_vec<M3N_F32>
-            : dtype == M3_HIP_F16 ? &m3_launch_silu_vec<M3N_F16>
-                                  : &m3_launch_silu_vec<M3N_BF16>;
+            dtype == M3_HIP_F32
+                ? in_rows ? &m3_launch_silu_vec<M3N_F32, true>
+                          : &m3_launch_silu_vec<M3N_F32, false>
+            : dtype == M3_HIP_F16
+                ? in_rows ? &m3_launch_silu_vec<M3N_F16, true>
+                          : &m3_launch_silu_vec<M3N_F16, false>
+            : in_rows ? &m3_launch_silu_vec<M3N_BF16, true>
+                      : &m3_launch_silu_vec<M3N_BF16, false>;
         const char *name = dtype == M3_HIP_F32   ? "m3_gated_silu"
                            : dtype == M3_HIP_F16 ? "m3_gated_silu_f16"
                                                  : "m3_gated_silu_bf16";

@@ -279,20 +279,6 @@ __device__ __forceinline__ uint4 m3_load4_any(const uint8_t *p)
                       h[1] >> 16U);
 }
 
-__device__ __forceinline__ void m3_store4_any(uint8_t *p, uint4 v)
-{
-    const m3_u32x4_any w = {v.x, v.y, v.z, v.w};
-
-    __builtin_nontemporal_store(w, (m3_u32x4_any *)p);
-}
-
-__device__ __forceinline__ void m3_store4_any(uint8_t *p, uint2 v)
-{
-    const m3_u32x2_any w = {v.x, v.y};
-
-    __builtin_nontemporal_store(w, (m3_u32x2_any *)p);
-}
-
 /* A tile of 64 (u) by 128 (n) elements through LDS: each lane reads four
  * elements along u at four consecutive n, transposes the 4 x 4 block in
  * registers, converts it and writes it as four vectors along n; the tile is
@@ -413,7 +399,7 @@ __global__ __launch_bounds__(256) void m3_transpose_kernel(m3_transpose_args a)
                 out + ((tile_u + r) * a.out_u_stride + n) * out_size;
 
             if (n + 4U <= a.n) {
-                m3_store4_any(p, w);
+                m3_stream_store((slot_type *)p, w);
                 continue;
             }
             const uint4 x = out_io::unpack(w);

@@ -206,7 +206,9 @@ int m3_hip_launch(m3_hip_device *device, const char *name, Launch launch,
 /* Streaming stores for kernel outputs: nontemporal vector stores that
  * write through without keeping the lines in the caches. Every output of
  * this library is written once and not read back by the same kernel; on
- * gfx950 these stores sustain a higher copy rate than ordinary ones. */
+ * gfx950 these stores sustain a higher copy rate than ordinary ones. The
+ * pointers, here and in the streaming loads, need an element's alignment
+ * only. */
 typedef uint32_t m3_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t m3_u32x2 __attribute__((ext_vector_type(2)));
 typedef float m3_f32x4 __attribute__((ext_vector_type(4)));
@@ -219,44 +221,44 @@ typedef float m3_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ void m3_stream_store(uint4 *p, uint4 v)
 {
-    m3_u32x4 w = {v.x, v.y, v.z, v.w};
+    m3_u32x4_any w = {v.x, v.y, v.z, v.w};
 
-    __builtin_nontemporal_store(w, (m3_u32x4 *)p);
+    __builtin_nontemporal_store(w, (m3_u32x4_any *)p);
 }
 
 __device__ __forceinline__ void m3_stream_store(uint2 *p, uint2 v)
 {
-    m3_u32x2 w = {v.x, v.y};
+    m3_u32x2_any w = {v.x, v.y};
 
-    __builtin_nontemporal_store(w, (m3_u32x2 *)p);
+    __builtin_nontemporal_store(w, (m3_u32x2_any *)p);
 }
 
 __device__ __forceinline__ void m3_stream_store(float4 *p, float4 v)
 {
-    m3_f32x4 w = {v.x, v.y, v.z, v.w};
+    m3_f32x4_any w = {v.x, v.y, v.z, v.w};
 
-    __builtin_nontemporal_store(w, (m3_f32x4 *)p);
+    __builtin_nontemporal_store(w, (m3_f32x4_any *)p);
 }
 
 /* Streaming loads for inputs that one kernel reads exactly once (not for
  * broadcast operands, which stay cached across the grid). */
 __device__ __forceinline__ uint4 m3_stream_load(const uint4 *p)
 {
-    m3_u32x4 w = __builtin_nontemporal_load((const m3_u32x4 *)p);
+    m3_u32x4 w = __builtin_nontemporal_load((const m3_u32x4_any *)p);
 
     return make_uint4(w.x, w.y, w.z, w.w);
 }
 
 __device__ __forceinline__ uint2 m3_stream_load(const uint2 *p)
 {
-    m3_u32x2 w = __builtin_nontemporal_load((const m3_u32x2 *)p);
+    m3_u32x2 w = __builtin_nontemporal_load((const m3_u32x2_any *)p);
 
     return make_uint2(w.x, w.y);
 }
 
 __device__ __forceinline__ float4 m3_stream_load(const float4 *p)
 {
-    m3_f32x4 w = __builtin_nontemporal_load((const m3_f32x4 *)p);
+    m3_f32x4 w = __builtin_nontemporal_load((const m3_f32x4_any *)p);
 
     return make_float4(w.x, w.y, w.z, w.w);
 }

@@ -11,12 +11,12 @@
  * division is the IEEE F32 quotient; this file is compiled with
  * -ffp-contract=off so no statement fuses. inv depends only on the channel
  * and is formed once per lane and loop iteration when the lane's groups lie
- * in one channel, else once per group of four outputs.
+ * in one channel, else once per group of four outputs (twice in a wave
+ * where a channel ends inside a group).
  *
- * The vector kernel handles contiguous, 16-byte aligned x and output with
- * L a multiple of 4: a lane takes four consecutive elements of one
- * channel, four groups in flight. Other layouts run per element over
- * stride tables.
+ * The vector kernel handles contiguous x and output of any length L of at
+ * least 4, at any alignment: a lane takes four consecutive elements, four
+ * groups in flight. Other layouts run per element over stride tables.
  */
 #include "m3_hip_internal.h"
 #include "m3_libm.h"
@@ -50,15 +50,17 @@ __device__ __forceinline__ float m3_snake(float x, float a, float inverse)
     return m3_snake_finish(x, m3_sinf(a * x), inverse);
 }
 
-/* Four outputs of one channel. When no lane of the wave has an angle with
+/* Four outputs, given each one's alpha and inverse. When no lane of the wave has an angle with
  * |a*x| >= 120 or a NaN angle (the common case by far), all four take the
  * branch-free sinf path, so the large-argument reduction costs one uniform
  * test per group instead of a divergent branch per element. That path
  * drops the sign of sinf: only its square is used, and the magnitude is
  * that of sinf for every |angle| < 120. */
-__device__ __forceinline__ float4 m3_snake4(float4 x, float a, float inverse)
+__device__ __forceinline__ float4 m3_snake4(float4 x, float4 a,
+                                            float4 inverse)
 {
-    const float4 angle = make_float4(a * x.x, a * x.y, a * x.z, a * x.w);
+    const float4 angle =
+        make_float4(a.x * x.x, a.y * x.y, a.z * x.z, a.w * x.w);
     /* one compare per element into a lane mask, the masks OR-ed as
      * scalars */
     const uint64_t large = __ballot(!(fabsf(angle.x) < 120.0F)) |
@@ -76,10 +78,10 @@ __device__ __forceinline__ float4 m3_snake4(float4 x, float a, float inverse)
                            m3_sinf_medium_magnitude(angle.z),
                            m3_sinf_medium_magnitude(angle.w));
     }
-    return make_float4(m3_snake_finish(x.x, sine.x, inverse),
-                       m3_snake_finish(x.y, sine.y, inverse),
-                       m3_snake_finish(x.z, sine.z, inverse),
-                       m3_snake_finish(x.w, sine.w, inverse));
+    return make_float4(m3_snake_finish(x.x, sine.x, inverse.x),
+                       m3_snake_finish(x.y, sine.y, inverse.y),
+                       m3_snake_finish(x.z, sine.z, inverse.z),
+                       m3_snake_finish(x.w, sine.w, inverse.w));
 }
 
 __device__ __forceinline__ float m3_snake_inverse(float a)
@@ -90,16 +92,37 @@ __device__ __forceinline__ float m3_snake_inverse(float a)
 }
 
 struct m3_snake_vec_args {
-    const float4 *input;
+    const float *input;
     const uint8_t *alpha; /* alpha element of channel 0 */
     int64_t alpha_stride; /* bytes between channels */
-    float4 *output;
+    float *output;
     uint32_t groups;      /* elements / 4 */
-    m3_fast_div length_in_groups; /* L / 4 */
+    uint32_t tail;        /* elements % 4 */
+    m3_fast_div length;   /* L >= 4 */
     m3_fast_div channels;
     m3_hip_gate list_gate;
 };
 
+__device__ __forceinline__ float4 m3_splat4(float v)
+{
+    return make_float4(v, v, v, v);
+}
+
+/* The alpha of row b*C + c. */
+__device__ __forceinline__ float m3_snake_alpha(const m3_snake_vec_args &a,
+                                                uint32_t row)
+{
+    const uint32_t channel =
+        row - m3_fast_div_q(a.channels, row) * a.channels.divisor;
+
+    return *(const float *)(a.alpha + (int64_t)channel * a.alpha_stride);
+}
+
+/* Groups of four consecutive elements, kUnroll per lane. L need not be a
+ * multiple of 4: a group that a row's end cuts takes the next row's alpha
+ * for its last elements, in the waves that hold one. Bound by HBM
+ * (x[2,1536,65536] 264 us, 6.1 TB/s; x[2,192,60001] 30.5 us, 6.0 TB/s,
+ * where one element per lane with 64-bit divisions took about 75). */
 __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
     m3_snake_vec_args a)
 {
@@ -111,60 +134,82 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
     for (uint32_t first = blockIdx.x * kThreads * kUnroll + threadIdx.x;
          first < a.groups; first += step) {
         const uint32_t last = first + (kUnroll - 1U) * kThreads;
-        const uint32_t row = m3_fast_div_q(a.length_in_groups, first);
+        const uint32_t row = m3_fast_div_q(a.length, 4U * first);
         float4 x[kUnroll];
 
-        /* The row b*C + c of group g is nondecreasing in g, so when the
-         * first and last group of a lane share a row, all of its groups
+        /* The row b*C + c of an element is nondecreasing in its index, so
+         * when a lane's first and last element share a row, all of them
          * do: one channel, one alpha and one division for the lane. */
         if (__all(last < a.groups &&
-                  m3_fast_div_q(a.length_in_groups, last) == row)) {
-            const uint32_t channel =
-                row - m3_fast_div_q(a.channels, row) * a.channels.divisor;
-            const float alpha = *(const float *)(
-                a.alpha + (int64_t)channel * a.alpha_stride);
+                  m3_fast_div_q(a.length, 4U * last + 3U) == row)) {
+            const float alpha = m3_snake_alpha(a, row);
 
 #pragma unroll
             for (uint32_t u = 0U; u < kUnroll; ++u) {
-                x[u] = m3_stream_load(&a.input[first + u * kThreads]);
+                x[u] = m3_stream_load((const float4 *)a.input + first +
+                                      u * kThreads);
             }
             const float inverse = m3_snake_inverse(alpha);
 
 #pragma unroll
             for (uint32_t u = 0U; u < kUnroll; ++u) {
-                m3_stream_store(&a.output[first + u * kThreads],
-                                m3_snake4(x[u], alpha, inverse));
+                m3_stream_store((float4 *)a.output + first + u * kThreads,
+                                m3_snake4(x[u], m3_splat4(alpha),
+                                          m3_splat4(inverse)));
             }
             continue;
         }
 
+        uint32_t rows[kUnroll];
         float alpha[kUnroll];
 
 #pragma unroll
         for (uint32_t u = 0U; u < kUnroll; ++u) {
-            uint32_t g = first + u * kThreads;
+            const uint32_t g = min(first + u * kThreads, a.groups - 1U);
 
-            if (g < a.groups) {
-                uint32_t q = m3_fast_div_q(a.length_in_groups, g);
-                uint32_t channel =
-                    q - m3_fast_div_q(a.channels, q) * a.channels.divisor;
-
-                x[u] = m3_stream_load(&a.input[g]);
-                alpha[u] = *(const float *)(a.alpha +
-                                            (int64_t)channel * a.alpha_stride);
-            }
+            rows[u] = m3_fast_div_q(a.length, 4U * g);
+            x[u] = m3_stream_load((const float4 *)a.input + g);
+            alpha[u] = m3_snake_alpha(a, rows[u]);
         }
 #pragma unroll
         for (uint32_t u = 0U; u < kUnroll; ++u) {
-            uint32_t g = first + u * kThreads;
+            const uint32_t g = min(first + u * kThreads, a.groups - 1U);
+            /* elements of the group before the row's end */
+            const uint32_t here =
+                a.length.divisor - (4U * g - rows[u] * a.length.divisor);
+            const float inverse = m3_snake_inverse(alpha[u]);
+            float4 alpha4 = m3_splat4(alpha[u]);
+            float4 inverse4 = m3_splat4(inverse);
 
-            if (g < a.groups) {
-                float inverse = m3_snake_inverse(alpha[u]);
+            if (M3_ANY_LANE(here < 4U)) {
+                /* every row has at least 4 elements: at most one end; a
+                 * group it does not cut takes its own row again */
+                const float other =
+                    m3_snake_alpha(a, rows[u] + (here < 4U ? 1U : 0U));
+                const float other_inverse = m3_snake_inverse(other);
 
-                m3_stream_store(&a.output[g],
-                                m3_snake4(x[u], alpha[u], inverse));
+                alpha4.y = here > 1U ? alpha4.y : other;
+                alpha4.z = here > 2U ? alpha4.z : other;
+                alpha4.w = here > 3U ? alpha4.w : other;
+                inverse4.y = here > 1U ? inverse4.y : other_inverse;
+                inverse4.z = here > 2U ? inverse4.z : other_inverse;
+                inverse4.w = here > 3U ? inverse4.w : other_inverse;
+            }
+            const float4 y = m3_snake4(x[u], alpha4, inverse4);
+
+            if (first + u * kThreads < a.groups) {
+                m3_stream_store((float4 *)a.output + g, y);
             }
         }
+    }
+    if (blockIdx.x == 0U && threadIdx.x < a.tail) {
+        /* the last elements % 4, in the last row */
+        const uint64_t e = 4ULL * a.groups + threadIdx.x;
+        const float alpha =
+            m3_snake_alpha(a, m3_fast_div_q(a.length, (uint32_t)e));
+
+        a.output[e] =
+            m3_snake(a.input[e], alpha, m3_snake_inverse(alpha));
     }
 }
 
@@ -237,19 +282,21 @@ extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
                                ? (int64_t)alpha->byte_strides[1]
                                : 0;
 
-    if (m3_view_is_contiguous(input) && length % 4U == 0U &&
-        output->element_count < (1ULL << 32U) &&
-        ((uintptr_t)in & 15U) == 0U && ((uintptr_t)out & 15U) == 0U) {
+    /* 32-bit element indices: below 2^32 with the lanes past the end (they
+     * read the last group) */
+    if (m3_view_is_contiguous(input) && length >= 4U &&
+        output->element_count < (1ULL << 32U)) {
         m3_snake_vec_args args;
 
         std::memset(&args, 0, sizeof(args));
         args.list_gate = device->gate;
-        args.input = (const float4 *)in;
+        args.input = (const float *)in;
         args.alpha = al;
         args.alpha_stride = alpha_stride;
-        args.output = (float4 *)out;
+        args.output = (float *)out;
         args.groups = (uint32_t)(output->element_count / 4U);
-        args.length_in_groups = m3_fast_div_make((uint32_t)(length / 4U));
+        args.tail = (uint32_t)(output->element_count % 4U);
+        args.length = m3_fast_div_make((uint32_t)length);
         args.channels = m3_fast_div_make((uint32_t)input->shape[1]);
         uint32_t blocks = m3_grid_blocks(device, args.groups,
                                          kThreads * kUnroll, kBlocksPerCu);
