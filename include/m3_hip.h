@@ -47,6 +47,9 @@
  *                                   (src/m3_backend_metal.m:210-216)
  *   m3_hip_prepare_program       no counterpart: compiles a program's
  *                                   kernel ahead of its first launch
+ *   m3_hip_launch_chain          no counterpart: consecutive commands,
+ *                                   each over the output of the one before,
+ *                                   in one launch
  *   m3_hip_launch_program        no counterpart: runs a run of ADD/SUB/
  *                                   MUL/DIV commands (per-element semantics
  *                                   of src/m3_op_execute_basic.c:61-77) that
@@ -159,6 +162,36 @@ int m3_hip_launch_binary(m3_hip_device *device, uint32_t op,
                          const m3_hip_view *left, const m3_hip_view *right,
                          const m3_hip_view *output, char *message,
                          size_t capacity);
+/* A run of operations in which each takes the output of the one before as
+ * an operand, as one launch that stores every output and reads none back:
+ * binary operations and casts between float dtypes over one shape, or
+ * SNAKE1D then TANH. The results are those of the operations launched one
+ * by one. *taken is 0, with nothing launched, when no kernel takes the run
+ * (an operand layout it does not know, an output that overlaps another
+ * output or what an operation reads); the caller then launches them one by
+ * one. */
+#define M3_HIP_MAX_CHAIN 3U
+
+typedef enum {
+    M3_HIP_CHAIN_BINARY = 0,
+    M3_HIP_CHAIN_CAST = 1,
+    M3_HIP_CHAIN_SNAKE1D = 2, /* left: input, right: alpha */
+    M3_HIP_CHAIN_TANH = 3
+} m3_hip_chain_kind;
+
+typedef struct {
+    uint32_t kind;
+    uint32_t op;       /* m3_hip_binary_op of a binary operation */
+    uint32_t link;     /* which operand is the output before: 0 left (or the
+                          only input), 1 right; ignored in the first */
+    m3_hip_view left;  /* or the only input */
+    m3_hip_view right; /* of a binary operation, or alpha */
+    m3_hip_view output;
+} m3_hip_chain_command;
+
+int m3_hip_launch_chain(m3_hip_device *device,
+                        const m3_hip_chain_command *commands, uint32_t count,
+                        int *taken, char *message, size_t capacity);
 /* Element conversion between any two of F32/F16/BF16/I32 (same dtype is a
  * copy). Float to I32 truncates; callers scan the input first. */
 int m3_hip_launch_cast(m3_hip_device *device, const m3_hip_view *input,

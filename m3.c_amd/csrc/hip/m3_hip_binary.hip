@@ -19,16 +19,23 @@
  *        ROW      offset = (f / I) mod P     (broadcast over inner axes,
  *                                             I a multiple of 4)
  *        SCALAR   offset = 0
+ *        TRAIL_CUT, ROW_CUT                  (the same two with P or I at
+ *                                             least 4 but no multiple of
+ *                                             it: a group of 4 may wrap or
+ *                                             take two elements)
  *        PERIODIC offset = (f / I) mod P     (any I, per-element loads)
- *   3. when both inputs classify and the output is contiguous and aligned,
- *      the vector kernel runs: each lane handles groups of 4 consecutive
- *      outputs with 16-byte (F32) or 8-byte (F16/BF16) loads and stores,
- *      two groups in flight per lane, grid-stride over the tensor; with
- *      F32 operands and a tensor whose lanes are all resident at once, its
- *      held form instead (all loads, then the stores after a timed wait);
- *      divisions by I and P use precomputed multiply-shift divisors;
+ *   3. when both inputs classify, the vector kernel runs: each lane handles
+ *      groups of 4 consecutive outputs with 16-byte (F32) or 8-byte
+ *      (F16/BF16) loads and stores at any alignment, two groups in flight
+ *      per lane, grid-stride over the tensor; with F32 operands and a
+ *      tensor whose lanes are all resident at once, its held form instead
+ *      (all loads, then the stores after a timed wait); divisions by I and
+ *      P use precomputed multiply-shift divisors;
  *   4. anything else runs the general kernel: per-element offsets from the
  *      coalesced stride table.
+ * A run of such operations and float casts in which each takes the one
+ * before as an operand is one launch of the chain kernel (m3_chain_kernel):
+ * every result is stored, none is read back.
  * All operands are read as F32 bit patterns, so NaN payloads survive
  * loads; m3_binary_f32_bits applies the operation and the NaN rule.
  */
@@ -43,7 +50,9 @@ enum m3_bin_mode : uint32_t {
     M3_BIN_TRAIL = 1,
     M3_BIN_ROW = 2,
     M3_BIN_SCALAR = 3,
-    M3_BIN_PERIODIC = 4
+    M3_BIN_PERIODIC = 4,
+    M3_BIN_TRAIL_CUT = 5,
+    M3_BIN_ROW_CUT = 6
 };
 
 struct m3_bin_operand {
@@ -65,6 +74,8 @@ struct m3_bin_vec_args {
 };
 
 constexpr uint32_t kThreads = 256U;
+/* a kernel's element type: one dtype throughout, or each operand's own */
+constexpr uint32_t kAnyDtype = 0xffffffffU;
 constexpr uint32_t kUnroll = 2U; /* groups in flight per lane (measured best) */
 
 __device__ __forceinline__ uint32_t m3_load_raw(const uint8_t *p,
@@ -74,7 +85,6 @@ __device__ __forceinline__ uint32_t m3_load_raw(const uint8_t *p,
                             : (uint32_t) * (const uint16_t *)p;
 }
 
-template <bool F32ONLY>
 __device__ __forceinline__ uint32_t m3_operand_index(const m3_bin_operand &o,
                                                      uint32_t f)
 {
@@ -82,6 +92,7 @@ __device__ __forceinline__ uint32_t m3_operand_index(const m3_bin_operand &o,
     case M3_BIN_FULL:
         return f;
     case M3_BIN_TRAIL:
+    case M3_BIN_TRAIL_CUT:
         return f - m3_fast_div_q(o.period, f) * o.period.divisor;
     case M3_BIN_SCALAR:
         return 0U;
@@ -93,25 +104,32 @@ __device__ __forceinline__ uint32_t m3_operand_index(const m3_bin_operand &o,
     }
 }
 
-template <bool F32ONLY>
+/* F32 bits of the operand's element at `index`. */
+template <uint32_t DT>
+__device__ __forceinline__ uint32_t m3_operand_at(const m3_bin_operand &o,
+                                                  uint32_t index)
+{
+    uint32_t dtype = DT == kAnyDtype ? o.dtype : DT;
+    uint32_t esize = dtype == M3N_F32 ? 4U : 2U;
+
+    return m3_load_as_f32_bits(
+        m3_load_raw(o.base + (uint64_t)index * esize, dtype), dtype);
+}
+
+template <uint32_t DT>
 __device__ __forceinline__ uint32_t m3_operand_element(const m3_bin_operand &o,
                                                        uint32_t f)
 {
-    uint32_t dtype = F32ONLY ? (uint32_t)M3N_F32 : o.dtype;
-    uint32_t esize = dtype == M3N_F32 ? 4U : 2U;
-    uint32_t raw = m3_load_raw(o.base + (uint64_t)m3_operand_index<F32ONLY>(
-                                            o, f) * esize,
-                               dtype);
-
-    return m3_load_as_f32_bits(raw, dtype);
+    return m3_operand_at<DT>(o, m3_operand_index(o, f));
 }
 
-/* F32 bits of operand elements f..f+3 (f a multiple of 4). */
-template <bool F32ONLY>
+/* F32 bits of operand elements f..f+3 (f a multiple of 4). WHOLE: the
+ * operand's mode is none of TRAIL_CUT, ROW_CUT and PERIODIC. */
+template <uint32_t DT, bool WHOLE = false>
 __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
                                                   uint32_t f)
 {
-    uint32_t dtype = F32ONLY ? (uint32_t)M3N_F32 : o.dtype;
+    uint32_t dtype = DT == kAnyDtype ? o.dtype : DT;
 
     if (o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL) {
         uint32_t index = o.mode == M3_BIN_FULL
@@ -122,53 +140,92 @@ __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
         /* a full operand is read once per launch: streamed; a trailing
          * broadcast operand is reread by every row: cached */
         if (dtype == M3N_F32) {
-            const uint4 *p = (const uint4 *)(o.base + (uint64_t)index * 4U);
+            const uint8_t *p = o.base + (uint64_t)index * 4U;
 
-            return o.mode == M3_BIN_FULL ? m3_stream_load(p) : *p;
+            if (o.mode == M3_BIN_FULL) {
+                return m3_stream_load((const uint4 *)p);
+            }
+            const m3_u32x4_any w = *(const m3_u32x4_any *)p;
+
+            return make_uint4(w[0], w[1], w[2], w[3]);
         }
-        const uint2 *h = (const uint2 *)(o.base + (uint64_t)index * 2U);
-        const uint2 half = o.mode == M3_BIN_FULL ? m3_stream_load(h) : *h;
+        const uint8_t *p = o.base + (uint64_t)index * 2U;
+        uint2 half;
 
-        return make_uint4(m3_load_as_f32_bits(half.x & 0xffffU, dtype),
-                          m3_load_as_f32_bits(half.x >> 16U, dtype),
-                          m3_load_as_f32_bits(half.y & 0xffffU, dtype),
-                          m3_load_as_f32_bits(half.y >> 16U, dtype));
+        if (o.mode == M3_BIN_FULL) {
+            half = m3_stream_load((const uint2 *)p);
+        } else {
+            const m3_u32x2_any h = *(const m3_u32x2_any *)p;
+
+            half = make_uint2(h[0], h[1]);
+        }
+        return m3_widen4_bits(half, dtype);
     }
-    if (o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR) {
-        uint32_t v = m3_operand_element<F32ONLY>(o, f);
+    if (WHOLE || o.mode == M3_BIN_SCALAR) {
+        uint32_t v = m3_operand_element<DT>(o, f);
 
         return make_uint4(v, v, v, v);
     }
-    return make_uint4(m3_operand_element<F32ONLY>(o, f),
-                      m3_operand_element<F32ONLY>(o, f + 1U),
-                      m3_operand_element<F32ONLY>(o, f + 2U),
-                      m3_operand_element<F32ONLY>(o, f + 3U));
+    if (o.mode == M3_BIN_ROW || o.mode == M3_BIN_ROW_CUT) {
+        /* one element, or two for a group in which a run of I ends: both
+         * from cache (the second is the first again in the others). A wave
+         * whose groups lie in one run, as most do when runs are long, finds
+         * and converts its element once, in scalar registers. */
+        const uint32_t q = m3_fast_div_q(o.inner, f);
+        const uint32_t here = (q + 1U) * o.inner.divisor - f;
+        const uint32_t run = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
+
+        if (__all(q == run && here >= 4U)) {
+            const uint32_t v = m3_operand_at<DT>(
+                o, run - m3_fast_div_q(o.period, run) * o.period.divisor);
+
+            return make_uint4(v, v, v, v);
+        }
+        const uint32_t next = here < 4U ? q + 1U : q;
+        const uint32_t v = m3_operand_at<DT>(
+            o, q - m3_fast_div_q(o.period, q) * o.period.divisor);
+        const uint32_t w = m3_operand_at<DT>(
+            o, next - m3_fast_div_q(o.period, next) * o.period.divisor);
+
+        return make_uint4(v, here > 1U ? v : w, here > 2U ? v : w,
+                          here > 3U ? v : w);
+    }
+    if (o.mode == M3_BIN_TRAIL_CUT) {
+        /* consecutive elements that may wrap to the period's start */
+        const uint32_t p = o.period.divisor;
+        const uint32_t i = f - m3_fast_div_q(o.period, f) * p;
+
+        return make_uint4(
+            m3_operand_at<DT>(o, i),
+            m3_operand_at<DT>(o, i + 1U < p ? i + 1U : i + 1U - p),
+            m3_operand_at<DT>(o, i + 2U < p ? i + 2U : i + 2U - p),
+            m3_operand_at<DT>(o, i + 3U < p ? i + 3U : i + 3U - p));
+    }
+    return make_uint4(m3_operand_element<DT>(o, f),
+                      m3_operand_element<DT>(o, f + 1U),
+                      m3_operand_element<DT>(o, f + 2U),
+                      m3_operand_element<DT>(o, f + 3U));
 }
 
-template <bool F32ONLY>
+template <uint32_t DT>
 __device__ __forceinline__ void m3_store4(uint8_t *out, uint32_t dtype,
                                           uint32_t f, uint4 v)
 {
-    if (F32ONLY || dtype == M3N_F32) {
+    if (DT == M3N_F32 || dtype == M3N_F32) {
         m3_stream_store((uint4 *)(out + (uint64_t)f * 4U), v);
         return;
     }
-    uint2 packed;
-
-    packed.x = m3_store_from_f32_bits(v.x, dtype) |
-               (m3_store_from_f32_bits(v.y, dtype) << 16U);
-    packed.y = m3_store_from_f32_bits(v.z, dtype) |
-               (m3_store_from_f32_bits(v.w, dtype) << 16U);
-    m3_stream_store((uint2 *)(out + (uint64_t)f * 2U), packed);
+    m3_stream_store((uint2 *)(out + (uint64_t)f * 2U),
+                    m3_narrow4_bits(v, dtype));
 }
 
-template <int OP, bool F32ONLY, int UNROLL = (int)kUnroll>
+template <int OP, uint32_t DT, int UNROLL = (int)kUnroll>
 __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
 {
     if (m3_gate_closed(a.list_gate)) {
         return; /* a check earlier in the list failed */
     }
-    const uint32_t out_dtype = F32ONLY ? (uint32_t)M3N_F32 : a.out_dtype;
+    const uint32_t out_dtype = DT == kAnyDtype ? a.out_dtype : DT;
     const uint32_t step = gridDim.x * kThreads * UNROLL;
 
     for (uint32_t first = blockIdx.x * kThreads * UNROLL + threadIdx.x;
@@ -181,8 +238,8 @@ __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
             uint32_t g = first + u * kThreads;
 
             if (g < a.groups) {
-                left[u] = m3_operand_load4<F32ONLY>(a.left, g * 4U);
-                right[u] = m3_operand_load4<F32ONLY>(a.right, g * 4U);
+                left[u] = m3_operand_load4<DT>(a.left, g * 4U);
+                right[u] = m3_operand_load4<DT>(a.right, g * 4U);
             }
         }
 #pragma unroll
@@ -196,7 +253,7 @@ __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
                 r.y = m3_binary_f32_bits(OP, left[u].y, right[u].y);
                 r.z = m3_binary_f32_bits(OP, left[u].z, right[u].z);
                 r.w = m3_binary_f32_bits(OP, left[u].w, right[u].w);
-                m3_store4<F32ONLY>(a.out, out_dtype, g * 4U, r);
+                m3_store4<DT>(a.out, out_dtype, g * 4U, r);
             }
         }
     }
@@ -204,8 +261,8 @@ __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
     if (blockIdx.x == 0U && threadIdx.x < a.count - a.groups * 4U) {
         uint32_t f = a.groups * 4U + threadIdx.x;
         uint32_t r = m3_binary_f32_bits(
-            OP, m3_operand_element<F32ONLY>(a.left, f),
-            m3_operand_element<F32ONLY>(a.right, f));
+            OP, m3_operand_element<DT>(a.left, f),
+            m3_operand_element<DT>(a.right, f));
         uint32_t raw = m3_store_from_f32_bits(r, out_dtype);
 
         if (out_dtype == M3N_F32) {
@@ -251,8 +308,8 @@ __global__ __launch_bounds__(256) void m3_binary_held_kernel(
         const uint32_t g = first + (uint32_t)k * kThreads;
 
         if (g < a.groups) {
-            left[k] = m3_operand_load4<true>(a.left, g * 4U);
-            right[k] = m3_operand_load4<true>(a.right, g * 4U);
+            left[k] = m3_operand_load4<M3N_F32, true>(a.left, g * 4U);
+            right[k] = m3_operand_load4<M3N_F32, true>(a.right, g * 4U);
         } else {
             left[k] = make_uint4(0U, 0U, 0U, 0U);
             right[k] = left[k];
@@ -273,7 +330,7 @@ __global__ __launch_bounds__(256) void m3_binary_held_kernel(
         const uint32_t g = first + (uint32_t)k * kThreads;
 
         if (g < a.groups) {
-            m3_store4<true>(a.out, M3N_F32, g * 4U, left[k]);
+            m3_store4<M3N_F32>(a.out, M3N_F32, g * 4U, left[k]);
         }
     }
     /* Tail: the last count % 4 elements. */
@@ -281,8 +338,163 @@ __global__ __launch_bounds__(256) void m3_binary_held_kernel(
         uint32_t f = a.groups * 4U + threadIdx.x;
 
         *(uint32_t *)(a.out + (uint64_t)f * 4U) = m3_binary_f32_bits(
-            OP, m3_operand_element<true>(a.left, f),
-            m3_operand_element<true>(a.right, f));
+            OP, m3_operand_element<M3N_F32>(a.left, f),
+            m3_operand_element<M3N_F32>(a.right, f));
+    }
+}
+
+/* ---- chains ----------------------------------------------------------------- */
+
+constexpr uint32_t kChainCast = 4U; /* an op after the four of m3_numeric.h */
+
+/* One operation of a chain: value = value (op) other, or other (op) value,
+ * or a cast; the result rounded to out_dtype and stored at out. */
+struct m3_chain_step {
+    m3_bin_operand other;
+    uint8_t *out;
+    uint32_t out_dtype;
+    uint32_t op;
+    uint32_t other_left;
+};
+
+struct m3_chain_args {
+    m3_bin_operand value; /* the first operation's left operand */
+    m3_chain_step steps[M3_HIP_MAX_CHAIN];
+    uint32_t count;  /* elements, < 2^32 */
+    uint32_t groups; /* count / 4 */
+    m3_hip_gate list_gate;
+};
+
+/* Four results of one operation (the same in every lane), with the NaN
+ * rule applied only in a wave that holds a NaN. */
+__device__ __forceinline__ uint4 m3_chain_op4(uint32_t op, uint4 x, uint4 y)
+{
+    const float4 a = make_float4(m3_bits_f32(x.x), m3_bits_f32(x.y),
+                                 m3_bits_f32(x.z), m3_bits_f32(x.w));
+    const float4 b = make_float4(m3_bits_f32(y.x), m3_bits_f32(y.y),
+                                 m3_bits_f32(y.z), m3_bits_f32(y.w));
+    float4 r;
+
+    if (op == M3N_ADD) {
+        r = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+    } else if (op == M3N_MUL) {
+        r = make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w);
+    } else if (op == M3N_SUB) {
+        r = make_float4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w);
+    } else {
+        r = make_float4(a.x / b.x, a.y / b.y, a.z / b.z, a.w / b.w);
+    }
+    uint4 v = make_uint4(m3_f32_bits(r.x), m3_f32_bits(r.y),
+                         m3_f32_bits(r.z), m3_f32_bits(r.w));
+
+    if (__any(r.x != r.x || r.y != r.y || r.z != r.z || r.w != r.w)) {
+        const int commutative = op == M3N_ADD || op == M3N_MUL;
+
+        v.x = m3_binary_nan_fix(v.x, x.x, y.x, commutative);
+        v.y = m3_binary_nan_fix(v.y, x.y, y.y, commutative);
+        v.z = m3_binary_nan_fix(v.z, x.z, y.z, commutative);
+        v.w = m3_binary_nan_fix(v.w, x.w, y.w, commutative);
+    }
+    return v;
+}
+
+/* Runs of up to M3_HIP_MAX_CHAIN operations over one element space, each
+ * taking the one before as an operand: a lane loads every operand of its
+ * groups of four, applies the operations in order, rounding each result to
+ * its output's dtype as a store and a load back would, and stores all
+ * results. Bound by HBM: a separate launch per operation also reads every
+ * intermediate result back. DT: every operand and output is of that dtype
+ * (kAnyDtype: each its own), which drops the choice per value that bound
+ * 16-bit chains by instructions. Measured against one launch per
+ * operation: F32 x[2,512,24001] * s[512,1] + b[512,1] 67.5 -> 44.8 us (6.6
+ * TB/s), BF16 107 -> 32.7, F16 120 -> 40.4; x[8,1024,1536] * c[1536] then
+ * to BF16 and back to F32 47.4 -> 28.8. Two groups per lane and one tile
+ * per workgroup: one group 29.8 and 46.0, four 30.6 and 46.8; 16 workgroups
+ * per CU in a loop the same within 1%. */
+template <int STEPS, uint32_t DT, int UNROLL>
+__global__ __launch_bounds__(256) void m3_chain_kernel(m3_chain_args a)
+{
+    if (m3_gate_closed(a.list_gate)) {
+        return; /* a check earlier in the list failed */
+    }
+    const uint32_t step = gridDim.x * kThreads * UNROLL;
+
+    for (uint32_t first = blockIdx.x * kThreads * UNROLL + threadIdx.x;
+         first < a.groups; first += step) {
+        uint4 value[UNROLL];
+        uint4 other[UNROLL][STEPS];
+
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            /* groups past the end read the last one and store nothing */
+            const uint32_t f =
+                4U * min(first + u * kThreads, a.groups - 1U);
+
+            value[u] = m3_operand_load4<DT>(a.value, f);
+#pragma unroll
+            for (int k = 0; k < STEPS; ++k) {
+                if (a.steps[k].op != kChainCast) {
+                    other[u][k] =
+                        m3_operand_load4<DT>(a.steps[k].other, f);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t g = first + u * kThreads;
+
+#pragma unroll
+            for (int k = 0; k < STEPS; ++k) {
+                const m3_chain_step &s = a.steps[k];
+                const uint32_t dtype = DT == kAnyDtype ? s.out_dtype : DT;
+
+                if (s.op != kChainCast) {
+                    const bool left = s.other_left != 0U;
+
+                    value[u] = m3_chain_op4(s.op,
+                                            left ? other[u][k] : value[u],
+                                            left ? value[u] : other[u][k]);
+                }
+                if (dtype == M3N_F32) {
+                    if (g < a.groups) {
+                        m3_stream_store((uint4 *)s.out + g, value[u]);
+                    }
+                    continue;
+                }
+                const uint2 raw = m3_narrow4_bits(value[u], dtype);
+
+                if (g < a.groups) {
+                    m3_stream_store((uint2 *)s.out + g, raw);
+                }
+                value[u] = m3_widen4_bits(raw, dtype);
+            }
+        }
+    }
+    /* Tail: the last count % 4 elements. */
+    if (blockIdx.x == 0U && threadIdx.x < a.count - a.groups * 4U) {
+        const uint32_t f = a.groups * 4U + threadIdx.x;
+        uint32_t v = m3_operand_element<DT>(a.value, f);
+
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k) {
+            const m3_chain_step &s = a.steps[k];
+            const uint32_t dtype = DT == kAnyDtype ? s.out_dtype : DT;
+
+            if (s.op != kChainCast) {
+                const uint32_t o = m3_operand_element<DT>(s.other, f);
+                const bool left = s.other_left != 0U;
+
+                v = m3_binary_f32_bits(s.op, left ? o : v, left ? v : o);
+            }
+            const uint32_t raw = m3_store_from_f32_bits(v, dtype);
+
+            if (dtype == M3N_F32) {
+                *(uint32_t *)(s.out + (uint64_t)f * 4U) = raw;
+            } else {
+                *(uint16_t *)(s.out + (uint64_t)f * 2U) = (uint16_t)raw;
+            }
+            v = m3_load_as_f32_bits(raw, dtype);
+        }
     }
 }
 
@@ -388,22 +600,21 @@ bool m3_classify_operand(const m3_index_plan &plan, uint32_t k,
     operand->inner = m3_fast_div_make((uint32_t)expected[live]);
     operand->period = m3_fast_div_make((uint32_t)plan.shape[live]);
     operand->mode = M3_BIN_PERIODIC;
-    if (expected[live] == 1U && plan.shape[live] % 4U == 0U) {
-        operand->mode = M3_BIN_TRAIL;
-    } else if (expected[live] % 4U == 0U) {
-        operand->mode = M3_BIN_ROW;
+    if (expected[live] == 1U && plan.shape[live] >= 4U) {
+        operand->mode = plan.shape[live] % 4U == 0U ? M3_BIN_TRAIL
+                                                    : M3_BIN_TRAIL_CUT;
+    } else if (expected[live] >= 4U) {
+        operand->mode = expected[live] % 4U == 0U ? M3_BIN_ROW
+                                                  : M3_BIN_ROW_CUT;
     }
     return true;
 }
 
-bool m3_vector_aligned(const m3_bin_operand &o)
+/* True for the modes that give a group one element or one vector. */
+bool m3_operand_whole(const m3_bin_operand &o)
 {
-    uint32_t bytes = o.dtype == M3N_F32 ? 16U : 8U;
-
-    if (o.mode != M3_BIN_FULL && o.mode != M3_BIN_TRAIL) {
-        return true;
-    }
-    return ((uintptr_t)o.base % bytes) == 0U;
+    return o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL ||
+           o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR;
 }
 
 template <int OP>
@@ -417,16 +628,13 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
     m3_index_plan plan;
     m3_bin_vec_args vec;
     uint8_t *out = (uint8_t *)output->base + output->byte_offset;
-    uint32_t out_bytes = output->dtype == M3N_F32 ? 16U : 8U;
 
     m3_plan_index_space(output, operands, 3U, &plan);
     std::memset(&vec, 0, sizeof(vec));
     vec.list_gate = device->gate;
     if (output->element_count < (1ULL << 32U) &&
-        ((uintptr_t)out % out_bytes) == 0U &&
         m3_classify_operand(plan, 1U, left, &vec.left) &&
-        m3_classify_operand(plan, 2U, right, &vec.right) &&
-        m3_vector_aligned(vec.left) && m3_vector_aligned(vec.right)) {
+        m3_classify_operand(plan, 2U, right, &vec.right)) {
         bool f32 = left->dtype == M3N_F32 && right->dtype == M3N_F32 &&
                    output->dtype == M3N_F32;
 
@@ -450,7 +658,9 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
         const uint64_t slots =
             (uint64_t)device->compute_units * kHeldBlocksPerCu;
         const bool hold = f32 && device->wall_clock_khz != 0U &&
-                          2U * held >= slots && held <= slots;
+                          2U * held >= slots && held <= slots &&
+                          m3_operand_whole(vec.left) &&
+                          m3_operand_whole(vec.right);
         /* the full operands' bytes (broadcast ones are read from cache) */
         const double read_bytes =
             4.0 * (double)vec.count *
@@ -469,12 +679,12 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
                         dim3((uint32_t)held), dim3(kThreads), 0,
                         device->stream, start, stop, 0U, vec, hold_ticks);
                 } else if (f32) {
-                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, true>),
+                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, M3N_F32>),
                                           dim3(blocks), dim3(kThreads), 0,
                                           device->stream, start, stop, 0U,
                                           vec);
                 } else {
-                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, false>),
+                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, kAnyDtype>),
                                           dim3(blocks), dim3(kThreads), 0,
                                           device->stream, start, stop, 0U,
                                           vec);
@@ -512,7 +722,155 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
         message, capacity);
 }
 
+typedef void (*m3_chain_launcher)(dim3, hipStream_t, hipEvent_t, hipEvent_t,
+                                  const m3_chain_args &);
+
+constexpr int kChainUnroll = 2; /* groups in flight per lane */
+constexpr uint32_t kChainBlocksPerCu = 1024U; /* one tile per workgroup */
+
+template <int STEPS, uint32_t DT>
+void m3_launch_chain(dim3 grid, hipStream_t stream, hipEvent_t start,
+                     hipEvent_t stop, const m3_chain_args &args)
+{
+    hipExtLaunchKernelGGL((m3_chain_kernel<STEPS, DT, kChainUnroll>),
+                          grid, dim3(kThreads), 0, stream, start, stop, 0U,
+                          args);
+}
+
+bool m3_chain_is_float(const m3_hip_view *view)
+{
+    return m3_view_is_valid(view) && view->dtype != M3_HIP_I32;
+}
+
+/* True when the two views are of one shape. */
+bool m3_chain_same_shape(const m3_hip_view *a, const m3_hip_view *b)
+{
+    return a->rank == b->rank && m3_view_broadcasts_to(a, b) &&
+           a->element_count == b->element_count;
+}
+
+/* Fills the kernel's arguments from a chain of binary operations and casts;
+ * false when the chain kernel does not take it: an operand that does not
+ * classify, more than 2^32 elements, or an output that overlaps what
+ * another operation reads or writes (the launch would no longer equal the
+ * operations in order). */
+bool m3_chain_plan(const m3_hip_chain_command *commands, uint32_t count,
+                   m3_chain_args *args)
+{
+    const m3_hip_view *space = &commands[0].output;
+
+    for (uint32_t k = 0U; k < count; ++k) {
+        const m3_hip_chain_command &c = commands[k];
+        const bool cast = c.kind == M3_HIP_CHAIN_CAST;
+        /* the operand that is not the chain's value (none of a cast) */
+        const bool other_left = k != 0U && !cast && c.link != 0U;
+        const m3_hip_view *value = other_left ? &c.right : &c.left;
+        const m3_hip_view *other = other_left ? &c.left : &c.right;
+        m3_chain_step *step = &args->steps[k];
+
+        if ((!cast && (c.kind != M3_HIP_CHAIN_BINARY || c.op > M3_HIP_DIV)) ||
+            !m3_chain_is_float(&c.output) || !m3_chain_is_float(value) ||
+            (!cast && !m3_chain_is_float(other)) ||
+            !m3_view_is_contiguous(&c.output) ||
+            !m3_chain_same_shape(&c.output, space)) {
+            return false;
+        }
+        for (uint32_t i = 0U; i < k; ++i) {
+            if (m3_views_overlap(&commands[i].output, &c.output) ||
+                (!cast && m3_views_overlap(&commands[i].output, other))) {
+                return false;
+            }
+        }
+        /* what this and earlier operations load, against this output */
+        for (uint32_t i = 0U; i <= k; ++i) {
+            const m3_hip_chain_command &e = commands[i];
+            const bool e_cast = e.kind == M3_HIP_CHAIN_CAST;
+            const bool e_left = i == 0U || (!e_cast && e.link != 0U);
+            const bool e_right = !e_cast && (i == 0U || e.link == 0U);
+
+            if ((e_left && m3_views_overlap(&e.left, &c.output)) ||
+                (e_right && m3_views_overlap(&e.right, &c.output))) {
+                return false;
+            }
+        }
+        const m3_hip_view *operands[3] = {&c.output, value,
+                                          cast ? value : other};
+        m3_index_plan plan;
+
+        if ((k == 0U && !m3_view_broadcasts_to(value, &c.output)) ||
+            (!cast && !m3_view_broadcasts_to(other, &c.output))) {
+            return false;
+        }
+        m3_plan_index_space(&c.output, operands, 3U, &plan);
+        if ((k == 0U && !m3_classify_operand(plan, 1U, value, &args->value)) ||
+            (!cast && !m3_classify_operand(plan, 2U, other, &step->other))) {
+            return false;
+        }
+        step->out = (uint8_t *)c.output.base + c.output.byte_offset;
+        step->out_dtype = c.output.dtype;
+        step->op = cast ? kChainCast : c.op;
+        step->other_left = other_left ? 1U : 0U;
+    }
+    args->count = (uint32_t)space->element_count;
+    args->groups = args->count / 4U;
+    return space->element_count != 0U &&
+           space->element_count < (1ULL << 32U);
+}
+
 } // namespace
+
+extern "C" int m3_hip_launch_chain(m3_hip_device *device,
+                                   const m3_hip_chain_command *commands,
+                                   uint32_t count, int *taken, char *message,
+                                   size_t capacity)
+{
+    /* [operations - 2][the one dtype throughout, or 3: several] */
+    static const m3_chain_launcher launchers[M3_HIP_MAX_CHAIN - 1][4] = {
+        {&m3_launch_chain<2, M3N_F32>, &m3_launch_chain<2, M3N_F16>,
+         &m3_launch_chain<2, M3N_BF16>, &m3_launch_chain<2, kAnyDtype>},
+        {&m3_launch_chain<3, M3N_F32>, &m3_launch_chain<3, M3N_F16>,
+         &m3_launch_chain<3, M3N_BF16>, &m3_launch_chain<3, kAnyDtype>}};
+    m3_chain_args args;
+    uint32_t dtype;
+
+    if (device == nullptr || commands == nullptr || taken == nullptr ||
+        count < 2U || count > M3_HIP_MAX_CHAIN) {
+        return m3_hip_fail(message, capacity, M3_HIP_INVALID,
+                           "chain launch arguments are malformed");
+    }
+    *taken = 0;
+    if (count == 2U && commands[0].kind == M3_HIP_CHAIN_SNAKE1D &&
+        commands[1].kind == M3_HIP_CHAIN_TANH) {
+        return m3_snake1d_tanh(device, commands, taken, message, capacity);
+    }
+    std::memset(&args, 0, sizeof(args));
+    if (!m3_chain_plan(commands, count, &args)) {
+        return M3_HIP_OK;
+    }
+    args.list_gate = device->gate;
+    dtype = args.value.dtype;
+    for (uint32_t k = 0U; k < count; ++k) {
+        if (args.steps[k].out_dtype != dtype ||
+            (args.steps[k].op != kChainCast &&
+             args.steps[k].other.dtype != dtype)) {
+            dtype = 3U;
+            break;
+        }
+    }
+    const dim3 grid(m3_grid_blocks(device,
+                                   args.groups == 0U ? 1U : args.groups,
+                                   kThreads * kChainUnroll,
+                                   kChainBlocksPerCu));
+    const m3_chain_launcher launcher = launchers[count - 2U][dtype];
+
+    *taken = 1;
+    return m3_hip_launch(
+        device, "m3_chain",
+        [&](hipEvent_t start, hipEvent_t stop) {
+            launcher(grid, device->stream, start, stop, args);
+        },
+        message, capacity);
+}
 
 extern "C" int m3_hip_launch_binary(m3_hip_device *device, uint32_t op,
                                     const m3_hip_view *left,

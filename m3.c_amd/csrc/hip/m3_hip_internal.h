@@ -263,6 +263,64 @@ __device__ __forceinline__ float4 m3_stream_load(const float4 *p)
     return make_float4(w.x, w.y, w.z, w.w);
 }
 
+/* Four F32 values (as bits) rounded to a 16-bit float dtype, packed. The
+ * hardware's conversions round to nearest even; v_cvt_pk_bf16_f32 gives the
+ * bits of m3_f32_to_bf16_bits for every F32, v_cvt_f16_f32 those of
+ * m3_f32_to_f16_bits for every F32 but NaN. */
+typedef _Float16 m3_f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 m3_bf16x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint2 m3_narrow4_bits(uint4 v, uint32_t dtype)
+{
+    const m3_f32x4 x = {m3_bits_f32(v.x), m3_bits_f32(v.y), m3_bits_f32(v.z),
+                        m3_bits_f32(v.w)};
+    m3_u32x2 h;
+
+    if (dtype == M3N_BF16) {
+        h = __builtin_bit_cast(m3_u32x2,
+                               __builtin_convertvector(x, m3_bf16x4));
+    } else {
+        h = __builtin_bit_cast(m3_u32x2,
+                               __builtin_convertvector(x, m3_f16x4));
+        if (__any(x[0] != x[0] || x[1] != x[1] || x[2] != x[2] ||
+                  x[3] != x[3])) {
+            h[0] = m3_f32_to_f16_bits(v.x) | (m3_f32_to_f16_bits(v.y) << 16U);
+            h[1] = m3_f32_to_f16_bits(v.z) | (m3_f32_to_f16_bits(v.w) << 16U);
+        }
+    }
+    return make_uint2(h[0], h[1]);
+}
+
+/* Four packed 16-bit floats widened to F32 bits; v_cvt_f32_f16 gives those
+ * of m3_f16_to_f32_bits for every value but a signalling NaN. */
+__device__ __forceinline__ uint4 m3_widen4_bits(uint2 h, uint32_t dtype)
+{
+    if (dtype == M3N_BF16) {
+        return make_uint4(h.x << 16U, h.x & 0xffff0000U, h.y << 16U,
+                          h.y & 0xffff0000U);
+    }
+    const m3_u32x2 w = {h.x, h.y};
+    const m3_f16x4 x = __builtin_bit_cast(m3_f16x4, w);
+    uint4 v = make_uint4(m3_f32_bits((float)x[0]), m3_f32_bits((float)x[1]),
+                         m3_f32_bits((float)x[2]), m3_f32_bits((float)x[3]));
+
+    if (__any(x[0] != x[0] || x[1] != x[1] || x[2] != x[2] || x[3] != x[3])) {
+        v = make_uint4(m3_f16_to_f32_bits(h.x & 0xffffU),
+                       m3_f16_to_f32_bits(h.x >> 16U),
+                       m3_f16_to_f32_bits(h.y & 0xffffU),
+                       m3_f16_to_f32_bits(h.y >> 16U));
+    }
+    return v;
+}
+
+/* SNAKE1D then TANH of its output in one launch (m3_hip_snake1d.hip); takes
+ * the chain (*taken = 1) only where the vector kernel runs. */
+int m3_snake1d_tanh(m3_hip_device *device,
+                    const m3_hip_chain_command *commands, int *taken,
+                    char *message, size_t capacity);
+/* True when the byte ranges that two views' elements lie in meet. */
+bool m3_views_overlap(const m3_hip_view *a, const m3_hip_view *b);
+
 /* Unsigned 32-bit division by an invariant divisor d >= 1:
  * q = (umulhi(n, mul) + n) >> shift with shift = ceil(log2 d) and
  * mul = floor(2^32 (2^shift - d) / d) + 1; the sum is formed in 64 bits,

@@ -96,6 +96,31 @@ bool m3_view_broadcasts_to(const m3_hip_view *input,
     return true;
 }
 
+/* First and one-past-last byte that a view's elements occupy. */
+static void m3_view_extent(const m3_hip_view *view, uintptr_t *first,
+                           uintptr_t *end)
+{
+    uint64_t span = m3_dtype_bytes(view->dtype);
+
+    for (uint32_t axis = 0U; axis < view->rank; ++axis) {
+        span += (view->shape[axis] - 1U) * view->byte_strides[axis];
+    }
+    *first = (uintptr_t)view->base + view->byte_offset;
+    *end = *first + span;
+}
+
+bool m3_views_overlap(const m3_hip_view *a, const m3_hip_view *b)
+{
+    uintptr_t a_first;
+    uintptr_t a_end;
+    uintptr_t b_first;
+    uintptr_t b_end;
+
+    m3_view_extent(a, &a_first, &a_end);
+    m3_view_extent(b, &b_first, &b_end);
+    return a_first < b_end && b_first < a_end;
+}
+
 uint32_t m3_grid_blocks(const m3_hip_device *device, uint64_t items,
                         uint32_t threads, uint32_t per_cu)
 {

@@ -96,6 +96,7 @@ struct m3_snake_vec_args {
     const uint8_t *alpha; /* alpha element of channel 0 */
     int64_t alpha_stride; /* bytes between channels */
     float *output;
+    float *tanh_output;   /* tanhf of the output (TANH) */
     uint32_t groups;      /* elements / 4 */
     uint32_t tail;        /* elements % 4 */
     m3_fast_div length;   /* L >= 4 */
@@ -118,11 +119,29 @@ __device__ __forceinline__ float m3_snake_alpha(const m3_snake_vec_args &a,
     return *(const float *)(a.alpha + (int64_t)channel * a.alpha_stride);
 }
 
+template <bool TANH>
+__device__ __forceinline__ void m3_snake_put4(const m3_snake_vec_args &a,
+                                              uint32_t g, float4 y)
+{
+    m3_stream_store((float4 *)a.output + g, y);
+    if (TANH) {
+        m3_stream_store((float4 *)a.tanh_output + g,
+                        make_float4(m3_tanhf_uniform(y.x),
+                                    m3_tanhf_uniform(y.y),
+                                    m3_tanhf_uniform(y.z),
+                                    m3_tanhf_uniform(y.w)));
+    }
+}
+
 /* Groups of four consecutive elements, kUnroll per lane. L need not be a
  * multiple of 4: a group that a row's end cuts takes the next row's alpha
  * for its last elements, in the waves that hold one. Bound by HBM
  * (x[2,1536,65536] 264 us, 6.1 TB/s; x[2,192,60001] 30.5 us, 6.0 TB/s,
- * where one element per lane with 64-bit divisions took about 75). */
+ * where one element per lane with 64-bit divisions took about 75). TANH:
+ * tanhf of the output is stored too, in the launch of the TANH command
+ * after it, which then does not read it back: 78 -> 64 us for the two over
+ * x[2,192,60001], by then bound by instructions as much as by HBM. */
+template <bool TANH>
 __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
     m3_snake_vec_args a)
 {
@@ -153,9 +172,9 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
 
 #pragma unroll
             for (uint32_t u = 0U; u < kUnroll; ++u) {
-                m3_stream_store((float4 *)a.output + first + u * kThreads,
-                                m3_snake4(x[u], m3_splat4(alpha),
-                                          m3_splat4(inverse)));
+                m3_snake_put4<TANH>(a, first + u * kThreads,
+                                    m3_snake4(x[u], m3_splat4(alpha),
+                                              m3_splat4(inverse)));
             }
             continue;
         }
@@ -198,7 +217,7 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
             const float4 y = m3_snake4(x[u], alpha4, inverse4);
 
             if (first + u * kThreads < a.groups) {
-                m3_stream_store((float4 *)a.output + g, y);
+                m3_snake_put4<TANH>(a, g, y);
             }
         }
     }
@@ -208,8 +227,13 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
         const float alpha =
             m3_snake_alpha(a, m3_fast_div_q(a.length, (uint32_t)e));
 
-        a.output[e] =
+        const float y =
             m3_snake(a.input[e], alpha, m3_snake_inverse(alpha));
+
+        a.output[e] = y;
+        if (TANH) {
+            a.tanh_output[e] = m3_tanhf_uniform(y);
+        }
     }
 }
 
@@ -249,11 +273,22 @@ __global__ __launch_bounds__(256) void m3_snake1d_general_kernel(
 
 } // namespace
 
-extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
-                                     const m3_hip_view *input,
-                                     const m3_hip_view *alpha,
-                                     const m3_hip_view *output,
-                                     char *message, size_t capacity)
+/* True for the layouts of the vector kernel. */
+static bool m3_snake_vector(const m3_hip_view *input,
+                            const m3_hip_view *output)
+{
+    /* 32-bit element indices: below 2^32 with the lanes past the end (they
+     * read the last group) */
+    return m3_view_is_contiguous(input) && input->shape[2] >= 4U &&
+           output->element_count < (1ULL << 32U);
+}
+
+/* SNAKE1D, and tanhf of its output into tanh_output when not null (which
+ * the caller passes only for the vector kernel's layouts). */
+static int m3_snake_launch(m3_hip_device *device, const m3_hip_view *input,
+                           const m3_hip_view *alpha,
+                           const m3_hip_view *output, float *tanh_output,
+                           char *message, size_t capacity)
 {
     if (device == nullptr || !m3_view_is_valid(input) ||
         !m3_view_is_valid(alpha) || !m3_view_is_valid(output) ||
@@ -282,10 +317,7 @@ extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
                                ? (int64_t)alpha->byte_strides[1]
                                : 0;
 
-    /* 32-bit element indices: below 2^32 with the lanes past the end (they
-     * read the last group) */
-    if (m3_view_is_contiguous(input) && length >= 4U &&
-        output->element_count < (1ULL << 32U)) {
+    if (m3_snake_vector(input, output)) {
         m3_snake_vec_args args;
 
         std::memset(&args, 0, sizeof(args));
@@ -294,6 +326,7 @@ extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
         args.alpha = al;
         args.alpha_stride = alpha_stride;
         args.output = (float *)out;
+        args.tanh_output = tanh_output;
         args.groups = (uint32_t)(output->element_count / 4U);
         args.tail = (uint32_t)(output->element_count % 4U);
         args.length = m3_fast_div_make((uint32_t)length);
@@ -302,11 +335,19 @@ extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
                                          kThreads * kUnroll, kBlocksPerCu);
 
         return m3_hip_launch(
-            device, "m3_snake1d",
+            device, tanh_output != nullptr ? "m3_snake1d_tanh" : "m3_snake1d",
             [&](hipEvent_t start, hipEvent_t stop) {
-                hipExtLaunchKernelGGL(m3_snake1d_vec_kernel, dim3(blocks),
-                                      dim3(kThreads), 0, device->stream, start,
-                                      stop, 0U, args);
+                if (tanh_output != nullptr) {
+                    hipExtLaunchKernelGGL((m3_snake1d_vec_kernel<true>),
+                                          dim3(blocks), dim3(kThreads), 0,
+                                          device->stream, start, stop, 0U,
+                                          args);
+                } else {
+                    hipExtLaunchKernelGGL((m3_snake1d_vec_kernel<false>),
+                                          dim3(blocks), dim3(kThreads), 0,
+                                          device->stream, start, stop, 0U,
+                                          args);
+                }
             },
             message, capacity);
     }
@@ -334,4 +375,44 @@ extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
                                   0U, general);
         },
         message, capacity);
+}
+
+extern "C" int m3_hip_launch_snake1d(m3_hip_device *device,
+                                     const m3_hip_view *input,
+                                     const m3_hip_view *alpha,
+                                     const m3_hip_view *output,
+                                     char *message, size_t capacity)
+{
+    return m3_snake_launch(device, input, alpha, output, nullptr, message,
+                           capacity);
+}
+
+int m3_snake1d_tanh(m3_hip_device *device,
+                    const m3_hip_chain_command *commands, int *taken,
+                    char *message, size_t capacity)
+{
+    const m3_hip_view *input = &commands[0].left;
+    const m3_hip_view *alpha = &commands[0].right;
+    const m3_hip_view *output = &commands[0].output;
+    const m3_hip_view *wave = &commands[1].output;
+
+    /* shapes as m3_snake_launch checks them; the second output apart from
+     * all the others, the first from alpha (in place over the input the
+     * launch of SNAKE1D alone is as good) */
+    if (!m3_view_is_valid(input) || !m3_view_is_valid(alpha) ||
+        !m3_view_is_valid(output) || !m3_view_is_valid(wave) ||
+        input->rank != 3U || output->rank != 3U ||
+        output->element_count == 0U || wave->dtype != M3_HIP_F32 ||
+        wave->element_count != output->element_count ||
+        !m3_view_is_contiguous(wave) || !m3_snake_vector(input, output) ||
+        m3_views_overlap(input, output) || m3_views_overlap(alpha, output) ||
+        m3_views_overlap(input, wave) || m3_views_overlap(alpha, wave) ||
+        m3_views_overlap(output, wave)) {
+        return M3_HIP_OK;
+    }
+    *taken = 1;
+    return m3_snake_launch(
+        device, input, alpha, output,
+        (float *)((uint8_t *)wave->base + wave->byte_offset), message,
+        capacity);
 }

@@ -67,8 +67,6 @@ __device__ __align__(16) uint32_t m3_minus_inf[3][4] = {
     {0xfc00fc00U, 0xfc00fc00U, 0U, 0U},                   /* F16 */
     {0xff80ff80U, 0xff80ff80U, 0U, 0U}};                  /* BF16 */
 
-typedef _Float16 m3_f16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 m3_bf16x4 __attribute__((ext_vector_type(4)));
 
 struct m3_softmax_args {
     const uint8_t *input;

@@ -823,6 +823,120 @@ static int m3_hip_enqueue(m3_hip_backend_context *context,
     }
 }
 
+/* Fills `out` for a command that can be part of a chain
+ * (m3_hip_launch_chain), without its link; false for any other kind. */
+static bool m3_hip_chain_command_of(const m3_command *command,
+                                    m3_hip_chain_command *out)
+{
+    const m3_op_binary *binary = m3_hip_binary_of(command);
+
+    out->link = 0U;
+    out->op = 0U;
+    if (binary != NULL) {
+        out->kind = M3_HIP_CHAIN_BINARY;
+        out->op = command->kind == M3_OP_ADD   ? M3_HIP_ADD
+                  : command->kind == M3_OP_MUL ? M3_HIP_MUL
+                  : command->kind == M3_OP_SUB ? M3_HIP_SUB
+                                               : M3_HIP_DIV;
+        m3_hip_view_of(binary->left, &out->left);
+        m3_hip_view_of(binary->right, &out->right);
+        m3_hip_view_of(binary->output, &out->output);
+        return true;
+    }
+    switch (command->kind) {
+    case M3_OP_CAST:
+        /* between float dtypes: one to I32 is checked, an equal one copies
+         * raw bits */
+        if (command->descriptor.cast.input->metadata.dtype == M3_DTYPE_I32 ||
+            command->descriptor.cast.output->metadata.dtype == M3_DTYPE_I32 ||
+            command->descriptor.cast.input->metadata.dtype ==
+                command->descriptor.cast.output->metadata.dtype) {
+            return false;
+        }
+        out->kind = M3_HIP_CHAIN_CAST;
+        m3_hip_view_of(command->descriptor.cast.input, &out->left);
+        m3_hip_view_of(command->descriptor.cast.output, &out->output);
+        return true;
+    case M3_OP_SNAKE1D:
+        out->kind = M3_HIP_CHAIN_SNAKE1D;
+        m3_hip_view_of(command->descriptor.snake1d.input, &out->left);
+        m3_hip_view_of(command->descriptor.snake1d.alpha, &out->right);
+        m3_hip_view_of(command->descriptor.snake1d.output, &out->output);
+        return true;
+    case M3_OP_TANH:
+        out->kind = M3_HIP_CHAIN_TANH;
+        m3_hip_view_of(command->descriptor.tanh.input, &out->left);
+        m3_hip_view_of(command->descriptor.tanh.output, &out->output);
+        return true;
+    default:
+        return false;
+    }
+}
+
+/* How many commands from commands[index] on form a chain (1: none): each
+ * after the first takes the output of the one before, the same view, as
+ * exactly one of its operands. SNAKE1D chains only with a TANH after it,
+ * binary operations and casts with each other. */
+static uint32_t m3_hip_chain_length(const m3_command *commands, size_t count,
+                                    size_t index,
+                                    m3_hip_chain_command *chain)
+{
+    uint32_t length = 1U;
+
+    if (index + 1U >= count ||
+        !m3_hip_chain_command_of(&commands[index], &chain[0]) ||
+        chain[0].kind == M3_HIP_CHAIN_TANH) {
+        return 1U;
+    }
+    while (length < M3_HIP_MAX_CHAIN && index + length < count) {
+        const m3_hip_chain_command *before = &chain[length - 1U];
+        m3_hip_chain_command *next = &chain[length];
+        bool left;
+        bool right;
+
+        if (!m3_hip_chain_command_of(&commands[index + length], next) ||
+            (before->kind == M3_HIP_CHAIN_SNAKE1D) !=
+                (next->kind == M3_HIP_CHAIN_TANH) ||
+            before->kind == M3_HIP_CHAIN_TANH ||
+            next->kind == M3_HIP_CHAIN_SNAKE1D) {
+            break;
+        }
+        left = m3_hip_same_view(&next->left, &before->output);
+        right = next->kind == M3_HIP_CHAIN_BINARY &&
+                m3_hip_same_view(&next->right, &before->output);
+        if (left == right) {
+            break;
+        }
+        next->link = right ? 1U : 0U;
+        length += 1U;
+    }
+    return length;
+}
+
+/* Launches the chain that begins at commands[index], if there is one that a
+ * kernel takes: *taken receives how many commands it was (0: none, nothing
+ * launched). */
+static int m3_hip_enqueue_chain(m3_hip_backend_context *context,
+                                const m3_command *commands, size_t count,
+                                size_t index, size_t *taken, char *message,
+                                size_t capacity)
+{
+    m3_hip_chain_command chain[M3_HIP_MAX_CHAIN];
+    uint32_t length = m3_hip_chain_length(commands, count, index, chain);
+    int made = 0;
+    int code = M3_HIP_OK;
+
+    *taken = 0U;
+    for (; length >= 2U && made == 0 && code == M3_HIP_OK; --length) {
+        code = m3_hip_launch_chain(context->device, chain, length, &made,
+                                   message, capacity);
+        if (made != 0) {
+            *taken = length;
+        }
+    }
+    return code;
+}
+
 static m3_status m3_hip_execute(void *opaque, const m3_command *commands,
                                 size_t count, m3_scratch_arena *scratch,
                                 m3_error *error)
@@ -869,6 +983,20 @@ static m3_status m3_hip_execute(void *opaque, const m3_command *commands,
         m3_hip_forget_outputs(context, &commands[i]);
         checked = m3_hip_fusable_check(commands, count, i, &kind);
         if (checked == NULL) {
+            size_t taken = 0U;
+
+            code = m3_hip_enqueue_chain(context, commands, count, i, &taken,
+                                        message, sizeof(message));
+            if (taken != 0U) {
+                for (; taken > 1U; --taken) {
+                    i += 1U;
+                    m3_hip_forget_outputs(context, &commands[i]);
+                }
+                continue;
+            }
+            if (code != M3_HIP_OK) {
+                continue;
+            }
             code = m3_hip_enqueue(context, &commands[i], message,
                                   sizeof(message));
             continue;
