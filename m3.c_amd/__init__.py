@@ -194,7 +194,7 @@ EXPORTS_HIP = [
     "m3_hip_device_properties", "m3_hip_arena_reserve",
     "m3_hip_arena_release", "m3_hip_copy_h2d", "m3_hip_copy_d2h",
     "m3_hip_fill_zero", "m3_hip_launch_binary", "m3_hip_launch_cast",
-    "m3_hip_launch_copy", "m3_hip_launch_softmax", "m3_hip_launch_snake1d",
+    "m3_hip_launch_chain", "m3_hip_launch_copy", "m3_hip_launch_softmax", "m3_hip_launch_snake1d",
     "m3_hip_scan_views", "m3_hip_synchronize", "m3_hip_timing_enable",
     "m3_hip_timing_reset", "m3_hip_timing_read", "m3_hip_timing_samples",
     "m3_hip_stream",
