@@ -1,0 +1,118 @@
+"""Host copies through the device's pinned staging memory (GPU).
+
+Copies of 257 bytes to 192 KiB to the device, and of up to 256 KiB or 1 to 4
+MiB from it, go through staging memory, reads in chunks; others, and those
+with timing on, take other paths. Sizes at the edges of the paths and chunks, at
+any byte offset, and from several threads over one device.
+"""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+from conftest import m3
+
+pytestmark = pytest.mark.gpu
+
+KIB = 1 << 10
+MIB = 1 << 20
+
+
+class Device:
+    def __init__(self, arena_bytes):
+        _, self.hip = m3.load()
+        vp, sz = ctypes.c_void_p, ctypes.c_size_t
+        self.hip.m3_hip_arena_reserve.argtypes = [vp, sz, ctypes.POINTER(vp),
+                                                  ctypes.c_char_p, sz]
+        self.hip.m3_hip_arena_release.argtypes = [vp, vp]
+        for name in ("m3_hip_copy_h2d", "m3_hip_copy_d2h"):
+            getattr(self.hip, name).argtypes = [vp, vp, vp, sz,
+                                                ctypes.c_char_p, sz]
+        self.device = vp()
+        self.base = vp()
+        message = ctypes.create_string_buffer(256)
+        assert self.hip.m3_hip_device_open(0, ctypes.byref(self.device),
+                                           message, 256) == 0
+        assert self.hip.m3_hip_arena_reserve(
+            self.device, arena_bytes, ctypes.byref(self.base), message,
+            256) == 0
+
+    def write(self, offset, array):
+        message = ctypes.create_string_buffer(256)
+        assert self.hip.m3_hip_copy_h2d(
+            self.device, self.base.value + offset,
+            array.ctypes.data, array.nbytes, message, 256) == 0, message.value
+
+    def read(self, offset, count):
+        out = np.empty(count, np.uint8)
+        message = ctypes.create_string_buffer(256)
+        assert self.hip.m3_hip_copy_d2h(
+            self.device, out.ctypes.data, self.base.value + offset, count,
+            message, 256) == 0, message.value
+        return out
+
+    def close(self):
+        self.hip.m3_hip_arena_release(self.device, self.base)
+        self.hip.m3_hip_device_close(self.device)
+
+
+@pytest.fixture()
+def device(gpu):
+    opened = Device(16 * MIB)
+    yield opened
+    opened.close()
+
+
+@pytest.mark.parametrize("count", [
+    1, 255, 256, 257, 1000, 4096, 192 * KIB, 192 * KIB + 1, 256 * KIB - 1, 256 * KIB, 256 * KIB + 1,
+    512 * KIB, 512 * KIB + 4, 700001, MIB - 65, MIB - 1, MIB, 3 * MIB + 7, 4 * MIB, 4 * MIB + 1])
+@pytest.mark.parametrize("offset", [0, 1, 2, 4, 6])
+def test_copy_sizes(device, count, offset):
+    rng = np.random.default_rng(count + offset)
+    room = count + 64
+    before = rng.integers(0, 256, room, np.uint8)
+    data = rng.integers(0, 256, count, np.uint8)
+    device.write(0, before)
+    device.write(offset, data)
+    expected = before.copy()
+    expected[offset:offset + count] = data
+    assert np.array_equal(device.read(0, room), expected)
+    assert np.array_equal(device.read(offset, count), data)
+
+
+def test_many_writes_in_order(device):
+    """Writes one after the other, overlapping and reusing the staging
+    memory, take effect in order."""
+    rng = np.random.default_rng(5)
+    expected = np.zeros(2 * MIB, np.uint8)
+    device.write(0, expected)
+    for k in range(200):
+        count = int(rng.integers(1, 300 * KIB))
+        offset = int(rng.integers(0, 2 * MIB - count))
+        data = np.full(count, k & 255, np.uint8)
+        device.write(offset, data)
+        data[:] = 77  # the caller's buffer is free when the call returns
+        expected[offset:offset + count] = k & 255
+    assert np.array_equal(device.read(0, 2 * MIB), expected)
+
+
+def test_threads_copy_through_one_device(device):
+    failures = []
+
+    def work(index):
+        rng = np.random.default_rng(index)
+        base = index * 4 * MIB
+        for _ in range(40):
+            count = int(rng.integers(257, 600 * KIB))
+            data = rng.integers(0, 256, count, np.uint8)
+            device.write(base, data)
+            if not np.array_equal(device.read(base, count), data):
+                failures.append((index, count))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not failures
