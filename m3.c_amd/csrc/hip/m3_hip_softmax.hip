@@ -505,7 +505,7 @@ __device__ __forceinline__ float m3_to_second_half(float x)
         (int)m3_f32_bits(x), (int)m3_f32_bits(x), 0x142, 0xA, 0xF, false));
 }
 
-/* Rows of 32Q + 1 .. 64Q columns, Q = 8 or 16, with the in-order sum
+/* Rows of 32Q + 1 .. 64Q columns, Q = 4, 8 or 16, with the in-order sum
  * carried in registers. A wave takes four consecutive rows, one per 16-lane
  * DPP row (lanes 16k..16k+15 hold row k); lane i of a row holds columns
  * 4i + 64j .. 4i + 64j + 3 (block j = 0..Q-1), so each load instruction
@@ -2168,10 +2168,10 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                 },
                 message, capacity);
         }
-        /* Rows of 257..2048 columns: the lane-row kernel, 8 or 16 float4
-         * per lane and, beyond 1024 columns, a row in two halves
-         * (index: [class][full][F32 I/O]). */
-        static const m3_softmax_launcher lane_launchers[3][2][2] = {
+        /* Rows of 257..2048 columns: the lane-row kernel, 4, 8 or 16 float4
+         * per lane, a row in one piece or in two halves (index:
+         * [class][full][F32 I/O]). */
+        static const m3_softmax_launcher lane_launchers[5][2][2] = {
             {{&m3_launch_lane_rows<8, false, false, false>,
               &m3_launch_lane_rows<8, false, false, true>},
              {&m3_launch_lane_rows<8, true, false, false>,
@@ -2183,11 +2183,27 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
             {{&m3_launch_lane_rows<16, false, true, false>,
               &m3_launch_lane_rows<16, false, true, true>},
              {&m3_launch_lane_rows<16, false, true, false>,
-              &m3_launch_lane_rows<16, false, true, true>}}};
-        const uint32_t lane_class = width <= 512U    ? 0U
-                                    : width <= 1024U ? 1U
-                                                     : 2U;
-        const uint32_t lane_rows = lane_class == 2U ? 2U : 4U; /* per wave */
+              &m3_launch_lane_rows<16, false, true, true>}},
+            {{&m3_launch_lane_rows<4, false, true, false>,
+              &m3_launch_lane_rows<4, false, true, true>},
+             {&m3_launch_lane_rows<4, false, true, false>,
+              &m3_launch_lane_rows<4, false, true, true>}},
+            {{&m3_launch_lane_rows<8, false, true, false>,
+              &m3_launch_lane_rows<8, false, true, true>},
+             {&m3_launch_lane_rows<8, false, true, false>,
+              &m3_launch_lane_rows<8, false, true, true>}}};
+        /* few rows (at most a wave of two per SIMD): two per wave in
+         * halves, half the exponentials per lane and so less latency: F32
+         * [16,777] 9.4 -> 7.5 us, [1000,777] 10.5 -> 8.4, [2000,1024] 10.8
+         * -> 9.5, [256,300] 6.0 -> 5.7; with more rows a SIMD has other
+         * waves to run, and four per wave need half the additions */
+        const bool few_rows =
+            rows <= 2U * 4U * (uint64_t)device->compute_units;
+        const uint32_t lane_class = width > 1024U ? 2U
+                                    : width > 512U ? few_rows ? 4U : 1U
+                                    : few_rows     ? 3U
+                                                   : 0U;
+        const uint32_t lane_rows = lane_class >= 2U ? 2U : 4U; /* per wave */
         const uint64_t lane_blocks =
             (rows + lane_rows * kWaves - 1U) / (lane_rows * kWaves);
 
@@ -2239,19 +2255,33 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
        &m3_launch_wide<Q, NW, true, false>},                                  \
       {&m3_launch_wide<Q, NW, false, true>,                                   \
        &m3_launch_wide<Q, NW, true, true>}}}
-            static const struct {
+            struct row_class {
                 uint32_t columns;
                 m3_softmax_launcher launch[2][2]; /* [ragged][F32 I/O] */
-            } classes[] = {M3_WIDE_ENTRY(8, 2),  M3_WIDE_ENTRY(16, 2),
-                           M3_WIDE_ENTRY(12, 4), M3_WIDE_ENTRY(16, 4),
-                           M3_WIDE_ENTRY(10, 8), M3_WIDE_ENTRY(12, 8),
-                           M3_WIDE_ENTRY(16, 8),  M3_WIDE_ENTRY(12, 16),
-                           M3_WIDE_ENTRY(16, 16)};
+            };
+            static const row_class many[] = {
+                M3_WIDE_ENTRY(8, 2),  M3_WIDE_ENTRY(16, 2),
+                M3_WIDE_ENTRY(12, 4), M3_WIDE_ENTRY(16, 4),
+                M3_WIDE_ENTRY(10, 8), M3_WIDE_ENTRY(12, 8),
+                M3_WIDE_ENTRY(16, 8), M3_WIDE_ENTRY(12, 16),
+                M3_WIDE_ENTRY(16, 16)};
+            /* at most a row per CU: nothing shares the CU with the row, so
+             * its latency is all that counts, and more waves of fewer
+             * values shorten all of it but the walk: F32 [16,4096] 12.3 ->
+             * 10.0 us, [16,8192] 19.4 -> 13.3, [256,8192] 20.0 -> 13.8,
+             * [16,16384] 20.5 -> 15.7, [16,32003] 24.0 -> 21.2; sixteen
+             * waves were slower for [16,20001], 19.9 against 19.1 */
+            static const row_class few[] = {
+                M3_WIDE_ENTRY(4, 4), M3_WIDE_ENTRY(4, 8),
+                M3_WIDE_ENTRY(4, 16), M3_WIDE_ENTRY(10, 8),
+                M3_WIDE_ENTRY(8, 16), M3_WIDE_ENTRY(12, 16),
+                M3_WIDE_ENTRY(16, 16)};
 #undef M3_WIDE_ENTRY
-            uint32_t which = 0U;
+            const row_class *chosen =
+                rows <= device->compute_units ? few : many;
 
-            while (classes[which].columns < width) {
-                ++which;
+            while (chosen->columns < width) {
+                ++chosen;
             }
             const uint64_t cap =
                 device->softmax_wide_grid != 0U &&
@@ -2259,7 +2289,8 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
                     ? device->softmax_wide_grid
                     : kMaxGrid;
             const dim3 grid((uint32_t)(rows < cap ? rows : cap));
-            const m3_softmax_launcher launcher = classes[which].launch[width % 4U != 0U][f32];
+            const m3_softmax_launcher launcher =
+                chosen->launch[width % 4U != 0U][f32];
 
             return m3_hip_launch(
                 device, "m3_softmax_rows_wide",

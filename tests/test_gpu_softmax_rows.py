@@ -129,3 +129,19 @@ def test_softmax_row_alignments(hip, width, dtypes):
                 [ViewSpec(0, dtypes[0], (rows, width)),
                  ViewSpec(0, dtypes[0], (rows, width))],
                 "rows in place %s w=%d" % (dtypes, width))
+
+
+@pytest.mark.parametrize("dtypes", [(m3.F32, m3.F32), (m3.BF16, m3.F32)])
+@pytest.mark.parametrize("width,rows", [
+    (257, 2049), (511, 2049), (513, 2049), (1021, 2049), (2049, 257),
+    (4097, 257), (8193, 300), (16385, 257)])
+def test_softmax_many_rows(hip, width, rows, dtypes):
+    """More rows than the layouts for a few rows take: the same widths in
+    the other layouts, with rows of every kind at every place of a wave."""
+    rng = np.random.default_rng(45000 + width)
+    source = elements(logits_of(rng, rows, width), dtypes[0])
+    out = np.zeros(rows * width * m3.DTYPE_SIZES[dtypes[1]], np.uint8)
+    compare(hip, [as_bytes(source), out],
+            [ViewSpec(0, dtypes[0], (rows, width)),
+             ViewSpec(1, dtypes[1], (rows, width))],
+            "many rows %s w=%d rows=%d" % (dtypes, width, rows))
