@@ -123,9 +123,8 @@ __device__ __forceinline__ uint32_t m3_operand_element(const m3_bin_operand &o,
     return m3_operand_at<DT>(o, m3_operand_index(o, f));
 }
 
-/* F32 bits of operand elements f..f+3 (f a multiple of 4). WHOLE: the
- * operand's mode is none of TRAIL_CUT, ROW_CUT and PERIODIC. */
-template <uint32_t DT, bool WHOLE = false>
+/* F32 bits of operand elements f..f+3 (f a multiple of 4). */
+template <uint32_t DT>
 __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
                                                   uint32_t f)
 {
@@ -138,14 +137,18 @@ __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
                                        o.period.divisor;
 
         /* a full operand is read once per launch: streamed; a trailing
-         * broadcast operand is reread by every row: cached */
+         * broadcast operand is reread by every row: cached, and written
+         * element by element (the compiler joins the accesses later): as
+         * one vector load it is merged with the streamed one above, which
+         * then is no longer nontemporal (x[8,1024,1536] * c[1536] 24.1
+         * against 17.7 us). */
         if (dtype == M3N_F32) {
             const uint8_t *p = o.base + (uint64_t)index * 4U;
 
             if (o.mode == M3_BIN_FULL) {
                 return m3_stream_load((const uint4 *)p);
             }
-            const m3_u32x4_any w = *(const m3_u32x4_any *)p;
+            const uint32_t *w = (const uint32_t *)p;
 
             return make_uint4(w[0], w[1], w[2], w[3]);
         }
@@ -155,13 +158,14 @@ __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
         if (o.mode == M3_BIN_FULL) {
             half = m3_stream_load((const uint2 *)p);
         } else {
-            const m3_u32x2_any h = *(const m3_u32x2_any *)p;
+            const uint16_t *h = (const uint16_t *)p;
 
-            half = make_uint2(h[0], h[1]);
+            half = make_uint2(h[0] | ((uint32_t)h[1] << 16U),
+                              h[2] | ((uint32_t)h[3] << 16U));
         }
         return m3_widen4_bits(half, dtype);
     }
-    if (WHOLE || o.mode == M3_BIN_SCALAR) {
+    if (o.mode == M3_BIN_SCALAR) {
         uint32_t v = m3_operand_element<DT>(o, f);
 
         return make_uint4(v, v, v, v);
@@ -285,6 +289,34 @@ constexpr uint32_t kHeldBlocksPerCu = 4U;
  * resident, 20-31 us). */
 constexpr double kBinaryHoldFactor = 1.1;
 
+/* F32 bits of operand elements f..f+3 for the held form: 16-byte aligned
+ * operands, every mode by its element indices. Its own function because
+ * twelve groups of two operands in flight are at the mercy of how the
+ * compiler lays out the choice of mode: with m3_operand_load4 it waits for
+ * each group's loads (x[8,1024,1536] * c[1536] 23.5 against 17.7 us). */
+__device__ __forceinline__ uint4 m3_held_load4(const m3_bin_operand &o,
+                                               uint32_t f)
+{
+    if (o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL) {
+        uint32_t index = o.mode == M3_BIN_FULL
+                             ? f
+                             : f - m3_fast_div_q(o.period, f) *
+                                       o.period.divisor;
+        const uint4 *p = (const uint4 *)(o.base + (uint64_t)index * 4U);
+
+        return o.mode == M3_BIN_FULL ? m3_stream_load(p) : *p;
+    }
+    if (o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR) {
+        uint32_t v = m3_operand_element<M3N_F32>(o, f);
+
+        return make_uint4(v, v, v, v);
+    }
+    return make_uint4(m3_operand_element<M3N_F32>(o, f),
+                      m3_operand_element<M3N_F32>(o, f + 1U),
+                      m3_operand_element<M3N_F32>(o, f + 2U),
+                      m3_operand_element<M3N_F32>(o, f + 3U));
+}
+
 /* The held form of the F32 vector kernel, for a launch whose workgroups
  * are all resident at once: each lane loads its kHeldGroups groups of both
  * operands, forms the results, and stores them only hold_ticks
@@ -308,8 +340,8 @@ __global__ __launch_bounds__(256) void m3_binary_held_kernel(
         const uint32_t g = first + (uint32_t)k * kThreads;
 
         if (g < a.groups) {
-            left[k] = m3_operand_load4<M3N_F32, true>(a.left, g * 4U);
-            right[k] = m3_operand_load4<M3N_F32, true>(a.right, g * 4U);
+            left[k] = m3_held_load4(a.left, g * 4U);
+            right[k] = m3_held_load4(a.right, g * 4U);
         } else {
             left[k] = make_uint4(0U, 0U, 0U, 0U);
             right[k] = left[k];
@@ -610,10 +642,12 @@ bool m3_classify_operand(const m3_index_plan &plan, uint32_t k,
     return true;
 }
 
-/* True for the modes that give a group one element or one vector. */
+/* True for an operand that gives a group one element or one 16-byte
+ * aligned vector. */
 bool m3_operand_whole(const m3_bin_operand &o)
 {
-    return o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL ||
+    return ((o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL) &&
+            ((uintptr_t)o.base & 15U) == 0U) ||
            o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR;
 }
 
