@@ -785,7 +785,7 @@ bool m3_chain_same_shape(const m3_hip_view *a, const m3_hip_view *b)
 
 /* Fills the kernel's arguments from a chain of binary operations and casts;
  * false when the chain kernel does not take it: an operand that does not
- * classify, more than 2^32 elements, or an output that overlaps what
+ * classify, no elements, 2^32 of them or more, or an output that overlaps what
  * another operation reads or writes (the launch would no longer equal the
  * operations in order). */
 bool m3_chain_plan(const m3_hip_chain_command *commands, uint32_t count,
@@ -793,6 +793,11 @@ bool m3_chain_plan(const m3_hip_chain_command *commands, uint32_t count,
 {
     const m3_hip_view *space = &commands[0].output;
 
+    /* before any divisor is formed from an extent: none of them is zero */
+    if (space->element_count == 0U ||
+        space->element_count >= (1ULL << 32U)) {
+        return false;
+    }
     for (uint32_t k = 0U; k < count; ++k) {
         const m3_hip_chain_command &c = commands[k];
         const bool cast = c.kind == M3_HIP_CHAIN_CAST;
@@ -847,8 +852,7 @@ bool m3_chain_plan(const m3_hip_chain_command *commands, uint32_t count,
     }
     args->count = (uint32_t)space->element_count;
     args->groups = args->count / 4U;
-    return space->element_count != 0U &&
-           space->element_count < (1ULL << 32U);
+    return true;
 }
 
 } // namespace

@@ -217,3 +217,25 @@ def test_snake1d_tanh(hip, shape):
           [(m3.OP_SNAKE1D, [x_view, a_view, ViewSpec(2, m3.F32, shape)]),
            (m3.OP_TANH, [ViewSpec(2, m3.F32, shape), x_view])],
           "snake1d, tanh over its input %s" % (shape,))
+
+
+@pytest.mark.parametrize("shape,dims", [((3, 0), (3, 1)), ((0, 4), (1, 4)),
+                                        ((2, 0, 5), (2, 1, 1)),
+                                        ((0, 3), (3,))])
+def test_lists_over_empty_tensors(hip, shape, dims):
+    """An empty run inside a list does nothing, and the commands around it
+    run."""
+    rng = np.random.default_rng(8)
+    empty = np.zeros(0, np.uint8)
+    other = values(rng, m3.F32, 16)
+    x, s = values(rng, m3.F32, 24), values(rng, m3.F32, 24)
+    arrays = [empty, other, empty.copy(), empty.copy(), x, s,
+              np.zeros(24, np.float32), np.zeros(24, np.float32)]
+    e = [ViewSpec(i, m3.F32, shape) for i in (0, 2, 3)]
+    o = ViewSpec(1, m3.F32, dims)
+    full = [ViewSpec(i, m3.F32, (24,)) for i in (4, 5, 6, 7)]
+    check(hip, arrays,
+          [(m3.OP_MUL, [full[0], full[1], full[2]]),
+           (m3.OP_MUL, [e[0], o, e[1]]), (m3.OP_ADD, [e[1], o, e[2]]),
+           (m3.OP_ADD, [full[2], full[1], full[3]])],
+          "empty %s %s" % (shape, dims))
