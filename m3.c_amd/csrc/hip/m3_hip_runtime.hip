@@ -9,6 +9,7 @@
  * (src/m3_backend_metal.m:189-216).
  */
 #include "m3_hip_internal.h"
+#include "m3_staging.h"
 
 #include <algorithm>
 #include <chrono>
@@ -705,31 +706,45 @@ static int m3_stage_copy(m3_hip_device *device, void *destination,
     return m3_hip_check(hipGetLastError(), "staged copy", message, capacity);
 }
 
-/* Queues the store of the stage's next sequence number. */
-static int m3_stage_mark(m3_hip_device *device, char *message,
-                         size_t capacity)
-{
-    hipLaunchKernelGGL(m3_done_kernel, dim3(1), dim3(64), 0, device->stream,
-                       device->stage.word, device->stage.sequence + 1U);
-    const int code = m3_hip_check(hipGetLastError(), "staged copy's mark",
-                                  message, capacity);
+/* The steps of a staged copy on the device's stream (m3_staging.h). */
+struct m3_stage_stream {
+    m3_hip_device *device;
+    char *message;
+    size_t capacity;
 
-    if (code == M3_HIP_OK) {
-        device->stage.sequence += 1U;
-    }
-    return code;
-}
+    int queue(uint8_t *destination, const uint8_t *source, size_t bytes,
+              uint32_t *sequence)
+    {
+        int code = m3_stage_copy(device, destination, source, bytes, message,
+                                 capacity);
 
-/* Waits for sequence number `sequence` of the stage. */
-static int m3_stage_wait(m3_hip_device *device, uint32_t sequence,
-                         char *message, size_t capacity)
-{
-    if (m3_hip_poll_word(device->stage.word, sequence)) {
-        return M3_HIP_OK;
+        if (code == M3_HIP_OK) {
+            hipLaunchKernelGGL(m3_done_kernel, dim3(1), dim3(64), 0,
+                               device->stream, device->stage.word,
+                               device->stage.sequence + 1U);
+            code = m3_hip_check(hipGetLastError(), "staged copy's mark",
+                                message, capacity);
+        }
+        if (code == M3_HIP_OK) {
+            *sequence = ++device->stage.sequence;
+        }
+        return code;
     }
-    return m3_hip_check(hipStreamSynchronize(device->stream),
-                        "hipStreamSynchronize", message, capacity);
-}
+
+    int wait(uint32_t sequence)
+    {
+        if (m3_hip_poll_word(device->stage.word, sequence)) {
+            return M3_HIP_OK;
+        }
+        return m3_hip_check(hipStreamSynchronize(device->stream),
+                            "hipStreamSynchronize", message, capacity);
+    }
+
+    bool drain()
+    {
+        return hipStreamSynchronize(device->stream) == hipSuccess;
+    }
+};
 
 /* The staging buffer of one direction and the completion word, allocated at
  * their first use; false when pinned memory is not to be had. */
@@ -760,6 +775,16 @@ static bool m3_stage_ready(m3_hip_device *device, uint8_t **buffer,
     return true;
 }
 
+/* What a staged copy returns; staging memory that queued work may still
+ * touch is not used again. */
+static int m3_stage_end(m3_hip_device *device, int code, bool reusable,
+                        char *message, size_t capacity)
+{
+    device->stage.unavailable = device->stage.unavailable || !reusable;
+    return code == M3_HIP_OK ? m3_hip_stream_errors(device, message, capacity)
+                             : code;
+}
+
 /* The host-to-device copy through the stage; *staged is false, with nothing
  * done, when it is not available. */
 static int m3_stage_upload(m3_hip_device *device, uint8_t *destination,
@@ -767,6 +792,8 @@ static int m3_stage_upload(m3_hip_device *device, uint8_t *destination,
                            char *message, size_t capacity)
 {
     const std::lock_guard<std::mutex> guard(device->stage.lock);
+    m3_stage_stream stream = {device, message, capacity};
+    bool reusable = false;
     int code;
 
     *staged = m3_stage_ready(device, &device->stage.up, kStageUpload);
@@ -774,18 +801,9 @@ static int m3_stage_upload(m3_hip_device *device, uint8_t *destination,
         return M3_HIP_OK;
     }
     device->host_waits += 1U;
-    std::memcpy(device->stage.up, source, bytes);
-    code = m3_stage_copy(device, destination, device->stage.up, bytes,
-                         message, capacity);
-    if (code == M3_HIP_OK) {
-        code = m3_stage_mark(device, message, capacity);
-    }
-    if (code == M3_HIP_OK) {
-        code = m3_stage_wait(device, device->stage.sequence, message,
-                             capacity);
-    }
-    return code == M3_HIP_OK ? m3_hip_stream_errors(device, message, capacity)
-                             : code;
+    code = m3_stage_write(stream, device->stage.up, destination, source,
+                          bytes, &reusable);
+    return m3_stage_end(device, code, reusable, message, capacity);
 }
 
 /* The device-to-host copy through the stage, as m3_stage_upload. */
@@ -794,36 +812,18 @@ static int m3_stage_download(m3_hip_device *device, uint8_t *destination,
                              bool *staged, char *message, size_t capacity)
 {
     const std::lock_guard<std::mutex> guard(device->stage.lock);
-    const size_t most = m3_stage_chunk(bytes);
-    uint32_t first;
-    int code = M3_HIP_OK;
+    m3_stage_stream stream = {device, message, capacity};
+    bool reusable = false;
+    int code;
 
     *staged = m3_stage_ready(device, &device->stage.down, kStageBytes);
     if (!*staged) {
         return M3_HIP_OK;
     }
     device->host_waits += 1U;
-    first = device->stage.sequence + 1U;
-    for (size_t done = 0U; code == M3_HIP_OK && done < bytes;
-         done += most) {
-        code = m3_stage_copy(device, device->stage.down + done, source + done,
-                             std::min(bytes - done, most), message,
-                             capacity);
-        if (code == M3_HIP_OK) {
-            code = m3_stage_mark(device, message, capacity);
-        }
-    }
-    for (size_t done = 0U; code == M3_HIP_OK && done < bytes;
-         done += most) {
-        code = m3_stage_wait(device, first + (uint32_t)(done / most),
-                             message, capacity);
-        if (code == M3_HIP_OK) {
-            std::memcpy(destination + done, device->stage.down + done,
-                        std::min(bytes - done, most));
-        }
-    }
-    return code == M3_HIP_OK ? m3_hip_stream_errors(device, message, capacity)
-                             : code;
+    code = m3_stage_read(stream, device->stage.down, destination, source,
+                         bytes, m3_stage_chunk(bytes), &reusable);
+    return m3_stage_end(device, code, reusable, message, capacity);
 }
 
 extern "C" int m3_hip_copy_h2d(m3_hip_device *device,
