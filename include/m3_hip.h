@@ -58,7 +58,9 @@
  *
  * All launches of one device go to that device's single HIP stream, in call
  * order, so a command list executes in order and m3_hip_synchronize waits
- * for all of it. A device handle is not thread-safe.
+ * for all of it. A device handle is not thread-safe, but for m3_hip_copy_h2d
+ * and m3_hip_copy_d2h: with timing off, several threads may copy through one
+ * handle at once (no other call on it running beside them).
  */
 #ifndef M3_HIP_H
 #define M3_HIP_H

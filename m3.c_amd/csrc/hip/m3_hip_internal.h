@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -124,16 +125,16 @@ struct m3_hip_device {
     uint32_t fused_epoch;
     uint32_t fused_kind;
     /* how many times the host has waited for the stream (synchronize,
-     * scan readback, blocking copies) since the device was opened */
-    uint64_t host_waits;
+     * scan readback, blocking copies) since the device was opened; atomic,
+     * as `polls`, because copies may run on several threads at once */
+    std::atomic<uint64_t> host_waits;
     /* the device address of the static scan scratch (m3_hip_runtime.hip) */
     uint32_t *static_scratch;
     /* completion word in coherent pinned host memory (may be null) and the
      * last sequence number a kernel was queued to store there */
     uint32_t *done_word;
     uint32_t done_sequence;
-    uint32_t unchecked_polls; /* polled completions since the last query
-                               * of the stream's error state */
+    std::atomic<uint32_t> polls; /* completions seen by polling a word */
     /* pinned staging of host copies (m3_hip_runtime.hip), taken at the first
      * copy in its direction and given back when the device closes; `lock`
      * guards all of it, so that threads may copy through one device */

@@ -415,13 +415,19 @@ extern "C" void m3_hip_device_close(m3_hip_device *device)
     delete device;
 }
 
+/* One more wait of the host for the stream. */
+static void m3_hip_count_wait(m3_hip_device *device)
+{
+    device->host_waits.fetch_add(1U, std::memory_order_relaxed);
+}
+
 extern "C" int m3_hip_host_waits(const m3_hip_device *device,
                                  uint64_t *waits)
 {
     if (device == nullptr || waits == nullptr) {
         return M3_HIP_INVALID;
     }
-    *waits = device->host_waits;
+    *waits = device->host_waits.load(std::memory_order_relaxed);
     return M3_HIP_OK;
 }
 
@@ -612,18 +618,21 @@ constexpr uint32_t kPollsPerErrorQuery = 64U;
 /* After a completion seen through the completion word: every
  * kPollsPerErrorQuery of them, an error the stream has recorded (a
  * kernel fault, say) is reported; not ready (the runtime has not retired
- * the work yet) is no error. Storage reads, frees and destroy wait on the
- * stream itself, which reports such errors too. */
+ * the work yet) is no error. The word itself is stored by a kernel behind
+ * the work: after a kernel that faulted it does not arrive, and the wait on
+ * the stream that follows the bounded poll reports the fault at once.
+ * Copies the runtime makes, frees and destroy wait on the stream itself;
+ * staged copies and runs come through here. */
 static int m3_hip_stream_errors(m3_hip_device *device, char *message,
                                 size_t capacity)
 {
     hipError_t state;
 
-    device->unchecked_polls += 1U;
-    if (device->unchecked_polls < kPollsPerErrorQuery) {
+    if ((device->polls.fetch_add(1U, std::memory_order_relaxed) + 1U) %
+            kPollsPerErrorQuery !=
+        0U) {
         return M3_HIP_OK;
     }
-    device->unchecked_polls = 0U;
     state = hipStreamQuery(device->stream);
     if (state == hipSuccess || state == hipErrorNotReady) {
         return M3_HIP_OK;
@@ -800,7 +809,7 @@ static int m3_stage_upload(m3_hip_device *device, uint8_t *destination,
     if (!*staged) {
         return M3_HIP_OK;
     }
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     code = m3_stage_write(stream, device->stage.up, destination, source,
                           bytes, &reusable);
     return m3_stage_end(device, code, reusable, message, capacity);
@@ -820,7 +829,7 @@ static int m3_stage_download(m3_hip_device *device, uint8_t *destination,
     if (!*staged) {
         return M3_HIP_OK;
     }
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     code = m3_stage_read(stream, device->stage.down, destination, source,
                          bytes, m3_stage_chunk(bytes), &reusable);
     return m3_stage_end(device, code, reusable, message, capacity);
@@ -873,7 +882,7 @@ extern "C" int m3_hip_copy_h2d(m3_hip_device *device,
                                        byte_count, hipMemcpyHostToDevice,
                                        device->stream),
                         "hipMemcpyAsync(host to device)", message, capacity);
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     if (code == M3_HIP_OK) {
         code = m3_hip_check(hipStreamSynchronize(device->stream),
                             "hipStreamSynchronize", message, capacity);
@@ -912,7 +921,7 @@ extern "C" int m3_hip_copy_d2h(m3_hip_device *device, void *host_destination,
                                        byte_count, hipMemcpyDeviceToHost,
                                        device->stream),
                         "hipMemcpyAsync(device to host)", message, capacity);
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     if (code == M3_HIP_OK) {
         code = m3_hip_check(hipStreamSynchronize(device->stream),
                             "hipStreamSynchronize", message, capacity);
@@ -937,7 +946,7 @@ extern "C" int m3_hip_synchronize(m3_hip_device *device, char *message,
      * next launch, and the timing events of the next launch read the
      * kernel's own duration (they read about 2 us long when the runtime
      * has not yet retired the previous work). */
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     if (device->done_word != nullptr && !device->timing) {
         const uint32_t sequence = device->done_sequence + 1U;
 
@@ -1237,7 +1246,7 @@ static int m3_hip_scan_wait(m3_hip_device *device, uint32_t sequence,
 {
     int code;
 
-    device->host_waits += 1U;
+    m3_hip_count_wait(device);
     if (device->done_word != nullptr && !device->timing &&
         m3_hip_poll_word(device->done_word, sequence)) {
         code = m3_hip_stream_errors(device, message, capacity);

@@ -34,6 +34,8 @@ class Device:
         message = ctypes.create_string_buffer(256)
         assert self.hip.m3_hip_device_open(0, ctypes.byref(self.device),
                                            message, 256) == 0
+        self.hip.m3_hip_host_waits.argtypes = [
+            vp, ctypes.POINTER(ctypes.c_uint64)]
         assert self.hip.m3_hip_arena_reserve(
             self.device, arena_bytes, ctypes.byref(self.base), message,
             256) == 0
@@ -51,6 +53,12 @@ class Device:
             self.device, out.ctypes.data, self.base.value + offset, count,
             message, 256) == 0, message.value
         return out
+
+    def host_waits(self):
+        waits = ctypes.c_uint64(0)
+        assert self.hip.m3_hip_host_waits(self.device,
+                                          ctypes.byref(waits)) == 0
+        return waits.value
 
     def close(self):
         self.hip.m3_hip_arena_release(self.device, self.base)
@@ -99,6 +107,7 @@ def test_many_writes_in_order(device):
 
 def test_threads_copy_through_one_device(device):
     failures = []
+    before = device.host_waits()
 
     def work(index):
         rng = np.random.default_rng(index)
@@ -116,3 +125,5 @@ def test_threads_copy_through_one_device(device):
     for thread in threads:
         thread.join()
     assert not failures
+    # every copy of more than 256 bytes waits once, and every wait is counted
+    assert device.host_waits() - before == 4 * 40 * 2
