@@ -17,7 +17,6 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
-#include <mutex>
 #include <vector>
 
 /* One timed launch: events recorded around a kernel on the device stream. */
@@ -135,17 +134,6 @@ struct m3_hip_device {
     uint32_t *done_word;
     uint32_t done_sequence;
     std::atomic<uint32_t> polls; /* completions seen by polling a word */
-    /* pinned staging of host copies (m3_hip_runtime.hip), taken at the first
-     * copy in its direction and given back when the device closes; `lock`
-     * guards all of it, so that threads may copy through one device */
-    struct {
-        std::mutex lock;
-        uint8_t *up;       /* host to device */
-        uint8_t *down;     /* device to host */
-        uint32_t *word;    /* completion word of the staged copies */
-        uint32_t sequence; /* the last number queued to be stored there */
-        bool unavailable;  /* an allocation failed: copies go unstaged */
-    } stage;
     bool timing;
     /* timing mode 1 attaches events to every launch; mode 2 only retires
      * each run on the stream, as mode 1 does, so that an external profiler

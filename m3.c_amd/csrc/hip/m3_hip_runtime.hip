@@ -211,6 +211,11 @@ static void *m3_scratch_address[kScratchOrdinals];
 /* one m3_hip_scan_views_static call at a time per device */
 static m3_scratch_guard<kScratchOrdinals> m3_scratch_in_use;
 
+/* Pinned staging memory of host copies: copies through one GPU at once that
+ * each find a set of their own. */
+constexpr int kStageSets = 4;
+static m3_stage_pool<kScratchOrdinals, kStageSets> m3_stage_memory;
+
 /* Device and pinned host allocations made by this library, counted so that
  * tests can show an entry point allocates nothing. */
 static std::atomic<uint64_t> m3_allocations{0};
@@ -341,6 +346,7 @@ extern "C" int m3_hip_device_open(int ordinal, m3_hip_device **device_output,
                 ? (uint32_t)std::strtoul(wide, nullptr, 10)
                 : 0U;
     }
+    m3_stage_memory.open(ordinal); /* m3_hip_device_close is its end */
     code = m3_hip_check(hipStreamCreateWithFlags(&device->stream,
                                                  hipStreamNonBlocking),
                         "hipStreamCreateWithFlags", message, capacity);
@@ -403,12 +409,8 @@ extern "C" void m3_hip_device_close(m3_hip_device *device)
     if (device->done_word != nullptr) {
         (void)hipHostFree(device->done_word);
     }
-    for (void *pinned : {(void *)device->stage.up, (void *)device->stage.down,
-                         (void *)device->stage.word}) {
-        if (pinned != nullptr) {
-            (void)hipHostFree(pinned);
-        }
-    }
+    m3_stage_memory.close(device->ordinal,
+                          [](uint8_t *memory) { (void)hipHostFree(memory); });
     if (device->stream != nullptr) {
         (void)hipStreamDestroy(device->stream);
     }
@@ -650,12 +652,17 @@ static int m3_hip_stream_errors(m3_hip_device *device, char *message,
  * stores a sequence number into a pinned completion word, which the host
  * polls:
  *   - host to device (up to kStageUpload): the bytes are copied into the
- *     staging buffer, and the call returns once the device has them;
- *   - device to host (up to 256 KB, and from 1 MB to kStageBytes): the host
- *     copies a chunk out while the next one arrives.
- * Both directions take the device's stage lock, so that several threads may
- * copy through one device, as with the runtime's own copies. With timing on,
- * without pinned memory, and for larger copies the runtime's copy is used.
+ *     staging memory, and the call returns once the device has them;
+ *   - device to host (up to 256 KB, and from 1 MB to kStageDownload): the
+ *     host copies a chunk out while the next one arrives.
+ * The pinned memory is the process's (m3_stage_pool): a few sets per GPU,
+ * each lent to one copy at a time, so that a session neither allocates nor
+ * frees any. A session of [16,1,1501] scores, created, used once and closed,
+ * with the runtime's copies: 77, 98 and 81 us; with staging memory of each
+ * handle's own, taken at its first copies: 105, 105 and 200; with the
+ * process's: 77, 80 and 140 (what the runtime's copies retire of the stream
+ * as they wait is retired at the end here). With timing on, without pinned
+ * memory, and for larger copies the runtime's copy is used.
  * Measured behind a queued kernel, the runtime's copy against the staged
  * one: writes 4 KB 15.8 and 12.6 us, 96 KB 21.8 and 16.4, 192 KB 23.4 and
  * 21.3, 320 KB 26.5 and 27.7, 1 MB 64 and 71; reads 4 KB 22.6 and 11.7, 96
@@ -663,8 +670,13 @@ static int m3_hip_stream_errors(m3_hip_device *device, char *message,
  * A session's read of 512 KB, behind no queued kernel, was 10 us slower
  * staged, so reads between 256 KB and 1 MB stay with the runtime.
  */
-constexpr size_t kStageBytes = 4U << 20U; /* staging memory for reads */
-constexpr size_t kStageUpload = 192U << 10U; /* and for writes */
+constexpr size_t kStageDownload = 4U << 20U; /* the largest staged read */
+constexpr size_t kStageUpload = 192U << 10U; /* and write */
+constexpr size_t kStageMost = 512U << 10U; /* bytes of a read's chunk */
+/* a set: the completion word, the bytes of a write, the chunks of a read */
+constexpr size_t kStageUp = 4096U;
+constexpr size_t kStageDown = kStageUp + kStageUpload;
+constexpr size_t kStageSetBytes = kStageDown + kStageChunks * kStageMost;
 
 /* The chunk a read moves at a time: half of it, so that the host's copy of
  * one half and the device's of the other overlap, but at least 256 KB (a
@@ -674,8 +686,7 @@ static size_t m3_stage_chunk(size_t bytes)
 {
     const size_t half = (bytes / 2U + 4095U) & ~(size_t)4095U;
 
-    return std::max((size_t)256U << 10U,
-                    std::min((size_t)512U << 10U, half));
+    return std::max((size_t)256U << 10U, std::min(kStageMost, half));
 }
 
 /* Copies `bytes` bytes between device and pinned host memory, 16 bytes per
@@ -718,6 +729,7 @@ static int m3_stage_copy(m3_hip_device *device, void *destination,
 /* The steps of a staged copy on the device's stream (m3_staging.h). */
 struct m3_stage_stream {
     m3_hip_device *device;
+    m3_stage_set *set;
     char *message;
     size_t capacity;
 
@@ -729,20 +741,20 @@ struct m3_stage_stream {
 
         if (code == M3_HIP_OK) {
             hipLaunchKernelGGL(m3_done_kernel, dim3(1), dim3(64), 0,
-                               device->stream, device->stage.word,
-                               device->stage.sequence + 1U);
+                               device->stream, word(),
+                               set->sequence + 1U);
             code = m3_hip_check(hipGetLastError(), "staged copy's mark",
                                 message, capacity);
         }
         if (code == M3_HIP_OK) {
-            *sequence = ++device->stage.sequence;
+            *sequence = ++set->sequence;
         }
         return code;
     }
 
     int wait(uint32_t sequence)
     {
-        if (m3_hip_poll_word(device->stage.word, sequence)) {
+        if (m3_hip_poll_word(word(), sequence)) {
             return M3_HIP_OK;
         }
         return m3_hip_check(hipStreamSynchronize(device->stream),
@@ -753,86 +765,68 @@ struct m3_stage_stream {
     {
         return hipStreamSynchronize(device->stream) == hipSuccess;
     }
+
+    uint32_t *word() const
+    {
+        return (uint32_t *)set->memory;
+    }
 };
 
-/* The staging buffer of one direction and the completion word, allocated at
- * their first use; false when pinned memory is not to be had. */
-static bool m3_stage_ready(m3_hip_device *device, uint8_t **buffer,
-                           size_t bytes)
+/* A set's memory, its completion word zero; null when pinned memory is not
+ * to be had. */
+static uint8_t *m3_stage_allocate(int ordinal)
 {
-    if (device->stage.unavailable) {
-        return false;
+    void *memory = nullptr;
+    int current = ordinal;
+
+    (void)hipGetDevice(&current);
+    if (current != ordinal) {
+        (void)hipSetDevice(ordinal);
     }
-    if (device->stage.word == nullptr) {
-        if (m3_hip_host_malloc((void **)&device->stage.word, 64U,
-                               hipHostMallocCoherent) != (int)hipSuccess) {
-            device->stage.word = nullptr;
-        } else {
-            __atomic_store_n(device->stage.word, 0U, __ATOMIC_RELEASE);
-        }
-    }
-    if (device->stage.word != nullptr && *buffer == nullptr &&
-        m3_hip_host_malloc((void **)buffer, bytes,
-                           hipHostMallocCoherent) != (int)hipSuccess) {
-        *buffer = nullptr;
-    }
-    if (device->stage.word == nullptr || *buffer == nullptr) {
+    if (m3_hip_host_malloc(&memory, kStageSetBytes, hipHostMallocCoherent) !=
+        (int)hipSuccess) {
         (void)hipGetLastError();
-        device->stage.unavailable = true;
-        return false;
+        memory = nullptr;
+    } else {
+        __atomic_store_n((uint32_t *)memory, 0U, __ATOMIC_RELEASE);
     }
-    return true;
+    if (current != ordinal) {
+        (void)hipSetDevice(current);
+    }
+    return (uint8_t *)memory;
 }
 
-/* What a staged copy returns; staging memory that queued work may still
- * touch is not used again. */
-static int m3_stage_end(m3_hip_device *device, int code, bool reusable,
-                        char *message, size_t capacity)
+/* A copy through the staging memory, in either direction; *staged is false,
+ * with nothing done, when no set is to be had. */
+static int m3_stage_transfer(m3_hip_device *device, bool down,
+                             void *destination, const void *source,
+                             size_t bytes, bool *staged, char *message,
+                             size_t capacity)
 {
-    device->stage.unavailable = device->stage.unavailable || !reusable;
+    m3_stage_set *set = m3_stage_memory.take(device->ordinal, [&]() {
+        return m3_stage_allocate(device->ordinal);
+    });
+    m3_stage_stream stream = {device, set, message, capacity};
+    bool reusable = false;
+    int code;
+
+    *staged = set != nullptr;
+    if (set == nullptr) {
+        return M3_HIP_OK;
+    }
+    m3_hip_count_wait(device);
+    if (down) {
+        code = m3_stage_read(stream, set->memory + kStageDown,
+                             (uint8_t *)destination, (const uint8_t *)source,
+                             bytes, m3_stage_chunk(bytes), &reusable);
+    } else {
+        code = m3_stage_write(stream, set->memory + kStageUp,
+                              (uint8_t *)destination, (const uint8_t *)source,
+                              bytes, &reusable);
+    }
+    m3_stage_memory.give(device->ordinal, set, reusable);
     return code == M3_HIP_OK ? m3_hip_stream_errors(device, message, capacity)
                              : code;
-}
-
-/* The host-to-device copy through the stage; *staged is false, with nothing
- * done, when it is not available. */
-static int m3_stage_upload(m3_hip_device *device, uint8_t *destination,
-                           const uint8_t *source, size_t bytes, bool *staged,
-                           char *message, size_t capacity)
-{
-    const std::lock_guard<std::mutex> guard(device->stage.lock);
-    m3_stage_stream stream = {device, message, capacity};
-    bool reusable = false;
-    int code;
-
-    *staged = m3_stage_ready(device, &device->stage.up, kStageUpload);
-    if (!*staged) {
-        return M3_HIP_OK;
-    }
-    m3_hip_count_wait(device);
-    code = m3_stage_write(stream, device->stage.up, destination, source,
-                          bytes, &reusable);
-    return m3_stage_end(device, code, reusable, message, capacity);
-}
-
-/* The device-to-host copy through the stage, as m3_stage_upload. */
-static int m3_stage_download(m3_hip_device *device, uint8_t *destination,
-                             const uint8_t *source, size_t bytes,
-                             bool *staged, char *message, size_t capacity)
-{
-    const std::lock_guard<std::mutex> guard(device->stage.lock);
-    m3_stage_stream stream = {device, message, capacity};
-    bool reusable = false;
-    int code;
-
-    *staged = m3_stage_ready(device, &device->stage.down, kStageBytes);
-    if (!*staged) {
-        return M3_HIP_OK;
-    }
-    m3_hip_count_wait(device);
-    code = m3_stage_read(stream, device->stage.down, destination, source,
-                         bytes, m3_stage_chunk(bytes), &reusable);
-    return m3_stage_end(device, code, reusable, message, capacity);
 }
 
 extern "C" int m3_hip_copy_h2d(m3_hip_device *device,
@@ -870,9 +864,9 @@ extern "C" int m3_hip_copy_h2d(m3_hip_device *device,
     if (byte_count <= kStageUpload && !device->timing) {
         bool staged = false;
 
-        code = m3_stage_upload(device, (uint8_t *)device_destination,
-                               (const uint8_t *)host_source, byte_count,
-                               &staged, message, capacity);
+        code = m3_stage_transfer(device, false, device_destination,
+                                 host_source, byte_count, &staged, message,
+                                 capacity);
         if (staged) {
             return code;
         }
@@ -906,13 +900,13 @@ extern "C" int m3_hip_copy_d2h(m3_hip_device *device, void *host_destination,
         return M3_HIP_OK;
     }
     if ((byte_count <= (256U << 10U) ||
-         (byte_count >= (1U << 20U) && byte_count <= kStageBytes)) &&
+         (byte_count >= (1U << 20U) && byte_count <= kStageDownload)) &&
         !device->timing) {
         bool staged = false;
 
-        code = m3_stage_download(device, (uint8_t *)host_destination,
-                                 (const uint8_t *)device_source, byte_count,
-                                 &staged, message, capacity);
+        code = m3_stage_transfer(device, true, host_destination,
+                                 device_source, byte_count, &staged, message,
+                                 capacity);
         if (staged) {
             return code;
         }

@@ -6,6 +6,9 @@ with timing on, take other paths. Sizes at the edges of the paths and chunks, at
 any byte offset, and from several threads over one device.
 """
 import ctypes
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -103,6 +106,80 @@ def test_many_writes_in_order(device):
         data[:] = 77  # the caller's buffer is free when the call returns
         expected[offset:offset + count] = k & 255
     assert np.array_equal(device.read(0, 2 * MIB), expected)
+
+
+def allocations():
+    _, hip = m3.load()
+    count = ctypes.c_uint64(0)
+    hip.m3_hip_allocation_count.argtypes = [ctypes.POINTER(ctypes.c_uint64)]
+    assert hip.m3_hip_allocation_count(ctypes.byref(count)) == 0
+    return count.value
+
+
+def test_handles_share_staging_memory(gpu):
+    """Handles opened, used and closed in turn, and several open at once:
+    after the first copies of the process no copy allocates, and closing one
+    handle leaves the others' copies whole."""
+    rng = np.random.default_rng(11)
+    data = rng.integers(0, 256, 4 * MIB, np.uint8)
+
+    def use(opened):
+        for count in (1000, 96 * KIB, 192 * KIB):
+            opened.write(16, data[:count])
+            assert np.array_equal(opened.read(16, count), data[:count])
+        opened.write(0, data[:2 * MIB])
+        assert np.array_equal(opened.read(0, 2 * MIB), data[:2 * MIB])
+
+    first = Device(5 * MIB)
+    use(first)
+    first.close()
+    opened = Device(5 * MIB)
+    before = allocations()
+    use(opened)
+    assert allocations() == before
+    several = [Device(5 * MIB) for _ in range(6)]
+    before = allocations()
+    for one in several + [opened]:
+        use(one)
+    assert allocations() == before
+    while several:
+        several.pop(0).close()
+        for one in several + [opened]:
+            use(one)
+    assert allocations() == before
+    opened.close()
+
+
+def test_staging_is_taken(gpu):
+    """In a process of its own: the copies meant for the staging memory take
+    it (one allocation, at the first of them), and the others do not."""
+    code = """
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+import test_gpu_staging as t
+device = t.Device(5 * t.MIB)
+def made(call):
+    before = t.allocations()
+    call()
+    return t.allocations() - before
+zeros = np.zeros(4 * t.MIB + 1, np.uint8)
+assert made(lambda: device.write(0, zeros[:256])) == 0
+assert made(lambda: device.write(0, zeros[:192 * t.KIB + 1])) == 0
+assert made(lambda: device.read(0, 4 * t.MIB + 1)) == 0
+assert made(lambda: device.read(0, 512 * t.KIB)) == 0
+assert made(lambda: device.%s) == 1
+assert made(lambda: device.write(0, zeros[:192 * t.KIB])) == 0
+assert made(lambda: device.read(0, 4 * t.MIB)) == 0
+device.close()
+print("taken")
+"""
+    here = os.path.dirname(os.path.abspath(__file__))
+    for first in ("read(0, 1)", "write(0, zeros[:257])", "read(0, t.MIB)"):
+        result = subprocess.run([sys.executable, "-c", code % (here, first)],
+                                capture_output=True, text=True, timeout=100)
+        assert result.returncode == 0, result.stderr
+        assert "taken" in result.stdout
 
 
 def test_threads_copy_through_one_device(device):
