@@ -76,9 +76,9 @@ def device(gpu):
 
 
 @pytest.mark.parametrize("count", [
-    1, 255, 256, 257, 1000, 4096, 192 * KIB, 192 * KIB + 1, 256 * KIB - 1, 256 * KIB, 256 * KIB + 1,
+    1, 8, 15, 16, 17, 31, 255, 256, 257, 1000, 4096, 192 * KIB, 192 * KIB + 1, 256 * KIB - 1, 256 * KIB, 256 * KIB + 1,
     512 * KIB, 512 * KIB + 4, 700001, MIB - 65, MIB - 1, MIB, 3 * MIB + 7, 4 * MIB, 4 * MIB + 1])
-@pytest.mark.parametrize("offset", [0, 1, 2, 4, 6])
+@pytest.mark.parametrize("offset", [0, 1, 2, 4, 6, 8, 15])
 def test_copy_sizes(device, count, offset):
     rng = np.random.default_rng(count + offset)
     room = count + 64
