@@ -146,9 +146,10 @@ void m3_hip_arena_release(m3_hip_device *device, void *base);
  * (h2d) or holds the data (d2h). A host-to-device copy of at most 256
  * bytes (a scalar the host rewrites between commands) travels in a
  * kernel's arguments and does not wait for the stream; a larger one waits
- * for the copy to complete. Copies of at most 192 KiB to the device, and of
- * at most 256 KiB or 1 to 4 MiB from it, go through its pinned staging
- * memory. */
+ * for the copy to complete. Copies of up to 128 KiB to the device, and of
+ * up to 256 KiB or 1 to 4 MiB from it, may go through pinned staging memory
+ * that the handles of a process share (up to four sets of 1.2 MiB per
+ * GPU). */
 int m3_hip_copy_h2d(m3_hip_device *device, void *device_destination,
                     const void *host_source, size_t byte_count,
                     char *message, size_t capacity);

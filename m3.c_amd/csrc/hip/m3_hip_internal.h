@@ -134,6 +134,9 @@ struct m3_hip_device {
     uint32_t *done_word;
     uint32_t done_sequence;
     std::atomic<uint32_t> polls; /* completions seen by polling a word */
+    /* how many staged copies of middle sizes came last on the stream, or
+     * kStageRow behind a copy of the runtime's (m3_stage_wanted) */
+    std::atomic<uint32_t> stage_row;
     bool timing;
     /* timing mode 1 attaches events to every launch; mode 2 only retires
      * each run on the stream, as mode 1 does, so that an external profiler
@@ -198,6 +201,7 @@ int m3_hip_launch(m3_hip_device *device, const char *name, Launch launch,
         return m3_hip_fail(message, capacity, code,
                            "cannot take timing events for %s", name);
     }
+    device->stage_row.store(0U, std::memory_order_relaxed);
     launch(slot.start, slot.stop);
     hipError_t status = hipGetLastError();
     m3_hip_time_end(device, &slot);

@@ -644,17 +644,15 @@ static int m3_hip_stream_errors(m3_hip_device *device, char *message,
 
 /* ---- staged copies ----------------------------------------------------------
  *
- * Host buffers are pageable, and a copy between one and the device
- * (hipMemcpyAsync, then a wait for the stream) takes several times as long
- * as one from pinned memory (46 against 10 us for 96 KB, 61 against 26 for
- * 1 MB, on an idle stream). Short copies go through pinned memory instead, moved
- * by a kernel on the device's stream, chunk by chunk; a kernel after it
- * stores a sequence number into a pinned completion word, which the host
- * polls:
- *   - host to device (up to kStageUpload): the bytes are copied into the
- *     staging memory, and the call returns once the device has them;
- *   - device to host (up to 256 KB, and from 1 MB to kStageDownload): the
- *     host copies a chunk out while the next one arrives.
+ * Host buffers are pageable. The runtime copies between one and the device
+ * with a copy engine, which has to be handed the stream by the kernels
+ * before it and to hand it back. Short copies go through pinned memory
+ * instead, moved by a kernel on the device's stream, which stores a sequence
+ * number into a pinned completion word that the host polls:
+ *   - host to device: the bytes are copied into the staging memory, and the
+ *     call returns once the device has them;
+ *   - device to host: in chunks, the host copies one out while the next one
+ *     arrives.
  * The pinned memory is the process's (m3_stage_pool): a few sets per GPU,
  * each lent to one copy at a time, so that a session neither allocates nor
  * frees any. A session of [16,1,1501] scores, created, used once and closed,
@@ -662,23 +660,67 @@ static int m3_hip_stream_errors(m3_hip_device *device, char *message,
  * handle's own, taken at its first copies: 105, 105 and 200; with the
  * process's: 77, 80 and 140 (what the runtime's copies retire of the stream
  * as they wait is retired at the end here). With timing on, without pinned
- * memory, and for larger copies the runtime's copy is used.
- * Measured behind a queued kernel, the runtime's copy against the staged
- * one: writes 4 KB 15.8 and 12.6 us, 96 KB 21.8 and 16.4, 192 KB 23.4 and
- * 21.3, 320 KB 26.5 and 27.7, 1 MB 64 and 71; reads 4 KB 22.6 and 11.7, 96
- * KB 24.6 and 15.7, 256 KB 31.4 and 24.6, 1 MB 78 and 61, 4 MB 242 and 185.
- * A session's read of 512 KB, behind no queued kernel, was 10 us slower
- * staged, so reads between 256 KB and 1 MB stay with the runtime.
+ * memory, and for other sizes (m3_stage_wanted) the runtime's copy is used.
  */
 constexpr size_t kStageDownload = 4U << 20U; /* the largest staged read */
-constexpr size_t kStageUpload = 192U << 10U; /* and write */
-constexpr size_t kStageMost = 512U << 10U; /* bytes of a read's chunk */
+constexpr size_t kStageUpload = 128U << 10U; /* and write */
+constexpr size_t kStageLeast = 256U << 10U; /* bytes of a read's chunk */
+constexpr size_t kStageMost = 512U << 10U;
 /* a set: the completion word, the bytes of a write, the chunks of a read,
  * with room for up to 15 bytes before the first of either (m3_stage_phase) */
 constexpr size_t kStageUp = 4096U;
 constexpr size_t kStageDown = kStageUp + kStageUpload + 4096U;
 constexpr size_t kStageSetBytes =
     kStageDown + kStageChunks * kStageMost + 4096U;
+
+/* Whether a copy goes through the staging memory. What it competes with:
+ * the runtime copies at most 16 KB with a kernel and more with a copy
+ * engine, from or to the caller's own pages. Changing between kernels and
+ * the copy engine costs the stream about 10 us, and behind a copy of its own
+ * the engine is the faster one: us for one write behind a kernel, and for
+ * each of many behind each other, the runtime's against the staged:
+ *     16 KB   20 and 13.9     18 and 10.1
+ *     64 KB   29 and 10.8     20 and 11.6
+ *    128 KB   30 and 12.1     23 and 14.5
+ *    192 KB   31 and 13.6     25 and 17.6
+ * (reads: 16 KB 27 and 21.4 against 18 and 10.5, 64 KB 31 and 11.7 against
+ * 21 and 11.7, 256 KB 39 and 19.6 against 31 and 22.9). So the first few
+ * between two runs gain, and the others lose less than that up to about
+ * six; a program that only copies (loading weights) is better off with the
+ * engine. Hence:
+ *   - at most kStageSmall bytes: always;
+ *   - writes up to kStageUpload and reads up to 256 KB: unless the copy
+ *     before was the runtime's, or kStageRow such copies went before with no
+ *     launch between (12 writes of 96 KB and a read behind a run take 170 us
+ *     staged, 165 with the engine and 195 when it changes after 8; a row of
+ *     40 writes of 128 KB 637 us staged, 496 with the engine and 549 when it
+ *     changes after 16);
+ *   - reads of 1 MB up to kStageDownload: always (1 MB behind a kernel 64 us
+ *     against 75 and in a row 58 against 50 to 61, 4 MB 187 against 238 and
+ *     179 against 217 to 240);
+ *   - other sizes: never. A read of 512 KB behind a run would be 8 us
+ *     faster, and the second and later ones slower by as much; a write of
+ *     192 KB 6 us faster, and each behind another 4 us slower. */
+constexpr size_t kStageSmall = 32U << 10U;
+constexpr uint32_t kStageRow = 16U;
+
+static bool m3_stage_wanted(m3_hip_device *device, size_t bytes, bool down)
+{
+    const uint32_t row = device->stage_row.load(std::memory_order_relaxed);
+    const bool always = bytes <= kStageSmall ||
+                        (down && bytes >= (1U << 20U) &&
+                         bytes <= kStageDownload);
+    const bool wanted =
+        always || (row < kStageRow &&
+                   bytes <= (down ? (size_t)256U << 10U : kStageUpload));
+
+    if (device->timing) {
+        return false;
+    }
+    device->stage_row.store(always ? 0U : wanted ? row + 1U : kStageRow,
+                            std::memory_order_relaxed);
+    return wanted;
+}
 
 /* The chunk a read moves at a time: half of it, so that the host's copy of
  * one half and the device's of the other overlap, but at least 256 KB (a
@@ -688,19 +730,27 @@ static size_t m3_stage_chunk(size_t bytes)
 {
     const size_t half = (bytes / 2U + 4095U) & ~(size_t)4095U;
 
-    return std::max((size_t)256U << 10U, std::min(kStageMost, half));
+    return std::max(kStageLeast, std::min(kStageMost, half));
 }
+
+/* Workgroups of a set's copy that have ended (zero between copies): each
+ * GPU holds its own, and the last workgroup announces the copy. */
+static __device__ uint32_t m3_stage_arrived[kStageSets];
 
 /* Copies `bytes` bytes between device and pinned host memory that lie alike
  * within 16 bytes: single bytes up to the first multiple of 16 (`head` of
  * them) and after the last, 16 bytes per lane between. (Byte by byte for an
  * odd address, a write of 64 KB took 26.7 us against 13.2 for an even one,
- * and the runtime's copy 10.7.) Each wave's stores are visible to the host
- * when it ends (system-scope fence), so a kernel after this one on the
- * stream may announce them. */
+ * and the runtime's copy 10.7.) Every wave makes its stores visible to the
+ * host (and, through the host, to other streams) before it ends. With a
+ * `word`, the workgroup that ends last stores `sequence` there; else a
+ * kernel behind this one does. The former takes 1 us less for one copy (4 KB
+ * read 9.5 against 10.7 us, 128 KB 15.4 against 16.0), the latter 5 less for
+ * chunks that follow each other (4 MB 177 against 182). */
 __global__ __launch_bounds__(256) void m3_stage_copy_kernel(
     uint8_t *destination, const uint8_t *source, uint32_t bytes,
-    uint32_t head, uint32_t vectors)
+    uint32_t head, uint32_t vectors, uint32_t *word, uint32_t sequence,
+    uint32_t set)
 {
     const uint32_t step = gridDim.x * blockDim.x;
     const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x;
@@ -717,6 +767,25 @@ __global__ __launch_bounds__(256) void m3_stage_copy_kernel(
         destination[rest + first] = source[rest + first];
     }
     __threadfence_system();
+    if (word == nullptr) {
+        return;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0U) {
+        return;
+    }
+    if (gridDim.x != 1U) {
+        if (__hip_atomic_fetch_add(&m3_stage_arrived[set], 1U,
+                                   __ATOMIC_ACQ_REL,
+                                   __HIP_MEMORY_SCOPE_AGENT) !=
+            gridDim.x - 1U) {
+            return;
+        }
+        __hip_atomic_store(&m3_stage_arrived[set], 0U, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __hip_atomic_store(word, sequence, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 /* How far into 16 bytes device memory at `address` starts: where a copy of
@@ -724,22 +793,6 @@ __global__ __launch_bounds__(256) void m3_stage_copy_kernel(
 static size_t m3_stage_phase(const void *address)
 {
     return (uintptr_t)address & 15U;
-}
-
-static int m3_stage_copy(m3_hip_device *device, void *destination,
-                         const void *source, size_t bytes, char *message,
-                         size_t capacity)
-{
-    const uint32_t head =
-        (uint32_t)std::min(bytes, (16U - m3_stage_phase(source)) & 15U);
-    const uint32_t vectors = (uint32_t)((bytes - head) / 16U);
-    const uint32_t blocks = m3_grid_blocks(device, vectors + 1U, 256U, 1U);
-
-    hipLaunchKernelGGL(m3_stage_copy_kernel, dim3(blocks), dim3(256), 0,
-                       device->stream, (uint8_t *)destination,
-                       (const uint8_t *)source, (uint32_t)bytes, head,
-                       vectors);
-    return m3_hip_check(hipGetLastError(), "staged copy", message, capacity);
 }
 
 /* The steps of a staged copy on the device's stream (m3_staging.h). */
@@ -752,16 +805,28 @@ struct m3_stage_stream {
     int queue(uint8_t *destination, const uint8_t *source, size_t bytes,
               uint32_t *sequence)
     {
-        int code = m3_stage_copy(device, destination, source, bytes, message,
-                                 capacity);
+        const uint32_t head =
+            (uint32_t)std::min(bytes, (16U - m3_stage_phase(source)) & 15U);
+        const uint32_t vectors = (uint32_t)((bytes - head) / 16U);
+        const uint32_t blocks = m3_grid_blocks(device, vectors + 1U, 256U,
+                                               1U);
+        const bool whole = bytes <= kStageLeast;
 
-        if (code == M3_HIP_OK) {
+        hipLaunchKernelGGL(m3_stage_copy_kernel, dim3(blocks), dim3(256), 0,
+                           device->stream, destination, source,
+                           (uint32_t)bytes, head, vectors,
+                           whole ? word() : nullptr, set->sequence + 1U,
+                           set->index);
+        int code = m3_hip_check(hipGetLastError(), "staged copy", message,
+                                capacity);
+
+        if (code == M3_HIP_OK && !whole) {
             hipLaunchKernelGGL(m3_done_kernel, dim3(1), dim3(64), 0,
-                               device->stream, word(),
-                               set->sequence + 1U);
+                               device->stream, word(), set->sequence + 1U);
             code = m3_hip_check(hipGetLastError(), "staged copy's mark",
                                 message, capacity);
         }
+
         if (code == M3_HIP_OK) {
             *sequence = ++set->sequence;
         }
@@ -881,7 +946,7 @@ extern "C" int m3_hip_copy_h2d(m3_hip_device *device,
             },
             message, capacity);
     }
-    if (byte_count <= kStageUpload && !device->timing) {
+    if (m3_stage_wanted(device, byte_count, false)) {
         bool staged = false;
 
         code = m3_stage_transfer(device, false, device_destination,
@@ -919,9 +984,7 @@ extern "C" int m3_hip_copy_d2h(m3_hip_device *device, void *host_destination,
     if (byte_count == 0U) {
         return M3_HIP_OK;
     }
-    if ((byte_count <= (256U << 10U) ||
-         (byte_count >= (1U << 20U) && byte_count <= kStageDownload)) &&
-        !device->timing) {
+    if (m3_stage_wanted(device, byte_count, true)) {
         bool staged = false;
 
         code = m3_stage_transfer(device, true, host_destination,

@@ -96,6 +96,7 @@ int m3_stage_read(Ops &ops, uint8_t *buffer, uint8_t *destination,
  * through the runtime instead. */
 struct m3_stage_set {
     uint8_t *memory;   /* null: not allocated */
+    uint32_t index;    /* among its GPU's sets */
     uint32_t sequence; /* the last completion number queued for it */
     bool lent;         /* or lost: queued work may still touch it */
     bool used;         /* since the last handle closed before */
@@ -161,6 +162,7 @@ public:
         }
         if (found != nullptr && found->memory == nullptr && !g.refused) {
             found->memory = allocate();
+            found->index = (uint32_t)(found - g.sets);
             g.refused = found->memory == nullptr;
         }
         if (found == nullptr || found->memory == nullptr) {

@@ -1,9 +1,10 @@
 """Host copies through the device's pinned staging memory (GPU).
 
-Copies of 257 bytes to 192 KiB to the device, and of up to 256 KiB or 1 to 4
-MiB from it, go through staging memory, reads in chunks; others, and those
-with timing on, take other paths. Sizes at the edges of the paths and chunks, at
-any byte offset, and from several threads over one device.
+Copies of 257 bytes to 128 KiB to the device, and of up to 256 KiB or 1 to 4
+MiB from it, go through staging memory, reads in chunks; others, those of
+middle sizes behind a runtime copy or in a long row, and those with timing on
+take other paths. Sizes at the edges of the paths and chunks, at any byte
+offset, in rows, and from several threads over one device.
 """
 import ctypes
 import os
@@ -76,7 +77,8 @@ def device(gpu):
 
 
 @pytest.mark.parametrize("count", [
-    1, 8, 15, 16, 17, 31, 255, 256, 257, 1000, 4096, 192 * KIB, 192 * KIB + 1, 256 * KIB - 1, 256 * KIB, 256 * KIB + 1,
+    1, 8, 15, 16, 17, 31, 255, 256, 257, 1000, 4096, 32 * KIB, 32 * KIB + 1,
+    128 * KIB, 128 * KIB + 1, 192 * KIB, 256 * KIB - 1, 256 * KIB, 256 * KIB + 1,
     512 * KIB, 512 * KIB + 4, 700001, MIB - 65, MIB - 1, MIB, 3 * MIB + 7, 4 * MIB, 4 * MIB + 1])
 @pytest.mark.parametrize("offset", [0, 1, 2, 4, 6, 8, 15])
 def test_copy_sizes(device, count, offset):
@@ -106,6 +108,24 @@ def test_many_writes_in_order(device):
         data[:] = 77  # the caller's buffer is free when the call returns
         expected[offset:offset + count] = k & 255
     assert np.array_equal(device.read(0, 2 * MIB), expected)
+
+
+@pytest.mark.parametrize("count", [32 * KIB, 96 * KIB, 128 * KIB, 256 * KIB])
+def test_rows_of_copies(device, count):
+    """Uniform rows, longer than those that stay staged, with runtime copies
+    and small ones between: every copy whole, in order."""
+    rng = np.random.default_rng(count)
+    data = rng.integers(0, 256, (40, count), np.uint8)
+    for k in range(40):
+        device.write((k & 3) * count, data[k])
+        if k % 17 == 16:
+            device.write(8 * MIB, data[0][:100])
+            device.write(9 * MIB, np.resize(data[0], 600 * KIB))
+        assert np.array_equal(device.read((k & 3) * count, count), data[k])
+    for k in range(40):
+        device.write((k & 15) * count, data[k])
+    for k in range(24, 40):
+        assert np.array_equal(device.read((k & 15) * count, count), data[k])
 
 
 def allocations():
@@ -165,11 +185,11 @@ def made(call):
     return t.allocations() - before
 zeros = np.zeros(4 * t.MIB + 1, np.uint8)
 assert made(lambda: device.write(0, zeros[:256])) == 0
-assert made(lambda: device.write(0, zeros[:192 * t.KIB + 1])) == 0
+assert made(lambda: device.write(0, zeros[:128 * t.KIB + 1])) == 0
 assert made(lambda: device.read(0, 4 * t.MIB + 1)) == 0
 assert made(lambda: device.read(0, 512 * t.KIB)) == 0
 assert made(lambda: device.%s) == 1
-assert made(lambda: device.write(0, zeros[:192 * t.KIB])) == 0
+assert made(lambda: device.write(0, zeros[:128 * t.KIB])) == 0
 assert made(lambda: device.read(0, 4 * t.MIB)) == 0
 device.close()
 print("taken")
