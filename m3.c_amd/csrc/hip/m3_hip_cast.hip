@@ -254,11 +254,21 @@ struct m3_transpose_args {
     m3_hip_gate list_gate;
 };
 
-/* The smallest extent of both axes for which tiles are used: at 16 a tile's
- * lanes are a quarter (u) or an eighth (n) full, and [1,50000,33], half
- * full, takes 6 us against 20 for one element per lane; below it the
- * kernel would mostly read and write nothing. */
+/* When tiles are used: both extents at least 16 (below it a tile's lanes are
+ * less than a quarter (u) or an eighth (n) full), and so much of the tiles
+ * that cover the two axes inside the tensor that the tile kernel's work for
+ * nothing stays below what one element per lane costs: 5 of 64 parts for a
+ * copy, 6 for a conversion, 9 for one from or to F16 (in integer
+ * instructions). Against the per-element kernel, many small planes of n x u,
+ * F32, BF16 and F16 to F32: 16 x 16 (2 parts) 60 -> 120, 59 -> 90 and 65 ->
+ * 209 us, 24 x 24 (4.5) 63 -> 61, 58 -> 46 and 65 -> 100, 24 x 32 (6) 62 ->
+ * 51, 58 -> 38 and 66 -> 78, 32 x 32 (8) 61 -> 39, 59 -> 29 and 66 -> 60, 32
+ * x 40 (10) 64 -> 34, 58 -> 26 and 66 -> 51; a plane that only just needs a
+ * second tile, 17 x 70 (4.6), 60 -> 84, 59 -> 65 and 65 -> 115. */
 constexpr uint32_t kTransposeLeast = 16U;
+constexpr uint32_t kTransposeFillCopy = 5U;
+constexpr uint32_t kTransposeFill = 6U;
+constexpr uint32_t kTransposeFillF16 = 9U;
 constexpr uint32_t kTileU = 64U;
 constexpr uint32_t kTileN = 128U;
 constexpr uint32_t kXcds = 8U;
@@ -600,9 +610,10 @@ m3_transpose_launcher m3_transpose_of(uint32_t in, uint32_t out)
 
 /* Fills `args` when the plan (operand 1 the input) is one that the
  * transposing kernel takes: the innermost axis strided in the input, some
- * other axis of unit stride there, both of at least kTransposeLeast. */
+ * other axis of unit stride there, both of at least kTransposeLeast and
+ * filling `fill` of 64 parts of their tiles. */
 bool m3_plan_transpose(const m3_index_plan &plan, uint32_t in_size,
-                       m3_transpose_args *args)
+                       uint32_t fill, m3_transpose_args *args)
 {
     const uint32_t inner = plan.rank - 1U;
     uint64_t out_strides[M3_HIP_MAX_RANK];
@@ -637,7 +648,9 @@ bool m3_plan_transpose(const m3_index_plan &plan, uint32_t in_size,
     const uint64_t tiles_u = (plan.shape[unit] + kTileU - 1U) / kTileU;
 
     /* two factors below 2^32 each, checked before the third */
-    if (tiles_n * tiles_u > 0x7fffffffULL ||
+    if (plan.shape[inner] * plan.shape[unit] <
+            tiles_n * tiles_u * (kTileN * kTileU / 64U * fill) ||
+        tiles_n * tiles_u > 0x7fffffffULL ||
         outer > 0x7fffffffULL / (tiles_n * tiles_u)) {
         return false;
     }
@@ -727,7 +740,13 @@ int m3_launch_unary(m3_hip_device *device, const m3_hip_view *input,
     m3_transpose_args transpose;
 
     std::memset(&transpose, 0, sizeof(transpose));
-    if (m3_plan_transpose(plan, (uint32_t)m3_dtype_bytes(input->dtype),
+    const uint32_t fill = input->dtype == output->dtype ? kTransposeFillCopy
+                          : input->dtype == M3_HIP_F16 ||
+                                  output->dtype == M3_HIP_F16
+                              ? kTransposeFillF16
+                              : kTransposeFill;
+
+    if (m3_plan_transpose(plan, (uint32_t)m3_dtype_bytes(input->dtype), fill,
                           &transpose)) {
         const m3_transpose_launcher launcher =
             m3_transpose_of(input->dtype, output->dtype);

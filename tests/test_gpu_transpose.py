@@ -1,8 +1,8 @@
 """COPY and CAST of permuted views through transposing tiles (GPU).
 
 An input whose unit-stride axis is not the output's innermost one runs a
-64 x 128 tile kernel when both axes have at least 16 elements, else the
-general kernel. The extents are the edges of the tiles and of the rule, and
+64 x 128 tile kernel when both axes have at least 16 elements and fill enough
+of their tiles, else the general kernel. The extents are the edges of the tiles and of the rule, and
 one to three elements past a multiple of four; the views are transposes
 with outer axes before, between and after, padded, broadcast and offset.
 Checked against the oracle bit for bit, NaN payloads included.
@@ -65,7 +65,8 @@ def source_of(rng, src, dst, count):
 @pytest.mark.parametrize("src,dst", PAIRS)
 @pytest.mark.parametrize("length,channels", [
     (16, 16), (15, 64), (64, 15), (17, 18), (63, 65), (64, 128), (65, 127),
-    (127, 66), (129, 67), (130, 64), (257, 131)])
+    (127, 66), (129, 67), (130, 64), (257, 131), (16, 64), (64, 16), (16, 48),
+    (24, 24), (24, 32), (32, 40), (40, 32), (30, 43), (16, 65), (160, 16)])
 def test_transposed(hip, src, dst, length, channels):
     rng = np.random.default_rng(51000 + length * 7 + channels)
     size = m3.DTYPE_SIZES[src]
