@@ -170,11 +170,27 @@ __device__ __forceinline__ uint4 m3_operand_load4(const m3_bin_operand &o,
 
         return make_uint4(v, v, v, v);
     }
-    if (o.mode == M3_BIN_ROW || o.mode == M3_BIN_ROW_CUT) {
-        /* one element, or two for a group in which a run of I ends: both
-         * from cache (the second is the first again in the others). A wave
-         * whose groups lie in one run, as most do when runs are long, finds
-         * and converts its element once, in scalar registers. */
+    if (o.mode == M3_BIN_ROW) {
+        /* one element, from cache; a wave whose groups lie in one run, as
+         * most do when runs are long, finds and converts it once, in scalar
+         * registers */
+        const uint32_t q = m3_fast_div_q(o.inner, f);
+        const uint32_t run = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
+
+        if (__all(q == run)) {
+            const uint32_t v = m3_operand_at<DT>(
+                o, run - m3_fast_div_q(o.period, run) * o.period.divisor);
+
+            return make_uint4(v, v, v, v);
+        }
+        const uint32_t v = m3_operand_at<DT>(
+            o, q - m3_fast_div_q(o.period, q) * o.period.divisor);
+
+        return make_uint4(v, v, v, v);
+    }
+    if (o.mode == M3_BIN_ROW_CUT) {
+        /* the same, or two elements for a group in which a run of I ends:
+         * both from cache (the second is the first again in the others) */
         const uint32_t q = m3_fast_div_q(o.inner, f);
         const uint32_t here = (q + 1U) * o.inner.divisor - f;
         const uint32_t run = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
@@ -223,12 +239,53 @@ __device__ __forceinline__ void m3_store4(uint8_t *out, uint32_t dtype,
                     m3_narrow4_bits(v, dtype));
 }
 
-template <int OP, uint32_t DT, int UNROLL = (int)kUnroll>
+/* What a group loads of an F32 operand, where that is known when the kernel
+ * is compiled: its own four elements, four of a trailing broadcast, or one
+ * element (of a row; a scalar is a row operand whose inner axis and period
+ * are 1). ANY: by the operand's mode. */
+enum m3_operand_kind : uint32_t {
+    M3_KIND_FULL = 0,
+    M3_KIND_TRAIL = 1,
+    M3_KIND_ONE = 2,
+    M3_KIND_ANY = 3
+};
+
+/* F32 bits of elements f..f+3 of an F32 operand of kind KIND (not ANY). */
+template <uint32_t KIND>
+__device__ __forceinline__ uint4 m3_kind_load4(const m3_bin_operand &o,
+                                               uint32_t f)
+{
+    if constexpr (KIND == M3_KIND_FULL) {
+        return m3_stream_load((const uint4 *)(o.base + (uint64_t)f * 4U));
+    } else if constexpr (KIND == M3_KIND_TRAIL) {
+        const uint32_t index =
+            f - m3_fast_div_q(o.period, f) * o.period.divisor;
+        const m3_u32x4 w =
+            *(const m3_u32x4_any *)(o.base + (uint64_t)index * 4U);
+
+        return make_uint4(w[0], w[1], w[2], w[3]);
+    } else {
+        const uint32_t run = m3_fast_div_q(o.inner, f);
+        const uint32_t v = m3_operand_at<M3N_F32>(
+            o, run - m3_fast_div_q(o.period, run) * o.period.divisor);
+
+        return make_uint4(v, v, v, v);
+    }
+}
+
+/* F32 operands of known kinds have an instance per pair of kinds: with all
+ * modes in one kernel, calls that need the simplest loads pay for the others'
+ * instructions (20,000 elements 3.3 us against 2.6, 3,000,000 times a scalar
+ * 6.1 against 4.8, 4,194,304 in rows of 8 times a column 8.1 against 5.8;
+ * without the modes that cut groups 3.1, 5.6 and 6.8). Otherwise the loads
+ * go by the modes (kinds ANY). */
+template <int OP, uint32_t DT, uint32_t LEFT, uint32_t RIGHT>
 __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
 {
     if (m3_gate_closed(a.list_gate)) {
         return; /* a check earlier in the list failed */
     }
+    constexpr uint32_t UNROLL = kUnroll;
     const uint32_t out_dtype = DT == kAnyDtype ? a.out_dtype : DT;
     const uint32_t step = gridDim.x * kThreads * UNROLL;
 
@@ -241,9 +298,17 @@ __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
         for (uint32_t u = 0U; u < UNROLL; ++u) {
             uint32_t g = first + u * kThreads;
 
-            if (g < a.groups) {
-                left[u] = m3_operand_load4<DT>(a.left, g * 4U);
-                right[u] = m3_operand_load4<DT>(a.right, g * 4U);
+            if constexpr (LEFT == M3_KIND_ANY) {
+                if (g < a.groups) {
+                    left[u] = m3_operand_load4<DT>(a.left, g * 4U);
+                    right[u] = m3_operand_load4<DT>(a.right, g * 4U);
+                }
+            } else {
+                /* groups past the end read the last one, store nothing */
+                const uint32_t f = 4U * min(g, a.groups - 1U);
+
+                left[u] = m3_kind_load4<LEFT>(a.left, f);
+                right[u] = m3_kind_load4<RIGHT>(a.right, f);
             }
         }
 #pragma unroll
@@ -278,7 +343,7 @@ __global__ __launch_bounds__(256) void m3_binary_vec_kernel(m3_bin_vec_args a)
 }
 
 /* Groups of four outputs per lane of the held form, and its workgroups
- * per CU (120 VGPRs: four waves per SIMD, all resident at once). */
+ * per CU (at most 128 VGPRs: four waves per SIMD, all resident at once). */
 constexpr int kHeldGroups = 12;
 constexpr uint32_t kHeldBlocksPerCu = 4U;
 /* Its wait before the stores, as a multiple of the time the launch's
@@ -289,41 +354,18 @@ constexpr uint32_t kHeldBlocksPerCu = 4U;
  * resident, 20-31 us). */
 constexpr double kBinaryHoldFactor = 1.1;
 
-/* F32 bits of operand elements f..f+3 for the held form: 16-byte aligned
- * operands, every mode by its element indices. Its own function because
- * twelve groups of two operands in flight are at the mercy of how the
- * compiler lays out the choice of mode: with m3_operand_load4 it waits for
- * each group's loads (x[8,1024,1536] * c[1536] 23.5 against 17.7 us). */
-__device__ __forceinline__ uint4 m3_held_load4(const m3_bin_operand &o,
-                                               uint32_t f)
-{
-    if (o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL) {
-        uint32_t index = o.mode == M3_BIN_FULL
-                             ? f
-                             : f - m3_fast_div_q(o.period, f) *
-                                       o.period.divisor;
-        const uint4 *p = (const uint4 *)(o.base + (uint64_t)index * 4U);
-
-        return o.mode == M3_BIN_FULL ? m3_stream_load(p) : *p;
-    }
-    if (o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR) {
-        uint32_t v = m3_operand_element<M3N_F32>(o, f);
-
-        return make_uint4(v, v, v, v);
-    }
-    return make_uint4(m3_operand_element<M3N_F32>(o, f),
-                      m3_operand_element<M3N_F32>(o, f + 1U),
-                      m3_operand_element<M3N_F32>(o, f + 2U),
-                      m3_operand_element<M3N_F32>(o, f + 3U));
-}
-
 /* The held form of the F32 vector kernel, for a launch whose workgroups
- * are all resident at once: each lane loads its kHeldGroups groups of both
- * operands, forms the results, and stores them only hold_ticks
- * (s_memrealtime) after its start, so that the launch's writes do not
- * compete with its reads still in flight. The wait is bounded by the
- * clock; results are those of m3_binary_vec_kernel. */
-template <int OP, int K>
+ * are all resident at once: each lane loads its K groups of both operands,
+ * forms the results, and stores them only hold_ticks after its start
+ * (s_memrealtime), so that the launch's writes do not compete with its reads
+ * still in flight. The wait is bounded by the clock; results are those of
+ * m3_binary_vec_kernel. An instance per pair of operand kinds, and lanes
+ * past the end read the last group, so that the loads are one straight line,
+ * all in flight: with the kinds tested among the loads, the time moved with
+ * every change of the code around them (x[131072,64] * c[64], the same loads:
+ * 12.5, 14.0 and 20.2 us; 12.8 here, and 12.8 instead of 19.2 times a
+ * column of 131,072). */
+template <int OP, int K, uint32_t LEFT, uint32_t RIGHT>
 __global__ __launch_bounds__(256) void m3_binary_held_kernel(
     m3_bin_vec_args a, uint32_t hold_ticks)
 {
@@ -337,15 +379,11 @@ __global__ __launch_bounds__(256) void m3_binary_held_kernel(
 
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const uint32_t g = first + (uint32_t)k * kThreads;
+        const uint32_t f =
+            4U * min(first + (uint32_t)k * kThreads, a.groups - 1U);
 
-        if (g < a.groups) {
-            left[k] = m3_held_load4(a.left, g * 4U);
-            right[k] = m3_held_load4(a.right, g * 4U);
-        } else {
-            left[k] = make_uint4(0U, 0U, 0U, 0U);
-            right[k] = left[k];
-        }
+        left[k] = m3_kind_load4<LEFT>(a.left, f);
+        right[k] = m3_kind_load4<RIGHT>(a.right, f);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -642,13 +680,61 @@ bool m3_classify_operand(const m3_index_plan &plan, uint32_t k,
     return true;
 }
 
+/* The kind of an F32 operand. */
+uint32_t m3_kind_of(const m3_bin_operand &o)
+{
+    return o.mode == M3_BIN_FULL    ? M3_KIND_FULL
+           : o.mode == M3_BIN_TRAIL ? M3_KIND_TRAIL
+           : o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR ? M3_KIND_ONE
+                                                             : M3_KIND_ANY;
+}
+
 /* True for an operand that gives a group one element or one 16-byte
  * aligned vector. */
 bool m3_operand_whole(const m3_bin_operand &o)
 {
-    return ((o.mode == M3_BIN_FULL || o.mode == M3_BIN_TRAIL) &&
-            ((uintptr_t)o.base & 15U) == 0U) ||
-           o.mode == M3_BIN_ROW || o.mode == M3_BIN_SCALAR;
+    const uint32_t kind = m3_kind_of(o);
+
+    return kind == M3_KIND_ONE ||
+           (kind != M3_KIND_ANY && ((uintptr_t)o.base & 15U) == 0U);
+}
+
+/* The F32 kernels of one pair of kinds: streamed (hold_ticks null) or held. */
+typedef void (*m3_binary_launcher)(dim3, hipStream_t, hipEvent_t, hipEvent_t,
+                                   const m3_bin_vec_args &, const uint32_t *);
+
+template <int OP, uint32_t LEFT, uint32_t RIGHT>
+void m3_launch_kinds(dim3 grid, hipStream_t stream, hipEvent_t start,
+                     hipEvent_t stop, const m3_bin_vec_args &args,
+                     const uint32_t *hold_ticks)
+{
+    if (hold_ticks != nullptr) {
+        hipExtLaunchKernelGGL(
+            (m3_binary_held_kernel<OP, kHeldGroups, LEFT, RIGHT>), grid,
+            dim3(kThreads), 0, stream, start, stop, 0U, args, *hold_ticks);
+        return;
+    }
+    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, M3N_F32, LEFT, RIGHT>),
+                          grid, dim3(kThreads), 0, stream, start, stop, 0U,
+                          args);
+}
+
+/* [left kind][right kind] */
+template <int OP>
+m3_binary_launcher m3_binary_launcher_of(uint32_t left, uint32_t right)
+{
+    static const m3_binary_launcher launchers[3][3] = {
+        {&m3_launch_kinds<OP, M3_KIND_FULL, M3_KIND_FULL>,
+         &m3_launch_kinds<OP, M3_KIND_FULL, M3_KIND_TRAIL>,
+         &m3_launch_kinds<OP, M3_KIND_FULL, M3_KIND_ONE>},
+        {&m3_launch_kinds<OP, M3_KIND_TRAIL, M3_KIND_FULL>,
+         &m3_launch_kinds<OP, M3_KIND_TRAIL, M3_KIND_TRAIL>,
+         &m3_launch_kinds<OP, M3_KIND_TRAIL, M3_KIND_ONE>},
+        {&m3_launch_kinds<OP, M3_KIND_ONE, M3_KIND_FULL>,
+         &m3_launch_kinds<OP, M3_KIND_ONE, M3_KIND_TRAIL>,
+         &m3_launch_kinds<OP, M3_KIND_ONE, M3_KIND_ONE>}};
+
+    return launchers[left][right];
 }
 
 template <int OP>
@@ -703,25 +789,43 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
         const uint32_t hold_ticks = (uint32_t)(
             kBinaryHoldFactor * read_bytes / 8.0e6 *
             (double)device->wall_clock_khz / 1000.0);
+        const uint32_t left_kind = f32 ? m3_kind_of(vec.left) : M3_KIND_ANY;
+        const uint32_t right_kind = f32 ? m3_kind_of(vec.right) : M3_KIND_ANY;
 
+        if (left_kind != M3_KIND_ANY && right_kind != M3_KIND_ANY) {
+            const m3_binary_launcher launcher =
+                m3_binary_launcher_of<OP>(left_kind, right_kind);
+
+            for (m3_bin_operand *o : {&vec.left, &vec.right}) {
+                if (o->mode == M3_BIN_SCALAR) {
+                    o->inner = m3_fast_div_make(1U);
+                    o->period = m3_fast_div_make(1U);
+                }
+            }
+            return m3_hip_launch(
+                device, names[OP],
+                [&](hipEvent_t start, hipEvent_t stop) {
+                    launcher(dim3(hold ? (uint32_t)held : blocks),
+                             device->stream, start, stop, vec,
+                             hold ? &hold_ticks : nullptr);
+                },
+                message, capacity);
+        }
         return m3_hip_launch(
             device, names[OP],
             [&](hipEvent_t start, hipEvent_t stop) {
-                if (hold) {
+                if (f32) {
                     hipExtLaunchKernelGGL(
-                        (m3_binary_held_kernel<OP, kHeldGroups>),
-                        dim3((uint32_t)held), dim3(kThreads), 0,
-                        device->stream, start, stop, 0U, vec, hold_ticks);
-                } else if (f32) {
-                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, M3N_F32>),
-                                          dim3(blocks), dim3(kThreads), 0,
-                                          device->stream, start, stop, 0U,
-                                          vec);
+                        (m3_binary_vec_kernel<OP, M3N_F32, M3_KIND_ANY,
+                                              M3_KIND_ANY>),
+                        dim3(blocks), dim3(kThreads), 0, device->stream,
+                        start, stop, 0U, vec);
                 } else {
-                    hipExtLaunchKernelGGL((m3_binary_vec_kernel<OP, kAnyDtype>),
-                                          dim3(blocks), dim3(kThreads), 0,
-                                          device->stream, start, stop, 0U,
-                                          vec);
+                    hipExtLaunchKernelGGL(
+                        (m3_binary_vec_kernel<OP, kAnyDtype, M3_KIND_ANY,
+                                              M3_KIND_ANY>),
+                        dim3(blocks), dim3(kThreads), 0, device->stream,
+                        start, stop, 0U, vec);
                 }
             },
             message, capacity);

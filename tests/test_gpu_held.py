@@ -80,6 +80,38 @@ def test_held_binary_f32(hip, op, case):
             "held binary op%d %s x %s" % (op, left_shape, right_shape))
 
 
+# an operand's shape by what a group of four loads of it
+KINDS = {"full": lambda a, b: (a, b), "trail": lambda a, b: (1, b),
+         "row": lambda a, b: (a, 1), "scalar": lambda a, b: (1, 1)}
+PAIRS = [("full", kind) for kind in KINDS] + [
+    (kind, "full") for kind in KINDS if kind != "full"] + [
+    ("trail", "row"), ("row", "trail")]
+
+
+@pytest.mark.parametrize("shape", [(3, 4), (257, 20), (4931, 1540)])
+@pytest.mark.parametrize("left_kind,right_kind", PAIRS)
+def test_binary_f32_kinds(hip, shape, left_kind, right_kind):
+    """Every pair of operand kinds with a kernel of its own, in tensors of a
+    few groups, of some workgroups and of the held form's size (on one
+    MI355X), at an aligned address and one element past it, where the
+    streaming form takes over."""
+    rng = np.random.default_rng(7100 + shape[0])
+    left_shape = KINDS[left_kind](*shape)
+    right_shape = KINDS[right_kind](*shape)
+    left = random_f32(rng, int(np.prod(left_shape)) + 1)
+    right = random_f32(rng, int(np.prod(right_shape)) + 1)
+    out = np.zeros(4 * (int(np.prod(shape)) + 1), np.uint8)
+    op = [m3.OP_ADD, m3.OP_MUL, m3.OP_SUB, m3.OP_DIV][
+        (list(KINDS).index(left_kind) + list(KINDS).index(right_kind)) % 4]
+    for shift in (0, 4):
+        compare(hip, op, [as_bytes(left), as_bytes(right), out],
+                [ViewSpec(0, m3.F32, left_shape, None, shift),
+                 ViewSpec(1, m3.F32, right_shape, None, shift),
+                 ViewSpec(2, m3.F32, shape, None, shift)],
+                "kinds %s %s %s op%d shift %d" % (shape, left_kind,
+                                                  right_kind, op, shift))
+
+
 def sixteen_bit_source(rng, count):
     """Every 16-bit pattern, then random ones."""
     every = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16)
