@@ -54,6 +54,8 @@ constexpr uint32_t kTanhUnroll = 2U;
  * process: GATED_SILU [16384, 3072] 94.5 against 100.5 us in F32 and 68.5
  * against 72.3 us in BF16; TANH x[2,1536,65536] 484 against 506 us. */
 constexpr uint32_t kBlocksPerCu = 1024U;
+/* lanes a CU holds at once: four SIMDs, eight waves of 64 each */
+constexpr uint32_t kLanesPerCu = 2048U;
 
 /* Stores four F32 results (as bits) rounded to dtype D at group g. */
 template <uint32_t D>
@@ -728,9 +730,20 @@ extern "C" int m3_hip_launch_gated_silu(m3_hip_device *device,
     const bool contiguous =
         m3_view_is_contiguous(gate) && m3_view_is_contiguous(up);
     /* rows: each operand contiguous or in rows, the same ones; four
-     * consecutive elements then lie in at most two rows */
+     * consecutive elements then lie in at most two rows. From as many
+     * elements on as the device has lanes at once (F32; 7/4 of them in 16
+     * bits, where an element costs less to load and as much to compute):
+     * below that the general kernel's one element per lane leaves no lane
+     * idle, while sixteen per lane take their turns in a few waves. Packed
+     * gate and up of width 3,072, general against rows kernel: F32 64 rows
+     * 3.6 and 4.6 us, 128 rows 4.4 and 4.8, 170 5.0 and 4.8; F16 64 rows 4.0
+     * and 7.2, 256 7.2 and 8.1, 341 8.6 and 7.9; BF16 64 rows 3.8 and 5.9,
+     * 256 6.3 and 6.7, 341 7.6 and 6.1. */
+    const uint64_t lanes = (uint64_t)device->compute_units * kLanesPerCu;
     const bool in_rows =
-        !contiguous && m3_silu_rows(gate, &gate_width, &gate_pitch) &&
+        !contiguous &&
+        count >= (dtype == M3_HIP_F32 ? lanes : lanes / 4U * 7U) &&
+        m3_silu_rows(gate, &gate_width, &gate_pitch) &&
         m3_silu_rows(up, &up_width, &up_pitch) &&
         (gate_width == up_width || gate_width == count ||
          up_width == count) &&
