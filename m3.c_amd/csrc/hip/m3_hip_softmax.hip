@@ -1944,15 +1944,18 @@ void m3_launch_lane_rows(dim3 grid, hipStream_t stream, hipEvent_t start,
  * six (at most 80) for four- and eight-wave workgroups of 48 with F32 I/O
  * (six and three per CU, the walking wave's values parked in LDS: faster
  * than five and two per CU, where for eight-wave workgroups of 40 three
- * per CU measured slower); five (at most 96) for two- and four-wave
- * workgroups of 64 values per lane with F32 I/O (ten and five per CU),
- * four-wave ones of 48 with 16-bit I/O and eight-wave ones of 40; four
- * (128 VGPRs) for the rest, which would spill registers at 96. */
+ * per CU measured slower; the ragged forms spill two registers); five (at
+ * most 96) for two- and four-wave workgroups of 64 values per lane with F32
+ * I/O and aligned rows (ten and five per CU), four-wave ones of up to 48
+ * and eight-wave ones of up to 40; four (128 VGPRs) for the rest, which
+ * would spill registers at 96, and for all of sixteen waves, of which a CU
+ * holds one workgroup at 80 VGPRs as at 128 (48 values at 80 spilled two
+ * registers: F32 [341,49152] 65.7 -> 64.0 us, [32,36865] 27.6 -> 26.6). */
 template <int Q, int NW, bool F32IO, bool RAGGED>
 constexpr int m3_wide_waves_per_eu()
 {
     return NW == 2 && Q == 8 ? 7
-           : Q == 12 && F32IO ? 6
+           : Q == 12 && F32IO && NW <= 8 ? 6
            : Q == 16 && RAGGED ? 4
            : (NW <= 4 && (F32IO || Q <= 12)) || (NW == 8 && Q <= 10) ? 5
                                                                     : 4;
