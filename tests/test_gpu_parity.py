@@ -308,9 +308,8 @@ def test_softmax_zero_tails(hip, width):
 def test_softmax_subnormal_ties(hip, width):
     """Quotients that land exactly on a rounding midpoint of the F32
     subnormal range (e_j = sum * (2k+1) * 2^-150) round to even, as the
-    reference's F32 division does, in every softmax kernel (widths 100,
-    102 and 10000 run the general kernel, 128 to 2048 the rows kernel,
-    4096 the tiled one)."""
+    reference's F32 division does, in every class of softmax rows up to
+    10,000 columns."""
     rng = np.random.default_rng(13000 + width)
     rows = 96
     logits = subnormal_tie_rows(rng, rows, width)
@@ -332,9 +331,7 @@ def softmax_source(logits, dtype):
 @pytest.mark.parametrize("width", [77, 1001, 2047, 2501, 9000, 9001, 16384,
                                    32768])
 def test_softmax_any_width(hip, width):
-    """Widths that are not a multiple of 4 move element by element (77,
-    1001 and 2047 in registers, 2501 and 9001 streamed); rows wider than
-    the LDS tile (9000, 16384, 32768) stream through three passes."""
+    """Ordinary widths of each class of rows, multiples of 4 and not."""
     rng = np.random.default_rng(15000 + width)
     rows = max(6, min(96, 600000 // width))
     logits = softmax_logits(rng, rows, width)
@@ -449,10 +446,10 @@ def lane_row_logits(rng, rows, width):
 @pytest.mark.parametrize("width", [516, 768, 1000, 1020, 1024])
 @pytest.mark.parametrize("rows", [1, 2, 7, 258])
 def test_softmax_lane_rows(hip, width, rows):
-    """F32 rows of 513..1024 columns, four to a wave, one per 16 lanes:
-    partial last waves (rows not a multiple of 4), widths that end inside
-    a lane's block, and special rows at every position within a wave next
-    to ordinary rows."""
+    """F32 rows of 513..1024 columns, so few that a wave takes two, each in
+    two halves: partial last waves, widths that end inside a lane's block,
+    and special rows at every position within a wave next to ordinary rows
+    (many rows, four to a wave: test_gpu_softmax_many.py)."""
     rng = np.random.default_rng(19000 + width * 7 + rows)
     logits = lane_row_logits(rng, rows, width)
     out = np.zeros(logits.nbytes, np.uint8)
@@ -479,8 +476,8 @@ def test_softmax_lane_rows(hip, width, rows):
 @pytest.mark.parametrize("width", [260, 300, 508, 512, 700, 1020, 1024])
 @pytest.mark.parametrize("rows", [7, 258])
 def test_softmax_lane_rows_dtypes(hip, dtypes, width, rows):
-    """The lane-row kernel with 16-bit input or output, 8 float4 per lane
-    (257..512 columns) and 16 (513..1024)."""
+    """The lane-row kernel with 16-bit input or output, in the halves that
+    few rows take: 4 float4 per lane (257..512 columns) and 8 (513..1024)."""
     rng = np.random.default_rng(21000 + width * 7 + rows + 3 * dtypes[0] +
                                 dtypes[1])
     logits = lane_row_logits(rng, rows, width)
@@ -494,19 +491,20 @@ def test_softmax_lane_rows_dtypes(hip, dtypes, width, rows):
 
 
 @pytest.fixture(scope="module")
-def hip_late(gpu):
-    """A HIP backend on which every wave of the lane-row softmax counts as
-    late (M3_HIP_SOFTMAX_LATE_US=0, read when the device opens), so every
-    sum runs the lane-to-lane form."""
-    saved = os.environ.get("M3_HIP_SOFTMAX_LATE_US")
-    os.environ["M3_HIP_SOFTMAX_LATE_US"] = "0"
+def hip_hold(gpu):
+    """A HIP backend on which every wave of the lane-row softmax holds its
+    stores for 30 us from its start (M3_HIP_SOFTMAX_HOLD_US, read when the
+    device opens), where launches of few rows hold them for a fraction of
+    one."""
+    saved = os.environ.get("M3_HIP_SOFTMAX_HOLD_US")
+    os.environ["M3_HIP_SOFTMAX_HOLD_US"] = "30"
     try:
         fixture = HipFixture()
     finally:
         if saved is None:
-            del os.environ["M3_HIP_SOFTMAX_LATE_US"]
+            del os.environ["M3_HIP_SOFTMAX_HOLD_US"]
         else:
-            os.environ["M3_HIP_SOFTMAX_LATE_US"] = saved
+            os.environ["M3_HIP_SOFTMAX_HOLD_US"] = saved
     yield fixture
     fixture.close()
 
@@ -515,22 +513,20 @@ def hip_late(gpu):
                                     (m3.BF16, m3.F32)])
 @pytest.mark.parametrize("width", [300, 516, 1000, 1024])
 @pytest.mark.parametrize("rows", [7, 258])
-def test_softmax_lane_rows_late_path(hip_late, dtypes, width, rows):
-    """The lane-row kernel with every sum passed from lane to lane, the
-    form that waves whose rows arrive late take: the same bits."""
-    if dtypes == (m3.F32, m3.F32) and width <= 512:
-        width += 512  # F32 rows of 257..512 columns take the rows kernel
+def test_softmax_lane_rows_held(hip_hold, dtypes, width, rows):
+    """The lane-row kernel with its stores held back long after the sums:
+    the same bits."""
     rng = np.random.default_rng(23000 + width * 7 + rows + 3 * dtypes[0] +
                                 dtypes[1])
     logits = lane_row_logits(rng, rows, width)
     out_size = 4 if dtypes[1] == m3.F32 else 2
-    compare(hip_late, m3.OP_SOFTMAX,
+    compare(hip_hold, m3.OP_SOFTMAX,
             [softmax_source(logits, dtypes[0]),
              np.zeros(rows * width * out_size, np.uint8)],
             [ViewSpec(0, dtypes[0], (rows, width)),
              ViewSpec(1, dtypes[1], (rows, width))],
-            "softmax lane rows, late path %s w=%d rows=%d" % (dtypes, width,
-                                                             rows))
+            "softmax lane rows, held %s w=%d rows=%d" % (dtypes, width,
+                                                        rows))
 
 
 # ---- snake1d -------------------------------------------------------------------
