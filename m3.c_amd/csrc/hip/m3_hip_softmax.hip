@@ -793,9 +793,9 @@ __device__ __forceinline__ float4 m3_exp4(float4 v, float m,
  * latency of one wave's load, exponentials and sum, hidden by the other
  * waves of its SIMD (at most 56 VGPRs: eight), so a wave takes no more than
  * four rows and passes the running sum from lane to lane
- * (m3_block_sum_passed, half the latency of m3_block_sum). The sum stops
- * after the block that holds the last column other than -inf in any of the
- * four rows. Measured against a wave of eight rows with lane l at columns
+ * (m3_block_sum_passed, half the latency of addends broadcast from their
+ * lanes). The sum stops after the block that holds the last column other
+ * than -inf in any of the four rows. Measured against a wave of eight rows with lane l at columns
  * 4l .. 4l + 3 and the sums in LDS: F32 [254200,33] 83 -> 28 us,
  * [83886,100] 27.3 -> 18.2, [32896,255] 54 -> 19, [32768,256] 14.2 -> 14.0;
  * BF16 [32768,256] 22.2 -> 15.3; two or four groups of four rows per wave

@@ -8,13 +8,15 @@ oracle run command by command: random operations, links on either side,
 dtypes, broadcasts of every class, special values, and lists in which an
 output overlaps another operand, where the commands must stay apart.
 """
+import ctypes
 import sys
 
 import numpy as np
 import pytest
 
 from conftest import m3
-from harness import HipFixture, ViewSpec, as_bytes, run_oracle
+from harness import (HipFixture, HipScanFixture, ViewSpec, as_bytes,
+                     run_oracle)
 
 pytestmark = pytest.mark.gpu
 
@@ -239,3 +241,112 @@ def test_lists_over_empty_tensors(hip, shape, dims):
            (m3.OP_MUL, [e[0], o, e[1]]), (m3.OP_ADD, [e[1], o, e[2]]),
            (m3.OP_ADD, [full[2], full[1], full[3]])],
           "empty %s %s" % (shape, dims))
+
+
+def launches(nodes, shape):
+    """The kernels, by launches, of one run of a session over `nodes`:
+    (kind, out dtype, operand names), "x" the input, "c" a constant of
+    shape's last axis, "s" a Snake1d alpha, and a number the value of that
+    node."""
+    rng = np.random.default_rng(9)
+    graph = m3.Graph()
+    values = {"x": graph.add_value(m3.INPUT, m3.F32, shape)}
+    for name, dims in (("c", (shape[-1],)), ("s", (1, shape[1], 1))):
+        if any(name in inputs for _, _, inputs in nodes):
+            values[name] = graph.add_value(m3.CONSTANT, m3.F32, dims)
+            graph.set_constant(values[name],
+                               (rng.random(dims) + 0.5).astype(np.float32))
+    for k, (kind, dtype, inputs) in enumerate(nodes):
+        values[k] = graph.add_value(m3.OUTPUT, dtype, shape)
+        graph.add_node(kind, [values[v] for v in inputs], [values[k]])
+    session = m3.Session(graph)
+    graph.free()
+    session.write(values["x"],
+                  rng.standard_normal(shape).astype(np.float32))
+    session.run()
+    session.timing_reset()
+    session.timing_enable(True)
+    session.run()
+    kernels = session.timing_read()
+    session.timing_enable(False)
+    session.free()
+    return {name: count for name, (count, _) in kernels.items()}
+
+
+def test_chains_are_taken(gpu, monkeypatch):
+    """Runs that a kernel takes are one launch, and others are not (in
+    sessions that leave the commands as they are: M3_HIP_FUSION=0)."""
+    monkeypatch.setenv("M3_HIP_FUSION", "0")
+    shape = (2, 16, 1000)
+    mul, cast = m3.OP_MUL, m3.OP_CAST
+    assert launches([(mul, m3.F32, ["x", "c"]), (cast, m3.BF16, [0])],
+                    shape) == {"m3_chain": 1}
+    assert launches([(mul, m3.F32, ["x", "c"]), (cast, m3.F16, [0]),
+                     (cast, m3.F32, [1])], shape) == {"m3_chain": 1}
+    assert launches([(m3.OP_SNAKE1D, m3.F32, ["x", "s"]),
+                     (m3.OP_TANH, m3.F32, [0])],
+                    shape) == {"m3_snake1d_tanh": 1}
+    # the second command reads something else than the first one's output
+    apart = launches([(mul, m3.F32, ["x", "c"]), (cast, m3.BF16, ["x"])],
+                     shape)
+    assert "m3_chain" not in apart and sum(apart.values()) == 2
+
+
+def test_overlapping_runs_are_refused(gpu):
+    """m3_hip_launch_chain over one device: taken with outputs apart, and
+    refused, with nothing launched, when an output overlaps another output
+    or an operand."""
+    _, hip_lib = m3.load()
+
+    class Command(ctypes.Structure):
+        _fields_ = [("kind", ctypes.c_uint32), ("op", ctypes.c_uint32),
+                    ("link", ctypes.c_uint32), ("left", m3.HipView),
+                    ("right", m3.HipView), ("output", m3.HipView)]
+
+    hip_lib.m3_hip_launch_chain.argtypes = [
+        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint32,
+        ctypes.POINTER(ctypes.c_int), ctypes.c_char_p, ctypes.c_size_t]
+    device = HipScanFixture()
+    try:
+        count = 1000
+        at = [device.upload(np.zeros(count, np.float32)) for _ in range(5)]
+
+        def view(address):
+            return device.view(address, m3.F32, (count,))
+
+        def taken(x, y, first, z, second):
+            commands = (Command * 2)()
+            commands[0] = Command(0, 0, 0, view(x), view(y), view(first))
+            commands[1] = Command(0, 1, 0, view(first), view(z),
+                                  view(second))
+            result = ctypes.c_int(7)
+            assert hip_lib.m3_hip_launch_chain(
+                device.device, commands, 2, ctypes.byref(result),
+                device.message, 256) == 0, device.message.value
+            return result.value
+
+        a, b, c, d, e = at
+        assert taken(a, b, c, d, e) == 1
+        assert taken(a, a, c, a, e) == 1
+        assert taken(a, b, a, d, e) == 0  # in place
+        assert taken(a, b, c, d, c) == 0  # both outputs one
+        assert taken(a, b, c, d, a) == 0  # over what the first reads
+        assert taken(a, b, c, d, d + 4 * (count - 1)) == 0  # one element
+        assert taken(a, b, c, c + 4, e) == 0  # reads a part of the link
+    finally:
+        device.close()
+
+
+@pytest.mark.parametrize("src,dst", [(m3.F16, m3.F32), (m3.BF16, m3.F32),
+                                     (m3.F16, m3.BF16), (m3.BF16, m3.F16)])
+def test_every_16bit_value(hip, src, dst):
+    """All 65,536 patterns of a 16-bit float through the chain kernel's
+    widening, rounding and NaN rules: converted, then converted back."""
+    patterns = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16)
+    size = m3.DTYPE_SIZES[dst]
+    shape = (1 << 16,)
+    check(hip, [patterns, np.zeros(size << 16, np.uint8),
+                np.zeros(1 << 16, np.uint16)],
+          [(m3.OP_CAST, [ViewSpec(0, src, shape), ViewSpec(1, dst, shape)]),
+           (m3.OP_CAST, [ViewSpec(1, dst, shape), ViewSpec(2, src, shape)])],
+          "every value %d->%d" % (src, dst))
