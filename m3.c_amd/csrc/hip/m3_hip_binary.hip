@@ -476,9 +476,10 @@ __device__ __forceinline__ uint4 m3_chain_op4(uint32_t op, uint4 x, uint4 y)
  * intermediate result back. DT: every operand and output is of that dtype
  * (kAnyDtype: each its own), which drops the choice per value that bound
  * 16-bit chains by instructions. Measured against one launch per
- * operation: F32 x[2,512,24001] * s[512,1] + b[512,1] 67.5 -> 44.8 us (6.6
- * TB/s), BF16 107 -> 32.7, F16 120 -> 40.4; x[8,1024,1536] * c[1536] then
- * to BF16 and back to F32 47.4 -> 28.8. Two groups per lane and one tile
+ * operation, passes over the same buffers: F32 x[2,512,24001] * s[512,1] +
+ * b[512,1] 67.5 -> 44.8 us (6.6 TB/s; over buffers that change from pass to
+ * pass 66.6 -> 54.6, 5.4 TB/s), BF16 107 -> 32.7, F16 120 -> 40.4;
+ * x[8,1024,1536] * c[1536] then to BF16 and back to F32 47.4 -> 28.8. Two groups per lane and one tile
  * per workgroup: one group 29.8 and 46.0, four 30.6 and 46.8; 16 workgroups
  * per CU in a loop the same within 1%. */
 template <int STEPS, uint32_t DT, int UNROLL>

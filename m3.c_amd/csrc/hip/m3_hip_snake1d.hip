@@ -139,8 +139,9 @@ __device__ __forceinline__ void m3_snake_put4(const m3_snake_vec_args &a,
  * (x[2,1536,65536] 264 us, 6.1 TB/s; x[2,192,60001] 30.5 us, 6.0 TB/s,
  * where one element per lane with 64-bit divisions took about 75). TANH:
  * tanhf of the output is stored too, in the launch of the TANH command
- * after it, which then does not read it back: 78 -> 64 us for the two over
- * x[2,192,60001], by then bound by instructions as much as by HBM. */
+ * after it, which then does not read it back: 30.5 + 34.0 us for the two
+ * over x[2,192,60001], 52.3 together, by then bound by instructions (100 per
+ * element, 38 us of issue) as much as by HBM. */
 template <bool TANH>
 __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
     m3_snake_vec_args a)

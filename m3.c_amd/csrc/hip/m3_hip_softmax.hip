@@ -2216,7 +2216,9 @@ extern "C" int m3_hip_launch_softmax(m3_hip_device *device,
              * HBM bandwidth (9.0 us for [16,1024,1024] F32, a pass among
              * others on one box: no hold 22.8 us causal and 27.0 not, 9.0 us
              * 22.4 and 27.2, 10.0 us 23.6 and 27.5, 10.5 us 24.3 and 27.5;
-             * causal [16,1000,1000]: 31.6 without, 28.9 at 9.0), when every
+             * causal [16,1000,1000]: 31.6 without, 28.9 at 9.0; in bench.py,
+             * where the host waits for each run, 24.9 without, 23.4 at 9.0,
+             * 22.7 at 9.5, 23.0 at 10.0, 23.4 at 10.5), when every
              * wave of the launch is resident at once so that all its reads
              * are issued at the start; otherwise none. M3_HIP_SOFTMAX_HOLD_US
              * sets it. */
