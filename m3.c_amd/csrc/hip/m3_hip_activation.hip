@@ -14,12 +14,14 @@
  * 8 bytes per F32 element, GATED_SILU 12 (F32) or 6 (16-bit operands).
  * The vector kernels take contiguous operands of one dtype at any
  * alignment, and for GATED_SILU also a gate and up whose rows are
- * contiguous and evenly spaced (both halves of one projection): a lane handles four consecutive elements
- * per group, kUnroll groups in flight, loads and stores streaming (every
- * element is read and written once). The last count % 4 elements are done
- * by the first lanes of block 0. Every other layout (strided inputs, mixed
- * dtypes for GATED_SILU) runs the general kernel over the coalesced index
- * space with per-element offsets.
+ * contiguous and evenly spaced (both halves of one projection), of about as
+ * many elements as the device has lanes or more (m3_least_elements): a lane
+ * handles four consecutive elements per group, kUnroll groups in flight,
+ * loads and stores streaming (every element is read and written once). The
+ * last count % 4 elements are done by the first lanes of block 0. Smaller
+ * tensors and every other layout (strided inputs, mixed dtypes for
+ * GATED_SILU) run the general kernel over the coalesced index space with
+ * per-element offsets.
  *
  * GATED_SILU's NaN rule costs a recomputation only in a wave where some
  * product is NaN: the plain arithmetic gives the host's bits for every
@@ -54,8 +56,9 @@ constexpr uint32_t kTanhUnroll = 2U;
  * process: GATED_SILU [16384, 3072] 94.5 against 100.5 us in F32 and 68.5
  * against 72.3 us in BF16; TANH x[2,1536,65536] 484 against 506 us. */
 constexpr uint32_t kBlocksPerCu = 1024U;
-/* lanes a CU holds at once: four SIMDs, eight waves of 64 each */
-constexpr uint32_t kLanesPerCu = 2048U;
+/* general against vector kernel: 20,000 elements 2.9 and 3.4 us, 100,000 3.0
+ * and 3.6, 300,000 3.4 and 3.7, 600,000 4.2 and 4.0 */
+constexpr uint32_t kTanhQuarters = 3U;
 
 /* Stores four F32 results (as bits) rounded to dtype D at group g. */
 template <uint32_t D>
@@ -666,7 +669,9 @@ extern "C" int m3_hip_launch_tanh(m3_hip_device *device,
     }
     /* below 2^32 elements the vector kernel's 32-bit group indices, plus
      * one grid stride (at most 2^28), stay below 2^32 */
-    if (m3_view_is_contiguous(input) && count < (1ULL << 32U)) {
+    if (m3_view_is_contiguous(input) &&
+        count >= m3_least_elements(device, kTanhQuarters) &&
+        count < (1ULL << 32U)) {
         m3_tanh_vec_args args;
 
         args.list_gate = device->gate;
@@ -730,27 +735,25 @@ extern "C" int m3_hip_launch_gated_silu(m3_hip_device *device,
     const bool contiguous =
         m3_view_is_contiguous(gate) && m3_view_is_contiguous(up);
     /* rows: each operand contiguous or in rows, the same ones; four
-     * consecutive elements then lie in at most two rows. From as many
-     * elements on as the device has lanes at once (F32; 7/4 of them in 16
-     * bits, where an element costs less to load and as much to compute):
-     * below that the general kernel's one element per lane leaves no lane
-     * idle, while sixteen per lane take their turns in a few waves. Packed
-     * gate and up of width 3,072, general against rows kernel: F32 64 rows
-     * 3.6 and 4.6 us, 128 rows 4.4 and 4.8, 170 5.0 and 4.8; F16 64 rows 4.0
-     * and 7.2, 256 7.2 and 8.1, 341 8.6 and 7.9; BF16 64 rows 3.8 and 5.9,
-     * 256 6.3 and 6.7, 341 7.6 and 6.1. */
-    const uint64_t lanes = (uint64_t)device->compute_units * kLanesPerCu;
+     * consecutive elements then lie in at most two rows */
     const bool in_rows =
-        !contiguous &&
-        count >= (dtype == M3_HIP_F32 ? lanes : lanes / 4U * 7U) &&
-        m3_silu_rows(gate, &gate_width, &gate_pitch) &&
+        !contiguous && m3_silu_rows(gate, &gate_width, &gate_pitch) &&
         m3_silu_rows(up, &up_width, &up_pitch) &&
         (gate_width == up_width || gate_width == count ||
          up_width == count) &&
         std::min(gate_width, up_width) >= 4U;
+    /* General against vector kernel, us, contiguous: F32 64K elements 3.4
+     * and 3.9, 384K 4.1 and 4.1, 512K 4.7 and 4.2; F16 64K 3.6 and 6.0, 768K
+     * 6.5 and 6.5, 1M 7.7 and 6.6; BF16 64K 3.4 and 4.8, 512K 4.7 and 4.9,
+     * 768K 5.8 and 5.0. Halves of rows of 2 x 3,072: F32 192K (64 rows) 3.6
+     * and 4.6, 512K 5.0 and 4.8; F16 192K 4.0 and 7.2, 768K 7.2 and 8.1, 1M
+     * 8.6 and 7.9; BF16 192K 3.8 and 5.9, 768K 6.3 and 6.7, 1M 7.6 and
+     * 6.1. */
+    static const uint32_t quarters[3][2] = {{3U, 4U}, {6U, 7U}, {4U, 7U}};
 
     if (gate->dtype == dtype && up->dtype == dtype &&
         (contiguous || in_rows) &&
+        count >= m3_least_elements(device, quarters[dtype][in_rows]) &&
         count < (1ULL << 32U)) { /* 32-bit group indices, as for TANH */
         m3_silu_vec_args args;
 

@@ -15,8 +15,10 @@
  * where a channel ends inside a group).
  *
  * The vector kernel handles contiguous x and output of any length L of at
- * least 4, at any alignment: a lane takes four consecutive elements, four
- * groups in flight. Other layouts run per element over stride tables.
+ * least 4, at any alignment, of about as many elements as the device has
+ * lanes or more: a lane takes four consecutive elements, four groups in
+ * flight. Smaller tensors and other layouts run per element over stride
+ * tables.
  */
 #include "m3_hip_internal.h"
 #include "m3_libm.h"
@@ -34,6 +36,10 @@ constexpr uint32_t kUnroll = 4U;
  * vector path takes fewer than 2^32 elements, so group indices plus one
  * grid stride (at most 2^28) stay below 2^32. */
 constexpr uint32_t kBlocksPerCu = 1024U;
+/* general against vector kernel (m3_least_elements): x[1,512,7] 2.8 and 3.8
+ * us, [1,128,255] 2.8 and 4.2, [2,64,1001] 3.1 and 3.9, [2,192,1001] 4.1 and
+ * 4.1, [2,192,2001] 5.8 and 3.8 */
+constexpr uint32_t kVectorQuarters = 3U;
 
 /* y = x + inverse * sin(a*x)^2 given sine = sin(a*x). */
 __device__ __forceinline__ float m3_snake_finish(float x, float sine,
@@ -193,7 +199,12 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
         }
 #pragma unroll
         for (uint32_t u = 0U; u < kUnroll; ++u) {
-            const uint32_t g = min(first + u * kThreads, a.groups - 1U);
+            const uint32_t at = first + u * kThreads;
+
+            if (!M3_ANY_LANE(at < a.groups)) {
+                break; /* a wave past the end forms nothing */
+            }
+            const uint32_t g = min(at, a.groups - 1U);
             /* elements of the group before the row's end */
             const uint32_t here =
                 a.length.divisor - (4U * g - rows[u] * a.length.divisor);
@@ -217,7 +228,7 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
             }
             const float4 y = m3_snake4(x[u], alpha4, inverse4);
 
-            if (first + u * kThreads < a.groups) {
+            if (at < a.groups) {
                 m3_snake_put4<TANH>(a, g, y);
             }
         }
@@ -318,7 +329,11 @@ static int m3_snake_launch(m3_hip_device *device, const m3_hip_view *input,
                                ? (int64_t)alpha->byte_strides[1]
                                : 0;
 
-    if (m3_snake_vector(input, output)) {
+    /* With the TANH of the command after it the vector kernel saves a
+     * launch, which counts for more than its lanes' turns. */
+    if (m3_snake_vector(input, output) &&
+        (tanh_output != nullptr ||
+         output->element_count >= m3_least_elements(device, kVectorQuarters))) {
         m3_snake_vec_args args;
 
         std::memset(&args, 0, sizeof(args));

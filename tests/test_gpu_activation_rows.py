@@ -1,8 +1,9 @@
 """SNAKE1D, TANH and GATED_SILU at odd lengths, alignments and row pitches
 (GPU), bit for bit against the oracle.
 
-The vector kernels take four consecutive elements per lane at any
-alignment. A Snake1d group that a channel's end cuts uses two alphas; a
+Tensors with fewer elements than the device has lanes (about: 393,216 to
+917,504 on one MI355X) run one element per lane; the vector kernels take four
+consecutive elements per lane at any alignment. A Snake1d group that a channel's end cuts uses two alphas; a
 GATED_SILU group that a row's end cuts reads its elements one by one when
 gate and up are rows of a wider tensor.
 """
@@ -48,7 +49,9 @@ def special(rng, values):
 
 @pytest.mark.parametrize("batch,channels,length", [
     (1, 1, 4), (1, 3, 4), (2, 5, 5), (2, 7, 6), (1, 64, 7), (3, 9, 63),
-    (2, 33, 65), (2, 3, 1021), (1, 2, 4098), (2, 5, 3), (2, 5, 1)])
+    (2, 33, 65), (2, 3, 1021), (1, 2, 4098), (2, 5, 3), (2, 5, 1),
+    (2, 66, 3001), (1, 99001, 4), (2, 40009, 5), (2, 30011, 7),
+    (3, 131, 1023), (1, 3, 150001)])
 def test_snake1d_lengths(hip, batch, channels, length):
     rng = np.random.default_rng(61000 + channels * 31 + length)
     shape = (batch, channels, length)
@@ -66,7 +69,8 @@ def test_snake1d_lengths(hip, batch, channels, length):
                 "snake1d %s shift %d" % (shape, shift))
 
 
-@pytest.mark.parametrize("count", [1, 3, 4, 5, 1023, 4097])
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 1023, 4097, 393215, 393216,
+                                   700003])
 @pytest.mark.parametrize("shift", [1, 2, 3])
 def test_tanh_alignments(hip, count, shift):
     rng = np.random.default_rng(62000 + count + shift)
@@ -76,6 +80,30 @@ def test_tanh_alignments(hip, count, shift):
             [ViewSpec(0, m3.F32, (count,), None, 4 * shift),
              ViewSpec(1, m3.F32, (count,), None, 4 * (4 - shift))],
             "tanh %d shift %d" % (count, shift))
+
+
+@pytest.mark.parametrize("dtype", [m3.F32, m3.F16, m3.BF16])
+@pytest.mark.parametrize("count", [5, 4099, 393215, 393217, 524289, 786435])
+def test_gated_silu_alignments(hip, dtype, count):
+    """Contiguous operands at different alignments, on both sides of the
+    sizes from which the vector kernels run."""
+    rng = np.random.default_rng(64000 + count)
+    size = m3.DTYPE_SIZES[dtype]
+    values = special(rng, (rng.standard_normal(2 * count + 8) * 4).astype(
+        np.float32))
+    if dtype == m3.F16:
+        with np.errstate(over="ignore"):
+            values = values.astype(np.float16).view(np.uint16)
+    elif dtype == m3.BF16:
+        values = (values.view(np.uint32) >> 16).astype(np.uint16)
+    for shift in (0, 1, 3):
+        out = np.full((count + 8) * size, 0xA5, np.uint8)
+        compare(hip, m3.OP_GATED_SILU, [as_bytes(values), out],
+                [ViewSpec(0, dtype, (count,), None, shift * size),
+                 ViewSpec(0, dtype, (count,), None,
+                          (count + 2 * shift) * size),
+                 ViewSpec(1, dtype, (count,), None, shift * size)],
+                "gated_silu %d shift %d dtype %d" % (count, shift, dtype))
 
 
 @pytest.mark.parametrize("dtype", [m3.F32, m3.F16, m3.BF16])
