@@ -24,13 +24,15 @@
  *                                             it: a group of 4 may wrap or
  *                                             take two elements)
  *        PERIODIC offset = (f / I) mod P     (any I, per-element loads)
- *   3. when both inputs classify, the vector kernel runs: each lane handles
- *      groups of 4 consecutive outputs with 16-byte (F32) or 8-byte
- *      (F16/BF16) loads and stores at any alignment, two groups in flight
- *      per lane, grid-stride over the tensor; with F32 operands and a
- *      tensor whose lanes are all resident at once, its held form instead
- *      (all loads, then the stores after a timed wait); divisions by I and
- *      P use precomputed multiply-shift divisors;
+ *   3. when both inputs classify, and there are enough elements (or their
+ *      loads are known when a kernel is compiled, m3_operand_kind), the
+ *      vector kernel runs: each lane handles groups of 4 consecutive
+ *      outputs with 16-byte (F32) or 8-byte (F16/BF16) loads and stores at
+ *      any alignment, two groups in flight per lane, grid-stride over the
+ *      tensor; with F32 operands and a tensor whose lanes are all resident
+ *      at once, its held form instead (all loads, then the stores after a
+ *      timed wait); divisions by I and P use precomputed multiply-shift
+ *      divisors;
  *   4. anything else runs the general kernel: per-element offsets from the
  *      coalesced stride table.
  * A run of such operations and float casts in which each takes the one
@@ -479,9 +481,9 @@ __device__ __forceinline__ uint4 m3_chain_op4(uint32_t op, uint4 x, uint4 y)
  * operation, passes over the same buffers: F32 x[2,512,24001] * s[512,1] +
  * b[512,1] 67.5 -> 44.8 us (6.6 TB/s; over buffers that change from pass to
  * pass 66.6 -> 54.6, 5.4 TB/s), BF16 107 -> 32.7, F16 120 -> 40.4;
- * x[8,1024,1536] * c[1536] then to BF16 and back to F32 47.4 -> 28.8. Two groups per lane and one tile
- * per workgroup: one group 29.8 and 46.0, four 30.6 and 46.8; 16 workgroups
- * per CU in a loop the same within 1%. */
+ * x[8,1024,1536] * c[1536] then to BF16 and back to F32 47.4 -> 28.8. Two
+ * groups per lane and one tile per workgroup: one group 29.8 and 46.0, four
+ * 30.6 and 46.8; 16 workgroups per CU in a loop the same within 1%. */
 template <int STEPS, uint32_t DT, int UNROLL>
 __global__ __launch_bounds__(256) void m3_chain_kernel(m3_chain_args a)
 {
@@ -700,6 +702,21 @@ bool m3_operand_whole(const m3_bin_operand &o)
            (kind != M3_KIND_ANY && ((uintptr_t)o.base & 15U) == 0U);
 }
 
+/* How many elements (m3_least_elements) operands that go by their modes want
+ * for the vector kernel; below, one element per lane is faster, contiguous or
+ * not. General against vector kernel, us: F32 in rows of 7 times a column
+ * 100,000 3.2 and 3.8, 300,000 3.6 and 3.9, 400,000 4.1 and 4.0; BF16 times
+ * BF16 20,000 3.0 and 4.0, 300,000 3.4 and 4.1, 524,288 3.8 and 4.2, 650,000
+ * 4.4 and 4.3; F16 in rows of 3 times a column 20,000 3.4 and 5.6, 650,000
+ * 5.4 and 5.8, 800,000 6.1 and 5.9. */
+uint32_t m3_any_quarters(const m3_bin_vec_args &vec, bool f32)
+{
+    const bool cut = m3_kind_of(vec.left) == M3_KIND_ANY ||
+                     m3_kind_of(vec.right) == M3_KIND_ANY;
+
+    return f32 ? 3U : cut ? 6U : 4U;
+}
+
 /* The F32 kernels of one pair of kinds: streamed (hold_ticks null) or held. */
 typedef void (*m3_binary_launcher)(dim3, hipStream_t, hipEvent_t, hipEvent_t,
                                    const m3_bin_vec_args &, const uint32_t *);
@@ -812,24 +829,27 @@ int m3_launch_binary_op(m3_hip_device *device, const m3_hip_view *left,
                 },
                 message, capacity);
         }
-        return m3_hip_launch(
-            device, names[OP],
-            [&](hipEvent_t start, hipEvent_t stop) {
-                if (f32) {
-                    hipExtLaunchKernelGGL(
-                        (m3_binary_vec_kernel<OP, M3N_F32, M3_KIND_ANY,
-                                              M3_KIND_ANY>),
-                        dim3(blocks), dim3(kThreads), 0, device->stream,
-                        start, stop, 0U, vec);
-                } else {
-                    hipExtLaunchKernelGGL(
-                        (m3_binary_vec_kernel<OP, kAnyDtype, M3_KIND_ANY,
-                                              M3_KIND_ANY>),
-                        dim3(blocks), dim3(kThreads), 0, device->stream,
-                        start, stop, 0U, vec);
-                }
-            },
-            message, capacity);
+        if (vec.count >= m3_least_elements(
+                             device, m3_any_quarters(vec, f32))) {
+            return m3_hip_launch(
+                device, names[OP],
+                [&](hipEvent_t start, hipEvent_t stop) {
+                    if (f32) {
+                        hipExtLaunchKernelGGL(
+                            (m3_binary_vec_kernel<OP, M3N_F32, M3_KIND_ANY,
+                                                  M3_KIND_ANY>),
+                            dim3(blocks), dim3(kThreads), 0, device->stream,
+                            start, stop, 0U, vec);
+                    } else {
+                        hipExtLaunchKernelGGL(
+                            (m3_binary_vec_kernel<OP, kAnyDtype, M3_KIND_ANY,
+                                                  M3_KIND_ANY>),
+                            dim3(blocks), dim3(kThreads), 0, device->stream,
+                            start, stop, 0U, vec);
+                    }
+                },
+                message, capacity);
+        }
     }
 
     m3_bin_general_args general;

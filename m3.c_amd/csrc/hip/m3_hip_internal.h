@@ -208,11 +208,11 @@ int m3_hip_launch(m3_hip_device *device, const char *name, Launch launch,
     return m3_hip_check(status, name, message, capacity);
 }
 
-/* How many elements a vector kernel of an activation wants: `quarters` of
- * four times as many as the device has lanes at once (four SIMDs per CU,
- * eight waves of 64 each). With fewer, the general kernel's one element per
- * lane leaves the work spread over all CUs, while a vector kernel's lanes
- * take eight or sixteen elements one after another in a few waves. */
+/* How many elements a vector kernel wants: `quarters` fourths of the lanes
+ * that the device has at once (four SIMDs per CU, eight waves of 64 each).
+ * With fewer, the general kernel's one element per lane leaves the work
+ * spread over all CUs, while a vector kernel's lanes take eight or sixteen
+ * elements one after another in a few waves. */
 static inline uint64_t m3_least_elements(const m3_hip_device *device,
                                          uint32_t quarters)
 {

@@ -112,6 +112,49 @@ def test_binary_f32_kinds(hip, shape, left_kind, right_kind):
                                                   right_kind, op, shift))
 
 
+# shapes of the second operand over [a, b]; b is a multiple of 4 in the
+# whole modes and not in the cut ones, 3 in the periodic ones
+MODES = [(1601, 640, "full"), (1601, 640, "trail"), (1601, 640, "row"),
+         (1601, 640, "scalar"), (1597, 641, "full"), (1597, 641, "trail"),
+         (1597, 641, "row"), (341333, 3, "trail"), (341333, 3, "row"),
+         (131, 3001, "trail"), (131, 3001, "row"), (131073, 3, "row"),
+         (77, 641, "trail"), (77, 640, "row"), (9001, 3, "row")]
+
+
+@pytest.mark.parametrize("a,b,kind", MODES)
+@pytest.mark.parametrize("dtypes", [(m3.F32, m3.F32, m3.F32),
+                                    (m3.BF16, m3.BF16, m3.BF16),
+                                    (m3.F16, m3.F16, m3.F16),
+                                    (m3.F32, m3.BF16, m3.F32),
+                                    (m3.F16, m3.F32, m3.BF16)])
+def test_binary_modes(hip, a, b, kind, dtypes):
+    """Every broadcast mode in 16 bits, mixed and F32, on both sides of the
+    sizes from which operands that go by their modes take the vector kernel
+    (393,216 to 786,432 elements on one MI355X), one element off alignment."""
+    rng = np.random.default_rng(7200 + a + b + dtypes[0])
+    op = [m3.OP_ADD, m3.OP_MUL, m3.OP_SUB, m3.OP_DIV][(a + b) % 4]
+
+    def values(count, dtype):
+        bits = random_f32(rng, count).view(np.uint32)
+        if dtype == m3.F32:
+            return as_bytes(bits)
+        if dtype == m3.BF16:
+            return as_bytes((bits >> 16).astype(np.uint16))
+        picks = rng.integers(0, 1 << 16, count)
+        return as_bytes(picks.astype(np.uint16))
+
+    dims = KINDS[kind](a, b)
+    sizes = [m3.DTYPE_SIZES[d] for d in dtypes]
+    compare(hip, op,
+            [values(a * b + 1, dtypes[0]),
+             values(int(np.prod(dims)) + 1, dtypes[1]),
+             np.zeros((a * b + 1) * sizes[2], np.uint8)],
+            [ViewSpec(0, dtypes[0], (a, b), None, sizes[0]),
+             ViewSpec(1, dtypes[1], dims, None, sizes[1]),
+             ViewSpec(2, dtypes[2], (a, b), None, sizes[2])],
+            "modes %s [%d,%d] %s op%d" % (kind, a, b, dtypes, op))
+
+
 def sixteen_bit_source(rng, count):
     """Every 16-bit pattern, then random ones."""
     every = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16)
