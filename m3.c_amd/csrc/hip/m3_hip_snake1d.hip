@@ -188,6 +188,12 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
 
         uint32_t rows[kUnroll];
         float alpha[kUnroll];
+        /* the wave's groups before the end, in steps of kThreads */
+        const uint32_t live =
+            (a.groups -
+             (uint32_t)__builtin_amdgcn_readfirstlane((int)first) +
+             kThreads - 1U) /
+            kThreads;
 
 #pragma unroll
         for (uint32_t u = 0U; u < kUnroll; ++u) {
@@ -199,11 +205,10 @@ __global__ __launch_bounds__(256) void m3_snake1d_vec_kernel(
         }
 #pragma unroll
         for (uint32_t u = 0U; u < kUnroll; ++u) {
-            const uint32_t at = first + u * kThreads;
-
-            if (!M3_ANY_LANE(at < a.groups)) {
+            if (u >= live) {
                 break; /* a wave past the end forms nothing */
             }
+            const uint32_t at = first + u * kThreads;
             const uint32_t g = min(at, a.groups - 1U);
             /* elements of the group before the row's end */
             const uint32_t here =
